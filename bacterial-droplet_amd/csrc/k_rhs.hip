@@ -2,8 +2,8 @@
 //
 // Replaces the reference's getRHS (TTSH3D.cu:363-468: 94 halo fills plus
 // getTempVari_1 :537-558, getTempVari_2 :561-605, getDtF :608-632) and
-// getVStar (:471-491) with one LDS-tiled pass that reads phi, P, v once and
-// writes phi^{n+1}, v*, P*:
+// getVStar (:471-491) with one pass that reads phi, P, v once and writes
+// phi^{n+1}, v*, P*:
 //
 //   G_ab  = D_a P_b                    mu0 = 2 aPhi (phi - 3phi^2 + 2phi^3) - kPhi L phi
 //   mu_b  = phi P_b + La^2 L P_b       Sig_ab = phi G_ab
@@ -18,124 +18,177 @@
 // zero for finite fields, so they are not evaluated; kappa therefore has no
 // effect, as in the reference.
 //
-// Stencils (TTSH3D.cu:3280-3343) in factored form, S = [1,4,1]/6:
-//   D_x f = 1/(2h) sum_dy S(dy) [S_z f(x+1, y+dy) - S_z f(x-1, y+dy)]
-//   D_z f = 1/(2h) sum_dx,dy S(dx) S(dy) [f(z+1) - f(z-1)](x+dx, y+dy)
-//   L f   = lc sum_{dx,dy=+-1} [f(z-1)+f(z+1)](x+dx,y+dy)
-//         + lf ([f(z-1)+f(z+1)] + f(x+-1) + f(y+-1)) + l0 f
-// so each plane is first "z-prepared" per xy position (f, f(z-1)+f(z+1),
-// f(z+1)-f(z-1), S_z f) and every derivative becomes a 2D stencil over those
-// arrays, sharing the partial sums between neighbouring cells.
+// Stencils (TTSH3D.cu:3280-3343).  With S = [1,4,1], d = [-1,0,1] and
+// s = 1/(72 h), lc = 1/(12 h^2),
+//   D_x = s d_x S_y S_z,  D_y = s S_x d_y S_z,  D_z = s S_x S_y d_z
+//   L f = lc (sum of the 8 corners + 8 sum of the 6 faces - 56 f)
+// is applied one axis at a time, each axis where its neighbours are cheapest:
+//   z  three planes of a value in registers, rotating with the z-march:
+//        t = f(z-1)+f(z+1), b = f(z+1)-f(z-1), a = S_z f = 4 f + t
+//   x  lanes of a wave are consecutive x; neighbours come by DPP wave shifts:
+//        X = d_x a, A = S_x a, B = S_x b, E = t(x-1)+t(x+1) + 8 f,
+//        O = t + f(x-1)+f(x+1) - 7 f
+//   y  a wave is one row; X, A, B, E of a row go to LDS as one 16-byte record
+//        and the rows at y-1 (m) and y+1 (p) are read back:
+//        D_x/s = 4 X + Xm + Xp, D_y/s = Ap - Am, D_z/s = 4 B + Bm + Bp,
+//        L/lc = 8 O + Em + Ep
+// The scales s and lc are folded into the pointwise factors.  The
+// intermediates (Sig, mu, mu0) take the same x and y stages, and their z
+// stage is an accumulation into the three output planes that a plane touches.
 //
-// Schedule: a work-group owns a TX x TY column of cells and marches through a
-// z-range.  Each thread keeps the three z-planes of its xy positions in
-// registers (phi, P over a 2-cell apron, v over a 1-cell apron) and loads the
-// next plane while the current one is used.  Per iteration: z-prepare the
-// plane behind the newest into LDS; compute the 13 intermediates (Sigma, mu,
-// mu0) over the 1-cell apron into LDS; add their contribution to the D.Sigma,
-// L mu, L mu0 of the three output planes they touch (registers); finish the
-// output plane two behind the newest input plane.
+// What bounds it: VALU issue.  The kernel that this one replaced kept whole
+// z-prepared tiles in LDS and read every 2D stencil from there: 226 LDS and
+// 704 VALU instructions per plane and wave, LDS 57-74% busy at about 120
+// bytes per clock and CU, the rate of 4- and 8-byte reads.  16-byte reads run
+// at 230.  A record per row and field needs one 16-byte write and two 16-byte
+// reads per field where the 2D stencils took 22 values, and each one-axis sum
+// is made once instead of by every neighbour: 44 LDS and 430 VALU
+// instructions per plane and wave.  Measured, same boxes, 16-row tiles
+// against the best of the former tiles: 64^3 37 -> 19 us (with the shallower
+// z-chunks below), 128^3 75 -> 55, 180^3 216 -> 119, 240^3 463 -> 234,
+// 256^3 498 -> 324.
+//
+// Tile: one wave per row of TX <= 60 cells, whose 64 lanes include the 2-cell
+// x apron; NW rows per work-group (8 or 16), one cell per lane.  N is cut
+// into ceil(N/60) tiles of equal width.  Wider tiles would need the apron
+// columns from other waves; two rows per wave (213 VGPRs, two waves per SIMD)
+// measured 4% slower at 128^3 and equal at 240^3 and 256^3.  The rows above
+// and below the tile are staged by all waves, one or two (row, field) pairs
+// each, and the first eight waves compute the intermediates of the two rows
+// next to the tile.
+//
+// 16 rows (1024 threads, 128 VGPRs, 160 KB of LDS: one group per CU, four
+// waves per SIMD) have the smaller share of apron rows and are faster
+// wherever the device is full: 240^3 234 against 317 us.  8 rows (98 KB) take
+// 2.1 us per plane instead of 3.2 when a CU holds one group, which wins for
+// small boxes.  Both do the same arithmetic in the same order (no contraction
+// in this file), so a droplet's result does not depend on the tile.
 #include <type_traits>
 
 #include "ttsh_dev.h"
 #include "ttsh_kernels.h"
 
+#pragma clang fp contract(off)
+
 namespace ttsh {
 
-// The three z-prepared arrays of one field: f, f(z+1)-f(z-1), S_z f.
-enum { ZF = 0, ZD = 1, ZS = 2, NZ = 3 };
+typedef float fvec4 __attribute__((ext_vector_type(4)));
 
-struct Der4 {
+__device__ __forceinline__ float fma_(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+
+// Keeps the compiler from sinking a value's computation past this point: sunk
+// past a barrier, all its inputs would stay live instead of the one value.
+__device__ __forceinline__ void pin(float& a) { asm volatile("" : "+v"(a)); }
+
+// A value that the compiler cannot derive, so that a global access keeps its
+// scalar base and 32-bit lane offset instead of a hoisted 64-bit address.
+__device__ __forceinline__ unsigned opaque(unsigned a)
+{
+    asm volatile("" : "+v"(a));
+    return a;
+}
+
+// The value of the lane at x-1 / x+1 (DPP wave_shr:1, wave_shl:1; 0 past the
+// ends of the wave, whose lanes are apron).
+__device__ __forceinline__ float from_left(float a)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(a), 0x138, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float from_right(float a)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(a), 0x130, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float xpair(float a) { return from_left(a) + from_right(a); }
+__device__ __forceinline__ float xdiff(float a) { return from_right(a) - from_left(a); }
+
+// A row of one field after its z and x stages; X, A, B, E are the record that
+// the neighbouring rows read.
+struct XRow {
+    float X, A, B, E, O;
+    __device__ __forceinline__ fvec4 record() const { return fvec4{X, A, B, E}; }
+};
+__device__ __forceinline__ XRow xrow(float fm, float f, float fp)
+{
+    XRow r;
+    const float t = fm + fp;
+    const float b = fp - fm;
+    const float a = fma_(4.f, f, t);
+    const float pt = xpair(t), pf = xpair(f);
+    r.X = xdiff(a);
+    r.A = fma_(4.f, a, fma_(4.f, pf, pt));
+    r.B = fma_(4.f, b, xpair(b));
+    r.E = fma_(8.f, f, pt);
+    r.O = fma_(-7.f, f, t + pf);
+    return r;
+}
+
+// D_x/s, D_y/s, D_z/s, L/lc of a row from its own stage and the records of
+// the rows below (m) and above (p).
+struct Der {
     float dx, dy, dz, l;
 };
-
-// LDS tiles hold the arrays of one position together (array-of-structs) with
-// an odd stride S in floats, so lanes at consecutive positions hit distinct
-// banks.  A stencil reads three rows through three row pointers, each at the
-// x-1 neighbour of its row: every value of a row then lies within 1 KiB of
-// the row pointer, the reach of a paired LDS read's immediate offsets, so no
-// per-pair base addresses are needed.
-using lcptr = __attribute__((address_space(3))) const float*;
-
-struct Rows {
-    lcptr m;  // row y-1, position x-1
-    lcptr c;  // row y
-    lcptr p;  // row y+1
-};
-
-// Row pointers of position pos in a tile with row stride W and position
-// stride S.  The LDS byte addresses, array base included, are made opaque to
-// the compiler so that it does not re-derive them from one far base.
-template <int W, int S>
-__device__ __forceinline__ Rows rows_at(const float* base, int pos)
+__device__ __forceinline__ Der yder(const XRow& r, const fvec4& m, const fvec4& p)
 {
-    const unsigned b0 = (unsigned)(size_t)(lcptr)base;
-    unsigned a = b0 + 4u * (unsigned)((pos - W - 1) * S);
-    unsigned b = b0 + 4u * (unsigned)((pos - 1) * S);
-    unsigned c = b0 + 4u * (unsigned)((pos + W - 1) * S);
-    asm volatile("" : "+v"(a), "+v"(b), "+v"(c));
-    return {(lcptr)(size_t)a, (lcptr)(size_t)b, (lcptr)(size_t)c};
-}
-
-// Laplacian from the f and S_z f arrays (field offset fo within a position).
-template <int S>
-__device__ __forceinline__ float lap_rows(const Rows& r, int fo, const Coef& co)
-{
-    auto F = [&](lcptr q, int dx) { return q[(dx + 1) * S + fo + ZF]; };
-    auto Z = [&](lcptr q, int dx) { return q[(dx + 1) * S + fo + ZS]; };
-    return co.lcs * ((Z(r.m, -1) + Z(r.m, 1)) + (Z(r.p, -1) + Z(r.p, 1)))
-         + co.lcf * ((F(r.m, -1) + F(r.m, 1)) + (F(r.p, -1) + F(r.p, 1)))
-         + co.lf * ((F(r.c, -1) + F(r.c, 1)) + (F(r.m, 0) + F(r.p, 0))) + co.l0s * Z(r.c, 0) + co.l0f * F(r.c, 0);
-}
-
-// D_x, D_y, D_z, L of the field at offset fo.
-template <int S>
-__device__ __forceinline__ Der4 der_rows(const Rows& r, int fo, const Coef& co)
-{
-    auto Z = [&](lcptr q, int dx) { return q[(dx + 1) * S + fo + ZS]; };
-    auto D = [&](lcptr q, int dx) { return q[(dx + 1) * S + fo + ZD]; };
-    Der4 d;
-    d.dx = co.e0 * (Z(r.c, 1) - Z(r.c, -1)) + co.e1 * ((Z(r.m, 1) - Z(r.m, -1)) + (Z(r.p, 1) - Z(r.p, -1)));
-    d.dy = co.e0 * (Z(r.p, 0) - Z(r.m, 0)) + co.e1 * ((Z(r.p, -1) - Z(r.m, -1)) + (Z(r.p, 1) - Z(r.m, 1)));
-    d.dz = co.f00 * D(r.c, 0) + co.f01 * ((D(r.c, -1) + D(r.c, 1)) + (D(r.m, 0) + D(r.p, 0)))
-         + co.f11 * ((D(r.m, -1) + D(r.m, 1)) + (D(r.p, -1) + D(r.p, 1)));
-    d.l = lap_rows<S>(r, fo, co);
+    Der d;
+    d.dx = fma_(4.f, r.X, m.x + p.x);
+    d.dy = p.y - m.y;
+    d.dz = fma_(4.f, r.B, m.z + p.z);
+    d.l = fma_(8.f, r.O, m.w + p.w);
     return d;
 }
 
-
-template <int TX, int TY, int WPS>
-__global__ __launch_bounds__(TX * TY, WPS) void k_rhs(const Drop* __restrict__ drops, const Work* __restrict__ work,
-                                                 const int* __restrict__ nwork_p, int parity, int kstep)
+// The intermediates of one P component after their x stage.  With
+// X = d_x Sig_xb and A = S_x Sig_yb, the row's part of S_y d_x Sig_x +
+// d_y S_x Sig_y is 4 X for itself, U = X + A for the row below it and
+// W = X - A for the row above; B = S_x Sig_zb; pm = mu(x-1)+mu(x+1).
+struct IRow {
+    float X, U, W, B, pm, m;
+};
+__device__ __forceinline__ IRow irow(float sx, float sy, float sz, float m)
 {
-    constexpr int NT = TX * TY;
-    constexpr int W2 = TX + 4, H2 = TY + 4, A2 = W2 * H2;  // phi, P, v planes: 2-cell apron layout
-    constexpr int W1 = TX + 2, H1 = TY + 2, A1 = W1 * H1;  // v and intermediates: 1-cell apron
-    constexpr int NRING = A1 - NT;
-    static_assert(NRING <= NT, "one ring position per thread at most");
-    // apron rings around the tile and the loads per thread that cover them
-    // as (position, field) pairs
-    constexpr int R2 = A2 - NT, R1 = A1 - NT;
-    constexpr int NR2 = (4 * R2 + NT - 1) / NT, NR1 = (3 * R1 + NT - 1) / NT;
-    // per position: phi, Px, Py, Pz x (f, dz, sz) | vx, vy, vz x (f, dz, sz) |
-    // Sigma(9, [3a+b]), mu(3), mu0 of one plane
-    constexpr int SP = 13, SV = 9, SS = 13;
-    // Tiles of which LDS fits one work-group per CU (WPS 1: two waves per
-    // SIMD at most) can spend registers on unrolling the z-march by its
-    // 3-slot rotation, which removes the register moves of the rotation.
-    constexpr bool kUnroll3 = WPS == 1;
-    __shared__ float zp[A2 * SP];
-    __shared__ float zv[A1 * SV];
-    __shared__ float sM[A1 * SS];
+    IRow o;
+    o.X = xdiff(sx);
+    const float A = fma_(4.f, sy, xpair(sy));
+    o.U = o.X + A;
+    o.W = o.X - A;
+    o.B = fma_(4.f, sz, xpair(sz));
+    o.pm = xpair(m);
+    o.m = m;
+    return o;
+}
 
-    const int tid = threadIdx.x;
-    const int tx = tid % TX, ty = tid / TX;
-    const int o2c = (ty + 2) * W2 + (tx + 2);  // own cell, 2-cell-apron layout
-    const int o1c = (ty + 1) * W1 + (tx + 1);  // own cell, 1-cell-apron layout
+// mu0 of a cell: -kPhi lc, the raw Laplacian, 2 aPhi
+__device__ __forceinline__ float mu0_of(float ph, float l, float kl, float a2)
+{
+    const float ph2 = ph * ph;
+    return fma_(-kl, l, a2 * fma_(2.f * ph2, ph, fma_(-3.f, ph2, ph)));
+}
+
+template <int NW>
+__global__ __launch_bounds__(64 * NW, NW / 4) void k_rhs(const Drop* __restrict__ drops, const Work* __restrict__ work,
+                                                         const int* __restrict__ nwork_p, int parity, int kstep)
+{
+    constexpr int HP = NW + 4, HV = NW + 2;  // rows of phi, P records; of v records and intermediates
+    // Two buffers of BUF records.  A plane uses them as: phi, P -> X; the
+    // intermediates -> Y; v -> X; then X and Y swap.  Each exchange then
+    // writes the buffer whose readers passed the previous barrier.
+    constexpr int BUF = 4 * HP * 64;
+    // intermediates: per component (U, W, B, pm), then (m_0, m_1, m_2, mu0),
+    // then mu0's pm
+    constexpr int IM = 3 * HV * 64, IP = 4 * HV * 64;
+    static_assert(IP + HV * 16 <= BUF, "the intermediates fit a buffer");
+    // apron rows of phi, P staged per wave: (field, inner row) and (field,
+    // outer row) for 8 waves, one of them for 16
+    constexpr int NT = NW == 8 ? 2 : 1;
+    static_assert(NW == 8 || NW == 16, "apron rows are dealt to 8 or 16 waves");
+    __shared__ fvec4 lds[2 * BUF];
+
+    const int lane = threadIdx.x & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int nwork = *nwork_p;
 
-    for (int v = blockIdx.x; v < xcd_span(nwork); v += gridDim.x) {
-        const int w = xcd_item(v, nwork);
+    for (int vi = blockIdx.x; vi < xcd_span(nwork); vi += gridDim.x) {
+        const int w = xcd_item(vi, nwork);
         if (w >= nwork) continue;
         const Work wk = work[w];
         const Drop& D = drops[wk.d];
@@ -143,7 +196,8 @@ __global__ __launch_bounds__(TX * TY, WPS) void k_rhs(const Drop* __restrict__ d
         const Coef co = D.co;
         const int N = D.N;
         const unsigned NN = (unsigned)N * (unsigned)N;
-        const int x0 = wk.a * TX, y0 = wk.b * TY;
+        const int TX = rhs_tile_width(N);
+        const int x0 = wk.a * TX, y0 = wk.b * NW;
         const int zb = wk.c & 0xffff;
         const int ze = wk.c >> 16;
         const gptr<const float> gin[4] = {glb<const float>(D.phi[parity]), glb<const float>(D.P[0]),
@@ -154,419 +208,289 @@ __global__ __launch_bounds__(TX * TY, WPS) void k_rhs(const Drop* __restrict__ d
         const gptr<float> ovs[3] = {glb(D.vs[parity][0]), glb(D.vs[parity][1]), glb(D.vs[parity][2])};
         const gptr<float> ops[3] = {glb(D.ps[parity][0]), glb(D.ps[parity][1]), glb(D.ps[parity][2])};
 
-        const int gx = x0 + tx, gy = y0 + ty;
-        const bool own = (gx < N) && (gy < N);
-        const unsigned gown = 4u * ((unsigned)gy * (unsigned)N + (unsigned)gx);
+        // own cell: lanes 2 .. TX+1 of the row; the other lanes load the
+        // apron (or, past it, any cell: x0 + lane - 2 < 2 N since N >= 32)
+        const int gx = x0 + lane - 2, gy = y0 + wv;
+        const int cx = wrapi(gx, N);
+        const bool own = lane >= 2 && lane < 2 + TX && gx < N && gy < N;
+        auto row_off = [&](int y) { return 4u * ((unsigned)wrapi(y, N) * (unsigned)N + (unsigned)cx); };
+        const unsigned off = row_off(gy);
+        // Apron rows: field `part` (phi, P_x, P_y, P_z) at the row next to the
+        // tile (inner: -1 or NW) or beyond it (-2 or NW+1), side 0 below and 1
+        // above.  Waves 0..7 stage an inner row and compute its intermediates;
+        // the outer rows go to the same waves (8 rows) or to waves 8..15, and
+        // with them v_x, v_y, v_z of the inner rows.
+        const int part = (wv & 7) >> 1, side = wv & 1;
+        const bool inner = wv < 8;
+        const bool vrow = part < 3 && (NW == 8 || !inner);
+        const int ri = side ? NW : -1, ro = side ? NW + 1 : -2;
+        const int r0 = inner ? ri : ro;  // first staged row; the second is ro
+        const unsigned off0 = row_off(y0 + r0), off1 = row_off(y0 + ro), offv = row_off(y0 + ri);
+        const gptr<const float> gp = part == 0 ? gin[0] : part == 1 ? gin[1] : part == 2 ? gin[2] : gin[3];
+        const gptr<const float> gpv = part == 0 ? gv[0] : part == 1 ? gv[1] : gv[2];
 
-        // Loads of a plane: the thread's own cell (a wave loads whole aligned
-        // rows), one per field, and the apron ring around the tile as
-        // (position, field) pairs spread over NR2 (phi, P) and NR1 (v) loads
-        // per thread.  Ring loads address the fields from the lowest field
-        // pointer of their group (one allocation: 32-bit offsets).
-        gptr<const float> gb2 = gin[0], gb1 = gv[0];
-#pragma unroll
-        for (int f = 1; f < 4; ++f) gb2 = gin[f] < gb2 ? gin[f] : gb2;
-#pragma unroll
-        for (int f = 1; f < 3; ++f) gb1 = gv[f] < gb1 ? gv[f] : gb1;
-        const unsigned own2 = 4u * ((unsigned)wrapi(gy, N) * (unsigned)N + (unsigned)wrapi(gx, N));
-        const unsigned own1 = own2;
-        unsigned roff2[NR2], roff1[NR1];
-        int rl2[NR2], rl1[NR1];  // LDS float index of the pair's f array (-1: past the last pair)
-#pragma unroll
-        for (int m = 0; m < NR2; ++m) {
-            const int j = min(tid + m * NT, 4 * R2 - 1), f = j / R2, r = j % R2;
-            int i;
-            if (r < 2 * W2) i = r;                                                  // rows y0-2, y0-1
-            else if (r < 4 * W2) i = (TY + 2) * W2 + (r - 2 * W2);                  // rows y0+TY, +TY+1
-            else if (r < 4 * W2 + 2 * TY) i = (2 + (r - 4 * W2) / 2) * W2 + (r - 4 * W2) % 2;
-            else i = (2 + (r - 4 * W2 - 2 * TY) / 2) * W2 + W2 - 2 + (r - 4 * W2 - 2 * TY) % 2;
-            roff2[m] = 4u * (unsigned)(gin[f] - gb2)
-                     + 4u * ((unsigned)wrapi(y0 - 2 + i / W2, N) * (unsigned)N + (unsigned)wrapi(x0 - 2 + i % W2, N));
-            rl2[m] = tid + m * NT < 4 * R2 ? i * SP + f * NZ : -1;
-        }
-#pragma unroll
-        for (int m = 0; m < NR1; ++m) {
-            const int j = min(tid + m * NT, 3 * R1 - 1), f = j / R1, r = j % R1;
-            int i;
-            if (r < W1) i = r;                                       // row y0-1
-            else if (r < 2 * W1) i = (TY + 1) * W1 + (r - W1);       // row y0+TY
-            else if (r < 2 * W1 + TY) i = (r - 2 * W1 + 1) * W1;     // column x0-1
-            else i = (r - 2 * W1 - TY + 1) * W1 + (W1 - 1);          // column x0+TX
-            roff1[m] = 4u * (unsigned)(gv[f] - gb1)
-                     + 4u * ((unsigned)wrapi(y0 - 1 + i / W1, N) * (unsigned)N + (unsigned)wrapi(x0 - 1 + i % W1, N));
-            rl1[m] = tid + m * NT < 3 * R1 ? i * SV + f * NZ : -1;
-        }
-        // three z-planes per value in registers, in slots rotating with the
-        // z-march: in phase K the slots K, K+1, K+2 (mod 3) hold planes zi-2,
-        // zi-1, zi
-        float in[4][3], inr[NR2][3];
-        float vin[3][3], vinr[NR1][3];
-        auto load_plane = [&](int slot, int z, unsigned o2, const unsigned* r2, unsigned o1, const unsigned* r1) {
-            const size_t zo = (size_t)wrapi(z, N) * NN;
-#pragma unroll
-            for (int f = 0; f < 4; ++f) in[f][slot] = ldb(gin[f] + zo, o2);
-#pragma unroll
-            for (int m = 0; m < NR2; ++m) inr[m][slot] = ldb(gb2 + zo, r2[m]);
-#pragma unroll
-            for (int f = 0; f < 3; ++f) vin[f][slot] = ldb(gv[f] + zo, o1);
-#pragma unroll
-            for (int m = 0; m < NR1; ++m) vinr[m][slot] = ldb(gb1 + zo, r1[m]);
+        // record indices: row q of a field at (q - first row)*64 + lane
+        const int lp = (wv + 2) * 64 + lane;
+        const int lv = (wv + 1) * 64 + lane;
+        const int l0 = (part * HP + r0 + 2) * 64 + lane, l1 = (part * HP + ro + 2) * 64 + lane;
+        const int lvr = (part * HV + ri + 1) * 64 + lane;
+        const int lir = (ri + 1) * 64 + lane;
+
+        auto put_i = [&](fvec4* y, int b, int i, const IRow& o) {
+            y[b * HV * 64 + i] = fvec4{o.U, o.W, o.B, o.pm};
+            ((float*)(y + IM + i))[b] = o.m;
         };
-        load_plane(0, zb - 2, own2, roff2, own1, roff1);
-        load_plane(1, zb - 1, own2, roff2, own1, roff1);
-        load_plane(2, zb, own2, roff2, own1, roff1);
+        auto put_m = [&](fvec4* y, int i, float pm, float m) {
+            ((float*)(y + IM + i))[3] = m;
+            ((float*)(y + IP))[i] = pm;
+        };
+
+        // three z-planes per value, in slots rotating with the z-march: in
+        // phase K the slots K, K+1, K+2 (mod 3) hold planes zm-1, zm, zm+1
+        float f[4][3], vf[3][3], tf[NT][3], tv[3];
+        auto load_p = [&](int slot, int z) {
+            const size_t zo = (size_t)wrapi(z, N) * NN;
+            const unsigned o = opaque(off);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) f[k][slot] = ldb(gin[k] + zo, o);
+            tf[0][slot] = ldb(gp + zo, opaque(off0));
+            if constexpr (NT == 2) tf[1][slot] = ldb(gp + zo, opaque(off1));
+        };
+        auto load_v = [&](int slot, int z) {
+            const size_t zo = (size_t)wrapi(z, N) * NN;
+            const unsigned o = opaque(off);
+#pragma unroll
+            for (int b = 0; b < 3; ++b) vf[b][slot] = ldb(gv[b] + zo, o);
+            tv[slot] = ldb(gpv + zo, opaque(offv));
+        };
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            load_p(k, zb - 2 + k);
+            load_v(k, zb - 2 + k);
+        }
         wait_vmem();
 
-        // D.Sigma, L mu, L mu0 accumulated per output plane, slot-rotated like
-        // the inputs: in phase K slot K is plane zm-1, K+1 is zm, K+2 is zm+1
-        float aS[3][3], aL[3][3], aL0[3];
-#pragma unroll
-        for (int q = 0; q < 3; ++q) {
-            aL0[q] = 0.f;
-#pragma unroll
-            for (int b = 0; b < 3; ++b) { aS[q][b] = 0.f; aL[q][b] = 0.f; }
-        }
-        // pointwise part of the update of the own cell, per plane:
+        // per output plane (same rotation): sums of D.Sig/s, L mu/lc, L mu0/lc,
+        // and the rest of the update
         //   [b]   v_b + Dt (-v.D v_b + mu L v_b + mu0 D_b phi)
         //   [3+b] P_b + Dt (-v.D P_b - alpha phi P_b - beta |P|^2 P_b - lambda0 P.D P_b - anchoring_b)
         //   [6]   phi + Dt (-v.D phi)
-        float cur[7], nxt[7];
+        float aS[3][3], aL[3][3], aL0[3], nx[3][7];
+        XRow xv[3];  // v of the plane staged last
+#pragma unroll
+        for (int b = 0; b < 3; ++b) {
+            aL0[b] = 0.f;
+            xv[b] = XRow{0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int q = 0; q < 3; ++q) { aS[q][b] = 0.f; aL[q][b] = 0.f; }
+        }
+#pragma unroll
+        for (int j = 0; j < 7; ++j) nx[0][j] = 0.f;
+        fvec4 *bx = lds, *by = lds + BUF;
+        const float s = co.d1 * (1.f / 36.f), lc = co.lc;
 
-        auto body = [&](auto ph, int zi) {
-            constexpr int S0 = decltype(ph)::value, S1 = (S0 + 1) % 3, S2 = (S0 + 2) % 3;
-            // LDS positions made opaque per plane: the compiler then folds each
-            // neighbour's constant offset into the LDS instruction instead of
-            // hoisting dozens of loop-invariant addresses into registers
-            // (the stencils' row pointers are opaque the same way)
-            int ti = tid;
-            asm volatile("" : "+v"(ti));
-            ti &= 0x7fff;  // known non-negative again (a no-op)
-            // likewise the in-plane global byte offsets, so that loads and
-            // stores take a scalar plane base plus this 32-bit offset
-            unsigned go = gown, o2 = own2, o1 = own1, q2[NR2], q1[NR1];
-            asm volatile("" : "+v"(go), "+v"(o2), "+v"(o1));
-#pragma unroll
-            for (int m = 0; m < NR2; ++m) {
-                q2[m] = roff2[m];
-                asm volatile("" : "+v"(q2[m]));
-            }
-#pragma unroll
-            for (int m = 0; m < NR1; ++m) {
-                q1[m] = roff1[m];
-                asm volatile("" : "+v"(q1[m]));
-            }
-            // ---- 1. z-prepare plane zm = zi-1 ------------------------------
-            // Two barriers per plane suffice: zp and zv are read only in stage
-            // 2, which every thread ends before the previous plane's barrier
-            // ahead of stage 3; sM is written in stage 2 and read in stage 3,
-            // and the barrier after stage 1 orders them across planes.
-            // f, f(z+1)-f(z-1), S_z f of one value into LDS at float index q
-            auto zprep = [&](float* q, const float* t) {
-                const float a = t[S0], b = t[S1], c = t[S2];
-                q[ZF] = b;
-                q[ZD] = c - a;
-                q[ZS] = co.sw0 * b + co.sw1 * (a + c);
-            };
+        __syncthreads();  // the previous item has read both buffers
+        auto body = [&](auto ph_, int zm) {
+            constexpr int S0 = decltype(ph_)::value, S1 = (S0 + 1) % 3, S2 = (S0 + 2) % 3;
+            // ---- a: y stage of v of plane zm-1 (records in Y), which ends its
+            // update terms; z and x stages of phi, P of plane zm
             {
-                int i2 = o2c * SP, i1 = o1c * SV;
-                asm volatile("" : "+v"(i2), "+v"(i1));
+                const float mulc = co.mu * lc;
+                const float vx = vf[0][S0] * s, vy = vf[1][S0] * s, vz = vf[2][S0] * s;
 #pragma unroll
-                for (int f = 0; f < 4; ++f) zprep(zp + i2 + f * NZ, in[f]);
-#pragma unroll
-                for (int f = 0; f < 3; ++f) zprep(zv + i1 + f * NZ, vin[f]);
+                for (int b = 0; b < 3; ++b) {
+                    const fvec4* q = by + b * HV * 64 + lv;
+                    const Der d = yder(xv[b], q[-64], q[64]);
+                    const float adv = fma_(vx, d.dx, fma_(vy, d.dy, vz * d.dz));
+                    nx[S0][b] = fma_(co.Dt, fma_(mulc, d.l, nx[S0][b]) - adv, vf[b][S0]);
+                    pin(nx[S0][b]);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
             }
+            // phi of the inner apron row, for its intermediates
+            const float phr = ldb(gin[0] + (size_t)wrapi(zm, N) * NN, opaque(offv));
+            XRow xp[4];
 #pragma unroll
-            for (int m = 0; m < NR2; ++m) {
-                int i = rl2[m];
-                asm volatile("" : "+v"(i));
-                if (i >= 0) zprep(zp + i, inr[m]);
-            }
-#pragma unroll
-            for (int m = 0; m < NR1; ++m) {
-                int i = rl1[m];
-                asm volatile("" : "+v"(i));
-                if (i >= 0) zprep(zv + i, vinr[m]);
-            }
-            if constexpr (kUnroll3) {
-                // prefetch plane zi+1 into the slot of plane zi-2
-                if (zi <= ze) load_plane(S0, zi + 1, o2, q2, o1, q1);
-            } else {
-                // roll the planes and prefetch plane zi+1 into the newest slot
-                auto roll = [](float* t) { t[0] = t[1]; t[1] = t[2]; };
-#pragma unroll
-                for (int f = 0; f < 4; ++f) roll(in[f]);
-#pragma unroll
-                for (int m = 0; m < NR2; ++m) roll(inr[m]);
-#pragma unroll
-                for (int f = 0; f < 3; ++f) roll(vin[f]);
-#pragma unroll
-                for (int m = 0; m < NR1; ++m) roll(vinr[m]);
-                if (zi <= ze) load_plane(2, zi + 1, o2, q2, o1, q1);
-            }
-            __syncthreads();
-
-            // ---- 2. intermediates of plane zm over the 1-cell apron --------
-            {
-                // own cell: intermediates and the pointwise update terms
-                const Rows rp = rows_at<W2, SP>(zp, o2c);
-                const Rows rv = rows_at<W1, SV>(zv, o1c);
-                float* const mo = sM + (size_t)o1c * SS;
-                const Der4 dph = der_rows<SP>(rp, 0, co);
-                const float ph = rp.c[SP + ZF];
-                const float ph2 = ph * ph;
-                const float mu0 = co.aPhi2 * (ph - 3.f * ph2 + 2.f * ph2 * ph) - co.kPhi * dph.l;
-                mo[12] = mu0;
+            for (int k = 0; k < 4; ++k) {
+                xp[k] = xrow(f[k][S0], f[k][S1], f[k][S2]);
+                pin(xp[k].O);
+                bx[k * HP * 64 + lp] = xp[k].record();
                 __builtin_amdgcn_sched_barrier(0);
-                float Pc[3], vc[3];
-#pragma unroll
-                for (int b = 0; b < 3; ++b) {
-                    Pc[b] = rp.c[SP + (1 + b) * NZ + ZF];
-                    vc[b] = rv.c[SV + b * NZ + ZF];
-                }
-                const float P2 = Pc[0] * Pc[0] + Pc[1] * Pc[1] + Pc[2] * Pc[2];
-                float an[3] = {0.f, 0.f, 0.f};
-                if (co.anchoring) {
-                    const float dP2 = dph.dx * dph.dx + dph.dy * dph.dy + dph.dz * dph.dz;
-                    const float sP = sqrtf(P2);
-                    const float dpP = dph.dx * Pc[0] + dph.dy * Pc[1] + dph.dz * Pc[2];
-                    const float Dp[3] = {dph.dx, dph.dy, dph.dz};
-#pragma unroll
-                    for (int b = 0; b < 3; ++b) an[b] = co.A * (dP2 * P2 * Pc[b] + sP * Dp[b] * dpP);
-                }
-#pragma unroll
-                for (int b = 0; b < 3; ++b) {
-                    const Der4 d = der_rows<SP>(rp, (1 + b) * NZ, co);
-                    mo[9 + b] = ph * Pc[b] + co.La2 * d.l;
-                    mo[0 * 3 + b] = ph * d.dx;
-                    mo[1 * 3 + b] = ph * d.dy;
-                    mo[2 * 3 + b] = ph * d.dz;
-                    const float vgp = vc[0] * d.dx + vc[1] * d.dy + vc[2] * d.dz;
-                    const float pgp = Pc[0] * d.dx + Pc[1] * d.dy + Pc[2] * d.dz;
-                    const float dtp = -vgp - co.alpha * ph * Pc[b] - co.beta * P2 * Pc[b] - co.lambda0 * pgp - an[b];
-                    nxt[3 + b] = Pc[b] + co.Dt * dtp;
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-                const float Dp[3] = {dph.dx, dph.dy, dph.dz};
-#pragma unroll
-                for (int b = 0; b < 3; ++b) {
-                    const Der4 d = der_rows<SV>(rv, b * NZ, co);
-                    const float vdv = vc[0] * d.dx + vc[1] * d.dy + vc[2] * d.dz;
-                    nxt[b] = vc[b] + co.Dt * (-vdv + co.mu * d.l + mu0 * Dp[b]);
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-                nxt[6] = ph + co.Dt * (-(vc[0] * dph.dx + vc[1] * dph.dy + vc[2] * dph.dz));
-                // materialise the carried terms here: sunk past the barrier,
-                // their inputs would stay live through stage 3
-#pragma unroll
-                for (int j = 0; j < 7; ++j) asm volatile("" : "+v"(nxt[j]));
             }
-            // Intermediates of the apron ring, spread over every wave as
-            // (position, part) pairs when one pass of the tile's threads covers
-            // them: four parts (mu0, then the intermediates of P_x, P_y, P_z),
-            // or three (those of P_b, with mu0 in part 0).  Otherwise each of
-            // the first NRING threads computes all 13 of one position.  All use
-            // the own cell's expressions.
-            // two waves with a ring of at most 64 positions: one part per wave
-            constexpr bool kWaveParts = !(3 * NRING <= NT) && NT == 128 && NRING <= 64;
-            constexpr int NPART = 4 * NRING <= NT ? 4 : 3 * NRING <= NT ? 3 : kWaveParts ? 2 : 1;
-            constexpr int PSTR = kWaveParts ? 64 : NRING;  // lane stride between parts
-            if (ti % PSTR < NRING && ti < NPART * PSTR) {
-                const int f = ti / PSTR, r = ti % PSTR;
-                int lx1, ly1;
-                if (r < W1) { lx1 = r; ly1 = 0; }
-                else if (r < 2 * W1) { lx1 = r - W1; ly1 = H1 - 1; }
-                else if (r < 2 * W1 + TY) { lx1 = 0; ly1 = 1 + (r - 2 * W1); }
-                else { lx1 = W1 - 1; ly1 = 1 + (r - 2 * W1 - TY); }
-                const int q2 = (ly1 + 1) * W2 + (lx1 + 1);
-                const int q1 = ly1 * W1 + lx1;
-                const Rows rq = rows_at<W2, SP>(zp, q2);
-                const float ph = rq.c[SP + ZF];
-                float* m = sM + q1 * SS;
-                // intermediates of P_b at this position
-                auto pint = [&](int b, int fo) {
-                    const Der4 d = der_rows<SP>(rq, fo, co);
-                    m[9 + b] = ph * rq.c[SP + fo + ZF] + co.La2 * d.l;
-                    m[0 * 3 + b] = ph * d.dx;
-                    m[1 * 3 + b] = ph * d.dy;
-                    m[2 * 3 + b] = ph * d.dz;
-                };
-                auto mu0 = [&]() {
-                    const float ph2 = ph * ph;
-                    m[12] = co.aPhi2 * (ph - 3.f * ph2 + 2.f * ph2 * ph) - co.kPhi * lap_rows<SP>(rq, 0, co);
-                };
-                if constexpr (NPART == 4) {
-                    if (f == 0) mu0();
-                    else pint(f - 1, f * NZ);
-                } else if constexpr (NPART == 3) {
-                    if (f == 0) mu0();
-                    pint(f, (1 + f) * NZ);
-                } else if constexpr (NPART == 2) {
-                    if (f == 0) {  // wave 0: mu0 and P_x
-                        mu0();
-                        pint(0, 1 * NZ);
-                    } else {  // wave 1: P_y and P_z
-                        pint(1, 2 * NZ);
-                        __builtin_amdgcn_sched_barrier(0);
-                        pint(2, 3 * NZ);
-                    }
-                } else {
-                    mu0();
+            XRow xi = xrow(tf[0][S0], tf[0][S1], tf[0][S2]);
+            pin(xi.O);
+            bx[l0] = xi.record();
+            if constexpr (NT == 2) {
+                __builtin_amdgcn_sched_barrier(0);
+                bx[l1] = xrow(tf[1][S0], tf[1][S1], tf[1][S2]).record();
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            load_p(S0, min(zm + 2, ze + 1));
+            __syncthreads();
+
+            // ---- b: y stage of phi, P; pointwise terms; x stage of the
+            // intermediates of plane zm
+            IRow im[3];
+            float m0, pm0;
+            {
+                const float ph = f[0][S1];
+                float w0, w1, w2, q1, an[3] = {0.f, 0.f, 0.f};
+                {
+                    const fvec4* q = bx + lp;
+                    const Der d = yder(xp[0], q[-64], q[64]);
+                    m0 = mu0_of(ph, d.l, co.kPhi * lc, co.aPhi2);
+                    pm0 = xpair(m0);
+                    put_m(by, lv, pm0, m0);
+                    const float P0 = f[1][S1], P1 = f[2][S1], P2 = f[3][S1];
+                    const float v0 = vf[0][S1], v1 = vf[1][S1], v2 = vf[2][S1];
+                    const float pp = fma_(P0, P0, fma_(P1, P1, P2 * P2));
+                    q1 = fma_(co.alpha, ph, co.beta * pp);
+                    // v + lambda0 P: the two advections of P are one
+                    w0 = s * fma_(co.lambda0, P0, v0);
+                    w1 = s * fma_(co.lambda0, P1, v1);
+                    w2 = s * fma_(co.lambda0, P2, v2);
+                    const float adv = s * fma_(v0, d.dx, fma_(v1, d.dy, v2 * d.dz));
+                    nx[S1][6] = fma_(-co.Dt, adv, ph);
+                    const float ms = m0 * s;
+                    nx[S1][0] = ms * d.dx;
+                    nx[S1][1] = ms * d.dy;
+                    nx[S1][2] = ms * d.dz;
 #pragma unroll
-                    for (int b = 0; b < 3; ++b) {
-                        pint(b, (1 + b) * NZ);
-                        __builtin_amdgcn_sched_barrier(0);
+                    for (int b = 0; b < 3; ++b) pin(nx[S1][b]);
+                    pin(nx[S1][6]);
+                    if (co.anchoring) {
+                        const float dx = d.dx * s, dy = d.dy * s, dz = d.dz * s;
+                        const float dd = fma_(dx, dx, fma_(dy, dy, dz * dz)) * pp;
+                        const float sp = sqrtf(pp) * fma_(dx, P0, fma_(dy, P1, dz * P2));
+                        an[0] = co.A * fma_(dd, P0, sp * dx);
+                        an[1] = co.A * fma_(dd, P1, sp * dy);
+                        an[2] = co.A * fma_(dd, P2, sp * dz);
                     }
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                const float phs = ph * s, la = co.La2 * lc;
+#pragma unroll
+                for (int b = 0; b < 3; ++b) {
+                    const fvec4* q = bx + (1 + b) * HP * 64 + lp;
+                    const Der d = yder(xp[1 + b], q[-64], q[64]);
+                    const float Pb = f[1 + b][S1];
+                    const float dt = fma_(q1, Pb, fma_(w0, d.dx, fma_(w1, d.dy, w2 * d.dz))) + an[b];
+                    nx[S1][3 + b] = fma_(-co.Dt, dt, Pb);
+                    pin(nx[S1][3 + b]);
+                    im[b] = irow(phs * d.dx, phs * d.dy, phs * d.dz, fma_(la, d.l, ph * Pb));
+                    put_i(by, b, lv, im[b]);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            if (NW == 8 || inner) {
+                const Der d = yder(xi, bx[l0 - 64], bx[l0 + 64]);
+                if (part == 0) {
+                    const float m = mu0_of(phr, d.l, co.kPhi * lc, co.aPhi2);
+                    put_m(by, lir, xpair(m), m);
+                } else {
+                    const float ps = phr * s;
+                    put_i(by, part - 1, lir,
+                          irow(ps * d.dx, ps * d.dy, ps * d.dz, fma_(co.La2 * lc, d.l, phr * tf[0][S1])));
                 }
             }
             __syncthreads();
 
-            // ---- 3. contribution of plane zm to outputs zm-1, zm, zm+1 ------
+            // ---- c: y stage of the intermediates, added to planes zm-1, zm,
+            // zm+1; store plane zm-1; z and x stages of v of plane zm
+            __builtin_amdgcn_sched_barrier(0);
             {
-                const Rows rs = rows_at<W1, SS>(sM, o1c);
-#define SM(f, dx, dy) ((dy) < 0 ? rs.m : (dy) > 0 ? rs.p : rs.c)[((dx) + 1) * SS + (f)]
+                const fvec4 mm = by[IM + lv - 64], mp = by[IM + lv + 64];
 #pragma unroll
                 for (int b = 0; b < 3; ++b) {
-                    const int fx = 0 * 3 + b, fy = 1 * 3 + b, fz = 2 * 3 + b;
-                    const float ax = co.e0 * (SM(fx, 1, 0) - SM(fx, -1, 0))
-                                   + co.e1 * ((SM(fx, 1, -1) - SM(fx, -1, -1)) + (SM(fx, 1, 1) - SM(fx, -1, 1)));
-                    const float ay = co.e0 * (SM(fy, 0, 1) - SM(fy, 0, -1))
-                                   + co.e1 * ((SM(fy, -1, 1) - SM(fy, -1, -1)) + (SM(fy, 1, 1) - SM(fy, 1, -1)));
-                    const float A = ax + ay;
-                    const float Bz = co.f00 * SM(fz, 0, 0)
-                                   + co.f01 * ((SM(fz, -1, 0) + SM(fz, 1, 0)) + (SM(fz, 0, -1) + SM(fz, 0, 1)))
-                                   + co.f11 * ((SM(fz, -1, -1) + SM(fz, 1, -1)) + (SM(fz, -1, 1) + SM(fz, 1, 1)));
-                    aS[S0][b] += co.sw1 * A + Bz;
-                    aS[S1][b] += co.sw0 * A;
-                    aS[S2][b] += co.sw1 * A - Bz;
-                    const int fm = 9 + b;
-                    const float cen = SM(fm, 0, 0);
-                    const float E = co.lc * ((SM(fm, -1, -1) + SM(fm, 1, -1)) + (SM(fm, -1, 1) + SM(fm, 1, 1))) + co.lf * cen;
-                    const float F = co.lf * ((SM(fm, -1, 0) + SM(fm, 1, 0)) + (SM(fm, 0, -1) + SM(fm, 0, 1))) + co.l0 * cen;
+                    const fvec4* q = by + b * HV * 64 + lv;
+                    const fvec4 im_ = q[-64], ip_ = q[64];
+                    const IRow& o = im[b];
+                    const float A = fma_(4.f, o.X, ip_.x + im_.y);
+                    const float B = fma_(4.f, o.B, im_.z + ip_.z);
+                    const float E = fma_(8.f, o.m, im_.w + ip_.w);
+                    const float F = fma_(-7.f, o.m, (mm[b] + mp[b]) + o.pm);
+                    aS[S0][b] += A + B;
+                    aS[S1][b] = fma_(4.f, A, aS[S1][b]);
+                    aS[S2][b] = A - B;
                     aL[S0][b] += E;
-                    aL[S1][b] += F;
-                    aL[S2][b] += E;
+                    aL[S1][b] = fma_(8.f, F, aL[S1][b]);
+                    aL[S2][b] = E;
+#pragma unroll
+                    for (int q3 = 0; q3 < 3; ++q3) { pin(aS[q3][b]); pin(aL[q3][b]); }
                     __builtin_amdgcn_sched_barrier(0);
                 }
-                {
-                    const float cen = SM(12, 0, 0);
-                    const float E = co.lc * ((SM(12, -1, -1) + SM(12, 1, -1)) + (SM(12, -1, 1) + SM(12, 1, 1))) + co.lf * cen;
-                    const float F = co.lf * ((SM(12, -1, 0) + SM(12, 1, 0)) + (SM(12, 0, -1) + SM(12, 0, 1))) + co.l0 * cen;
-                    aL0[S0] += E;
-                    aL0[S1] += F;
-                    aL0[S2] += E;
-                }
-#undef SM
+                const float* const q = (const float*)(by + IP) + lv;
+                const float E = fma_(8.f, m0, q[-64] + q[64]);
+                const float F = fma_(-7.f, m0, (mm.w + mp.w) + pm0);
+                aL0[S0] += E;
+                aL0[S1] = fma_(8.f, F, aL0[S1]);
+                aL0[S2] = E;
+#pragma unroll
+                for (int q3 = 0; q3 < 3; ++q3) pin(aL0[q3]);
             }
-
-            // ---- 4. finish output plane zo = zi-2 ---------------------------
-            const int zo = zi - 2;
-            if (zo >= zb && own) {
-                const size_t pz = (size_t)zo * NN;
-                stb(ophi + pz, go, cur[6] + co.Dt * (co.gamma * aL0[S0]));
+            if (zm - 1 >= zb && own) {
+                const size_t pz = (size_t)(zm - 1) * NN;
+                const float ka = co.Dt * co.cA * s, ke = co.Dt * co.eta * lc, kg = co.Dt * co.gamma * lc;
+                const unsigned o = opaque(off);
+                stb(ophi + pz, o, fma_(kg, aL0[S0], nx[S0][6]));
 #pragma unroll
                 for (int b = 0; b < 3; ++b) {
-                    stb(ovs[b] + pz, go, cur[b] + co.Dt * (co.cA * aS[S0][b]));
-                    stb(ops[b] + pz, go, cur[3 + b] + co.Dt * (co.eta * aL[S0][b]));
+                    stb(ovs[b] + pz, o, fma_(ka, aS[S0][b], nx[S0][b]));
+                    stb(ops[b] + pz, o, fma_(ke, aL[S0][b], nx[S0][3 + b]));
                 }
             }
-            if constexpr (kUnroll3) {
-                // slot S0 becomes plane zm+2 in the next phase
-                aL0[S0] = 0.f;
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int b = 0; b < 3; ++b) {
-                    aS[S0][b] = 0.f;
-                    aL[S0][b] = 0.f;
-                }
-            } else {
-                // rotate the output planes: zm becomes the next zm-1
-                aL0[0] = aL0[1];
-                aL0[1] = aL0[2];
-                aL0[2] = 0.f;
-#pragma unroll
-                for (int b = 0; b < 3; ++b) {
-                    aS[0][b] = aS[1][b];
-                    aS[1][b] = aS[2][b];
-                    aS[2][b] = 0.f;
-                    aL[0][b] = aL[1][b];
-                    aL[1][b] = aL[2][b];
-                    aL[2][b] = 0.f;
-                }
+            for (int b = 0; b < 3; ++b) {
+                xv[b] = xrow(vf[b][S0], vf[b][S1], vf[b][S2]);
+                pin(xv[b].O);
+                bx[b * HV * 64 + lv] = xv[b].record();
+                __builtin_amdgcn_sched_barrier(0);
             }
-#pragma unroll
-            for (int j = 0; j < 7; ++j) cur[j] = nxt[j];
+            if (vrow) bx[lvr] = xrow(tv[S0], tv[S1], tv[S2]).record();
+            load_v(S0, min(zm + 2, ze));
+            __syncthreads();
+            fvec4* const t = bx;
+            bx = by;
+            by = t;
         };
-
-        // z-march over zi = zb .. ze+1
-        if constexpr (kUnroll3) {
-            for (int zi = zb;;) {
-                body(Ph<0>{}, zi);
-                if (++zi > ze + 1) break;
-                body(Ph<1>{}, zi);
-                if (++zi > ze + 1) break;
-                body(Ph<2>{}, zi);
-                if (++zi > ze + 1) break;
-            }
-        } else {
-            for (int zi = zb; zi <= ze + 1; ++zi) body(Ph<0>{}, zi);
+        // planes zb-1 .. ze; plane zm-1 is stored in the iteration of zm
+        for (int zm = zb - 1;;) {
+            body(Ph<0>{}, zm);
+            if (++zm > ze) break;
+            body(Ph<1>{}, zm);
+            if (++zm > ze) break;
+            body(Ph<2>{}, zm);
+            if (++zm > ze) break;
         }
     }
 }
 
 // ---------------------------------------------------------------------------
-template <int TX, int TY, int WPS>
-static hipError_t launch_rhs_t(const Drop* drops, const Work* work, const int* nwork_p, int parity, int kstep,
-                               int grid, hipStream_t st)
-{
-    if (grid <= 0) return hipSuccess;
-    return launch_kernel(k_rhs<TX, TY, WPS>, dim3(grid), dim3(TX * TY), st, drops, work, nwork_p, parity, kstep);
-}
-
-// Tile variants: TX x TY cells per work-group and the waves per SIMD the
-// register allocation targets (the second __launch_bounds__ argument: 2 allows
-// 256 VGPRs, 3 allows 168, 1 allows 512).
+// Tile variants: the nominal tile a box has to hold, and the rows of the
+// kernel that runs it.
 struct RhsVar {
-    int tx, ty, wps;
+    int tx, ty, rows;
 };
 static const RhsVar kRhsVars[RHS_NVARIANTS] = {
-    {32, 8, 2}, {16, 16, 2}, {64, 4, 2}, {16, 8, 2}, {32, 8, 3}, {32, 16, 1}, {64, 8, 1},
+    {32, 8, 8}, {16, 16, 16}, {64, 4, 8}, {16, 8, 8}, {32, 8, 8}, {32, 16, 16}, {64, 8, 8},
 };
 
 hipError_t launch_rhs(int variant, const Drop* drops, const Work* work, const int* nwork_p, int parity, int kstep,
                       int grid, hipStream_t st)
 {
-    switch (variant) {
-    case 0: return launch_rhs_t<32, 8, 2>(drops, work, nwork_p, parity, kstep, grid, st);
-    case 1: return launch_rhs_t<16, 16, 2>(drops, work, nwork_p, parity, kstep, grid, st);
-    case 2: return launch_rhs_t<64, 4, 2>(drops, work, nwork_p, parity, kstep, grid, st);
-    case 3: return launch_rhs_t<16, 8, 2>(drops, work, nwork_p, parity, kstep, grid, st);
-    case 4: return launch_rhs_t<32, 8, 3>(drops, work, nwork_p, parity, kstep, grid, st);
-    case 5: return launch_rhs_t<32, 16, 1>(drops, work, nwork_p, parity, kstep, grid, st);
-    case 6: return launch_rhs_t<64, 8, 1>(drops, work, nwork_p, parity, kstep, grid, st);
-    default: return hipErrorInvalidValue;
-    }
+    if (grid <= 0) return hipSuccess;
+    if (variant < 0 || variant >= RHS_NVARIANTS) return hipErrorInvalidValue;
+    if (kRhsVars[variant].rows == 8)
+        return launch_kernel(k_rhs<8>, dim3(grid), dim3(512), st, drops, work, nwork_p, parity, kstep);
+    return launch_kernel(k_rhs<16>, dim3(grid), dim3(1024), st, drops, work, nwork_p, parity, kstep);
 }
 
-// Work-groups per CU that the LDS of a tile allows (160 KiB per CU): the
-// phi/P planes over a 2-cell apron (13 floats a position), v and the
-// intermediates over a 1-cell apron (9 and 13).
-int rhs_groups_per_cu(int variant)
-{
-    int tx, ty;
-    rhs_tile(variant, &tx, &ty);
-    if (tx <= 0) return 1;
-    const int bytes = 4 * ((tx + 4) * (ty + 4) * 13 + (tx + 2) * (ty + 2) * (9 + 13));
-    return std::max(1, (160 * 1024) / bytes);
-}
+int rhs_rows(int variant) { return variant >= 0 && variant < RHS_NVARIANTS ? kRhsVars[variant].rows : 0; }
 
-void rhs_tile(int variant, int* tx, int* ty)
+bool rhs_fits(int variant, int N)
 {
-    if (variant >= 0 && variant < RHS_NVARIANTS) {
-        *tx = kRhsVars[variant].tx;
-        *ty = kRhsVars[variant].ty;
-    } else {
-        *tx = 0;
-        *ty = 0;
-    }
+    return variant >= 0 && variant < RHS_NVARIANTS && N >= kRhsVars[variant].tx + 2 && N >= kRhsVars[variant].ty + 2;
 }
 
 }  // namespace ttsh

@@ -85,15 +85,11 @@ size_t droplet_bytes(int N)
            align256(sizeof(float)) + align256(n * sizeof(float));
 }
 
-static int default_rhs_variant(int N) { return (N % 32 == 0 && N >= 64) ? RHS_32x8 : RHS_16x16; }
+// K_rhs variant of a size without a tuning entry; 16x16 fits every supported N.
+static int default_rhs_variant(int) { return RHS_16x16; }
 
-// A K_rhs tile needs N >= TX+2 and N >= TY+2; 16x16 fits every supported N.
-static bool variant_fits(int v, int N)
-{
-    int tx, ty;
-    rhs_tile(v, &tx, &ty);
-    return N >= tx + 2 && N >= ty + 2;
-}
+// K_rhs work items of one z-range.
+static int rhs_tiles(int variant, int N) { return rhs_tiles_x(N) * ((N + rhs_rows(variant) - 1) / rhs_rows(variant)); }
 
 struct Slot {
     bool used = false;
@@ -106,6 +102,7 @@ struct Slot {
     int64_t steps = 0;      // steps since set_state / admission
     int64_t limit = -1;     // max steps, -1 = none
     double T = 0.0;         // T accumulated in double as the reference (TTSH3D.cu:342)
+    int rhs_want = -1;      // K_rhs variant asked for or tuned for this droplet
     int rhs_tz = 16, proj_tz = 8;
     bool rhs_tz_set = false;  // rhs_tz came from the parameters, not the tuning table
     int64_t fin_call = -1;    // the step call that took the droplet's last step (limit reached)
@@ -481,7 +478,7 @@ struct Engine {
         if (!tune_lookup(N, &tv, &ttz, &tpz) || tv < 0 || tv >= RHS_NVARIANTS) { tv = -1; ttz = 0; tpz = 0; }
         const int want = p.rhs_variant >= 0 ? p.rhs_variant : (tv >= 0 ? tv : default_rhs_variant(N));
         int v = rhs_variant < 0 ? want : rhs_variant;
-        if (!variant_fits(v, N)) {
+        if (!rhs_fits(v, N)) {
             if (p.rhs_variant >= 0) return fail(TTSH_EUNSUPPORTED, "grid smaller than the requested K_rhs tile");
             v = RHS_16x16;  // engine-wide: every droplet fits it
         }
@@ -569,6 +566,7 @@ struct Engine {
         s.steps = 0;
         s.limit = -1;
         s.T = p.T0;
+        s.rhs_want = want;
         s.rhs_tz = std::min(p.rhs_tz > 0 ? p.rhs_tz : (ttz > 0 ? ttz : 16), N);
         s.rhs_tz_set = p.rhs_tz > 0;
         s.proj_tz = std::min(p.corr_tz > 0 ? p.corr_tz : (tpz > 0 ? tpz : 8), N);
@@ -635,19 +633,19 @@ struct Engine {
 
     // Layout of a batch that fills the device.  The tuned tile and z-depth of
     // a size are chosen for that droplet alone, with enough z-chunks to fill
-    // the device; each chunk re-reads two warm-up planes.  A batch that fills
-    // the device by itself runs every droplet's K_rhs with one tile (the
-    // batch entry of the tuning table; by default 32x8, three groups per CU)
-    // and chunks of at least batch_rhs_tz planes, which cuts the warm-up share
-    // and gives items of nearly equal cost.  It applies when at least two
-    // droplets are active, none asks for a tile, every one fits the tile, and
-    // the items make at least two rounds of resident groups.  K_rhs has no
-    // reductions, so a droplet's result does not depend on this layout.
-    // K_corr (no reductions either) and K_div take chunks of about
-    // batch_corr_tz planes in the same batches.  K_div's sums, which set the
-    // k = 0 coefficient and sigma, stay per tuned chunk (Drop::part), so they
-    // do not change either.
-    int batch_rhs_variant = RHS_32x8, batch_rhs_tz = 32, batch_corr_tz = 32;
+    // the device; each chunk computes two more planes than it stores.  A batch
+    // that fills the device by itself runs every droplet's K_rhs with one tile
+    // (the batch entry of the tuning table; by default 16 rows) and chunks of
+    // at least batch_rhs_tz planes, which cuts the share of those planes and
+    // gives items of nearly equal cost.  It applies when at least two droplets
+    // are active, none asks for a tile, every one fits the tile, and the items
+    // make at least two rounds of one group per CU.  K_rhs has no reductions
+    // and every variant does the same arithmetic, so a droplet's result does
+    // not depend on this layout.  K_corr (no reductions either) and K_div take
+    // chunks of about batch_corr_tz planes in the same batches.  K_div's sums,
+    // which set the k = 0 coefficient and sigma, stay per tuned chunk
+    // (Drop::part), so they do not change either.
+    int batch_rhs_variant = RHS_16x16, batch_rhs_tz = 32, batch_corr_tz = 32;
     int tune_gen_seen = -1;
 
     // Re-read the batch entry of the tuning table after a reload; a running
@@ -657,9 +655,9 @@ struct Engine {
         const int g = tune_generation();
         if (g == tune_gen_seen) return;
         tune_gen_seen = g;
-        int v = RHS_32x8, rtz = 32, ctz = 32;
+        int v = RHS_16x16, rtz = 32, ctz = 32;
         if (!tune_batch_lookup(&v, &rtz, &ctz) || v < 0 || v >= RHS_NVARIANTS) {
-            v = RHS_32x8;
+            v = RHS_16x16;
             rtz = 32;
             ctz = 32;
         }
@@ -673,16 +671,33 @@ struct Engine {
     {
         int active = 0;
         int64_t items = 0;
-        int tx, ty;
-        rhs_tile(batch_rhs_variant, &tx, &ty);
         for (const Slot& s : slots) {
             if (!s.used || remaining(s) <= 0) continue;
-            if (s.prm.rhs_variant >= 0 || !variant_fits(batch_rhs_variant, s.N)) return false;
+            if (s.prm.rhs_variant >= 0 || !rhs_fits(batch_rhs_variant, s.N)) return false;
             ++active;
             const int tz = std::min(std::max(s.rhs_tz, batch_rhs_tz), s.N);
-            items += (int64_t)((s.N + tx - 1) / tx) * ((s.N + ty - 1) / ty) * ((s.N + tz - 1) / tz);
+            items += (int64_t)rhs_tiles(batch_rhs_variant, s.N) * ((s.N + tz - 1) / tz);
         }
-        return active >= 2 && items >= 2 * (int64_t)rhs_groups_per_cu(batch_rhs_variant) * cus;
+        return active >= 2 && items >= 2 * (int64_t)cus;
+    }
+
+    // K_rhs variant of the launches when the batch layout does not apply: the
+    // engine's when a droplet asks for one, else the tuned one of the largest
+    // active droplet, which has most of the work.
+    int lone_variant() const
+    {
+        int v = rhs_variant < 0 ? 0 : rhs_variant, N = 0;
+        for (const Slot& s : slots) {
+            if (!s.used || remaining(s) <= 0) continue;
+            if (s.prm.rhs_variant >= 0) return rhs_variant;
+            if (s.N > N) {
+                N = s.N;
+                v = s.rhs_want;
+            }
+        }
+        for (const Slot& s : slots)
+            if (s.used && remaining(s) > 0 && !rhs_fits(v, s.N)) return RHS_16x16;
+        return v;
     }
 
     // Rebuild descriptor and work tables from the active slots.
@@ -694,14 +709,13 @@ struct Engine {
         up_pending = false;
         std::vector<Work> w[kNTables];
         const bool batch = batch_layout();
-        const int rv = batch ? batch_rhs_variant : (rhs_variant < 0 ? 0 : rhs_variant);
+        const int rv = batch ? batch_rhs_variant : lone_variant();
         if (rv != rhs_active) {
             HIPCHK(hipStreamSynchronize(st));
             rhs_active = rv;
             drop_graphs();  // captured launches name the tile's kernel
         }
-        int tx, ty;
-        rhs_tile(rhs_active, &tx, &ty);
+        const int ty = rhs_rows(rhs_active);
         for (int si = 0; si < (int)slots.size(); ++si) {
             Slot& s = slots[si];
             h_drops[si] = s.drop;
@@ -719,7 +733,7 @@ struct Engine {
             for (int k = 0; k < nzr; ++k) {
                 const int zb = k * N / nzr, ze = (k + 1) * N / nzr;
                 for (int by = 0; by < (N + ty - 1) / ty; ++by)
-                    for (int bx = 0; bx < (N + tx - 1) / tx; ++bx)
+                    for (int bx = 0; bx < rhs_tiles_x(N); ++bx)
                         w[T_RHS].push_back(Work{si, bx, by, zb | (ze << 16)});
             }
             // divergence: the droplet's tuned z-chunks are its reduction blocks

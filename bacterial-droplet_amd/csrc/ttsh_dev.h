@@ -99,6 +99,12 @@ struct Work {
     int d, a, b, c;
 };
 
+// Width of K_rhs's tiles for a box of N: a wave holds at most 60 cells of a
+// row beside the 2-cell apron, and the row is cut into equal parts.
+constexpr int kRhsMaxTX = 60;
+__host__ __device__ constexpr int rhs_tiles_x(int N) { return (N + kRhsMaxTX - 1) / kRhsMaxTX; }
+__host__ __device__ constexpr int rhs_tile_width(int N) { return (N + rhs_tiles_x(N) - 1) / rhs_tiles_x(N); }
+
 // Work-groups are dispatched round-robin over the 8 XCDs, each with its own
 // L2.  Visit v of the grid-stride loop maps to work item
 //   (v mod 8) * chunk + v / 8,   chunk = ceil(nwork / 8),

@@ -1,14 +1,14 @@
 """Autotuner for the TTSH3D step kernels.
 
-For each grid size N it times, with HIP events through ttsh_profile, every
-K_rhs tile variant that fits N at several z-depths, and several z-depths of
-the divergence/corrector stencils, on a droplet of that size; then writes the
-fastest choices as the tuning table libttsh3d.so reads (tuned.txt beside the
-library, lines "N rhs_variant rhs_tz proj_tz").
+For each grid size N it times, with HIP events through ttsh_profile, the two
+K_rhs kernels (16 and 8 rows per work-group) at several z-depths, and several
+z-depths of the divergence/corrector stencils, on a droplet of that size; then
+writes the fastest choices as the tuning table libttsh3d.so reads (tuned.txt
+beside the library, lines "N rhs_variant rhs_tz proj_tz").
 
 With --batch it tunes the layout of a batch that fills the device instead:
 on the 64-droplet sweep mix (L in {48, 64, 96, 128}) as one graph batch, it
-times whole batch steps for every K_rhs tile that fits all sizes, minimum
+times whole batch steps for both K_rhs kernels, minimum
 K_rhs z-depth and divergence/corrector z-depth, through the table's "batch"
 line (re-read between candidates; the batch is laid out again at its next
 step), and keeps the fastest.  The FFT passes' lines per work-group are
@@ -27,7 +27,15 @@ import time
 
 from . import F64, TTSHError, Batch, Simulation, default_params, init_droplet, lib, LIB_PATH, tuning_reload
 
+# nominal tile of each variant: the box has to hold it
 RHS_VARIANTS = {0: (32, 8), 1: (16, 16), 2: (64, 4), 3: (16, 8), 4: (32, 8), 5: (32, 16), 6: (64, 8)}
+# one variant of each kernel, with the smallest nominal tile: 16 and 8 rows
+TUNED_VARIANTS = (1, 3)
+# z-depths: the engine splits z into ceil(N/tz) near-equal chunks; a chunk
+# computes two planes more than it stores, and the number of chunks times the
+# tiles of a plane should come just below a multiple of the CUs
+RHS_DEPTHS = (1, 2, 3, 4, 5, 6, 8, 9, 10, 11, 13, 16, 18, 20, 22, 24, 26, 29, 32, 36, 40, 43, 48, 52, 60, 64, 86, 128)
+PROJ_DEPTHS = (1, 2, 3, 4, 6, 8, 11, 16, 22, 32)
 DEFAULT_TABLE = os.path.join(os.path.dirname(LIB_PATH), "tuned.txt")
 
 
@@ -45,13 +53,13 @@ def tune_size(N: int, steps: int = 30, log=print):
     base = dict(N=N, dt0=0.01, cA=-2.0)
     best_rhs, best_proj = None, None
     results = []
-    # z-depths: the engine splits z into ceil(N/tz) near-equal chunks, so
-    # depths like 11 or 43 set the number of work items per CU
-    tzs = sorted({t for t in (8, 11, 16, 22, 32, 43, 64) if t <= N})
-    for var, (tx, ty) in RHS_VARIANTS.items():
-        if N < tx + 2 or N < ty + 2:
-            continue
-        for tz in tzs:
+    depths, nz = [], set()
+    for tz in RHS_DEPTHS:
+        if tz <= N and (N + tz - 1) // tz not in nz:  # depths of the same number of chunks are the same
+            nz.add((N + tz - 1) // tz)
+            depths.append(tz)
+    for var in TUNED_VARIANTS:
+        for tz in depths:
             try:
                 k = _time(default_params(rhs_variant=var, rhs_tz=tz, corr_tz=8, **base), state, steps)
             except TTSHError as e:
@@ -60,8 +68,10 @@ def tune_size(N: int, steps: int = 30, log=print):
             results.append({"kind": "rhs", "variant": var, "tz": tz, "ms": k["K_rhs"]})
             if best_rhs is None or k["K_rhs"] < best_rhs[2]:
                 best_rhs = (var, tz, k["K_rhs"])
-            log(f"N={N} K_rhs variant {var} ({tx}x{ty}) tz {tz}: {k['K_rhs'] * 1e3:.1f} us")
-    for ptz in [t for t in (4, 6, 8, 11, 16, 32) if t <= N]:
+            log(f"N={N} K_rhs variant {var} tz {tz}: {k['K_rhs'] * 1e3:.1f} us")
+            if best_rhs[0] == var and k["K_rhs"] > 2 * best_rhs[2] and tz > best_rhs[1]:
+                break  # too few chunks by now: deeper ones leave more of the device idle
+    for ptz in [t for t in PROJ_DEPTHS if t <= N]:
         k = _time(default_params(rhs_variant=best_rhs[0], rhs_tz=best_rhs[1], corr_tz=ptz, **base), state, steps)
         t = k["K_div"] + k["K_corr"]
         results.append({"kind": "proj", "tz": ptz, "ms": t})
@@ -107,7 +117,7 @@ def tune_batch(table: str, steps: int = 48, log=print):
     entries, _ = read_table(table)
     cases = workloads.sweep_mix(__import__("ttsh3d"))
     sizes = sorted({L for _, L, _ in cases})
-    variants = [v for v, (tx, ty) in RHS_VARIANTS.items() if all(L >= tx + 2 and L >= ty + 2 for L in sizes)]
+    variants = [v for v in TUNED_VARIANTS if all(L >= max(RHS_VARIANTS[v]) + 2 for L in sizes)]
     scratch = table + ".tuning"
     results = []
     best = None
@@ -116,8 +126,8 @@ def tune_batch(table: str, steps: int = 48, log=print):
         for p, L, s in cases:
             b.admit(p, *workloads.mix_state(__import__("ttsh3d"), L, s))
         for var in variants:
-            for rtz in (16, 24, 32, 48, 64):
-                for ctz in (16, 32, 64):
+            for rtz in (8, 12, 16, 24, 32, 48, 64):
+                for ctz in (8, 16, 32):
                     write_table(entries, scratch, (var, rtz, ctz))
                     tuning_reload(scratch)
                     b.step(16)  # re-layout and graph capture
