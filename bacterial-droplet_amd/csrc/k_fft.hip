@@ -293,39 +293,149 @@ struct Xch {
     }
 };
 
-// -1/(k^2 N^3) at integer wavenumbers (fftfreq order), k2[0] = 1.
+// -1/(k^2 N^3) at integer wavenumbers (fftfreq order), k2[0] = 1.  With
+// k^2 = k2s m2, m2 a whole number, it is pk0/m2; the reciprocal of m2 is the
+// hardware's (one unit in the last place) with one Newton step, so within one
+// unit, at a third of the instructions of an IEEE division.
 __device__ __forceinline__ float poisson_factor(const Coef& co, int N, int kx, int ky, int kz)
 {
     const int mx = kx < N / 2 ? kx : kx - N;
     const int my = ky < N / 2 ? ky : ky - N;
     const int mz = kz < N / 2 ? kz : kz - N;
     const int m2 = mx * mx + my * my + mz * mz;
-    const float k2 = m2 == 0 ? 1.f : co.k2s * (float)m2;
-    return -co.inv_n3 / k2;
+    const float x = (float)m2;
+    float r = __builtin_amdgcn_rcpf(x);
+    r = __builtin_fmaf(__builtin_fmaf(-x, r, 1.f), r, r);
+    return m2 == 0 ? -co.inv_n3 : co.pk0 * r;
 }
 
 // Work item (d, a, b): droplet d; the pass's lines are the L consecutive
 // lines starting at line-block a of the plane b (x pass: rows y of plane z=b;
-// y pass: columns x of plane z=b; z pass: columns x of row y=b).
+// y pass: columns x of plane z=b; z pass: columns x of row y=b).  One
+// work-group of PlanT<N>::NB or more threads; sx holds Xch<N, AXIS>::SIZE and
+// stw N elements.
 template <int N, int AXIS, int MODE>
-__global__ __launch_bounds__(PlanT<N>::NB) void k_fft(const Drop* __restrict__ drops, const Work* __restrict__ work,
-                                              const int* __restrict__ nwork_p, int kstep)
+__device__ __forceinline__ void fft_lines(const Drop& D, const Work& wk, float2* __restrict__ sx,
+                                          float2* __restrict__ stw)
 {
     using P = PlanT<N>;
     constexpr int R1 = P::R1, R2 = P::R2, L = P::L, T = P::T, NT = P::NT;
     using X = Xch<N, AXIS>;
-    __shared__ float2 sx[X::SIZE];
-    __shared__ float2 stw[N];
-
-    const int tid = threadIdx.x;
+    // opaque, so that a kernel with many sizes keeps no addresses of one size
+    // in registers while it runs another (425 VGPRs instead of 84)
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+    tid &= 0x3ff;
     const bool active = tid < NT;
     // lane -> (line l, thread-in-line t)
     int l, t;
     if constexpr (AXIS == 0) { l = tid / T; t = tid % T; }
     else { t = tid / L; l = tid % L; }
-    const int nwork = *nwork_p;
     constexpr size_t es = AXIS == 0 ? 1 : (AXIS == 1 ? (size_t)N : (size_t)N * N);
+    // first element of line l
+    size_t base;
+    int lx = 0, ly = 0;  // for the Poisson factor: the line's fixed indices
+    if constexpr (AXIS == 0) {
+        ly = wk.a * L + l;
+        base = ((size_t)wk.b * N + ly) * N;
+    } else if constexpr (AXIS == 1) {
+        lx = wk.a * L + l;
+        base = (size_t)wk.b * N * N + lx;
+    } else {
+        lx = wk.a * L + l;
+        ly = wk.b;
+        base = (size_t)ly * N + lx;
+    }
+    const gptr<float2> c = glb(D.c);
 
+    // the Poisson pass's work item holding kx = ky = 0 sets the k = 0
+    // coefficient from the FP64 sum of s (k_proj_stats)
+    const bool has0 = MODE == FFT_POISSON && wk.a == 0 && wk.b == 0;
+    // the first forward pass divides the imaginary part by sigma (a
+    // power of two: exact)
+    float isg = 1.f;
+    if constexpr (AXIS == 0 && MODE == FFT_FWD) isg = 1.f / glb(D.sigma)[0];
+
+    constexpr int DIR0 = MODE == FFT_INV ? 1 : -1;
+    float2 u[R1 > R2 ? R1 : R2];
+    // ---- step A: R1 threads, length-R2 DFTs -----------------------------
+    // The line's loads are issued before the twiddle table's, so both
+    // are in flight together; the table's LDS stores wait for all of them.
+    if (active && t < R1) {
+#pragma unroll
+        for (int n2 = 0; n2 < R2; ++n2) u[n2] = ld2(c, base + (size_t)(t + R1 * n2) * es);
+    }
+    for (int i = tid; i < N; i += blockDim.x) stw[i] = ld2(glb(D.tw), i);
+    if (active && t < R1) {
+        if constexpr (AXIS == 0 && MODE == FFT_FWD) {
+#pragma unroll
+            for (int n2 = 0; n2 < R2; ++n2) u[n2].y *= isg;
+        }
+        Dft<R2, DIR0>::run(u);
+    }
+    __syncthreads();  // stw
+    if (active && t < R1) {
+#pragma unroll
+        for (int k2 = 0; k2 < R2; ++k2) {
+            const float2 wv = stw[(t * k2) % N];
+            const float2 w2 = f2(wv.x, DIR0 == -1 ? wv.y : -wv.y);
+            sx[X::at(l, t, k2)] = k2 == 0 ? u[0] : mul2(u[k2], w2);
+        }
+    }
+    __syncthreads();
+    // ---- step B: R2 threads, length-R1 DFTs -----------------------------
+    if (active && t < R2) {
+#pragma unroll
+        for (int n1 = 0; n1 < R1; ++n1) u[n1] = sx[X::at(l, n1, t)];
+        Dft<R1, DIR0>::run(u);
+    }
+    if constexpr (MODE != FFT_POISSON) {
+        if (active && t < R2) {
+#pragma unroll
+            for (int k1 = 0; k1 < R1; ++k1) st2(c, base + (size_t)(t + R2 * k1) * es, u[k1]);
+        }
+    } else {
+        // multiply by -1/(k^2 N^3); element index kz = t + R2 k1
+        if (active && t < R2) {
+            const Coef co = D.co;
+#pragma unroll
+            for (int k1 = 0; k1 < R1; ++k1) {
+                const int kz = t + R2 * k1;
+                float2 s = u[k1];
+                if (has0 && l == 0 && kz == 0) s = f2((float)glb(D.stat)[0], (float)glb(D.stat)[1]);
+                const float m = poisson_factor(co, N, lx, ly, kz);
+                u[k1] = f2(s.x * m, s.y * m);
+            }
+            // inverse, roles swapped: n' = t + R2 k1, thread t = n1' < R2,
+            // length-R1 DFT over k1 in registers
+            Dft<R1, 1>::run(u);
+        }
+        __syncthreads();  // every thread has read sx in step B
+        if (active && t < R2) {
+#pragma unroll
+            for (int m2 = 0; m2 < R1; ++m2) {
+                const float2 wv = stw[(t * m2) % N];
+                sx[X::at(l, m2, t)] = m2 == 0 ? u[0] : mul2(u[m2], f2(wv.x, -wv.y));
+            }
+        }
+        __syncthreads();
+        if (active && t < R1) {
+#pragma unroll
+            for (int n1 = 0; n1 < R2; ++n1) u[n1] = sx[X::at(l, t, n1)];
+            Dft<R2, 1>::run(u);
+#pragma unroll
+            for (int m1 = 0; m1 < R2; ++m1) st2(c, base + (size_t)(t + R1 * m1) * es, u[m1]);
+        }
+    }
+}
+
+template <int N, int AXIS, int MODE>
+__global__ __launch_bounds__(PlanT<N>::NB) void k_fft(const Drop* __restrict__ drops, const Work* __restrict__ work,
+                                                      const int* __restrict__ nwork_p, int kstep)
+{
+    __shared__ float2 sx[Xch<N, AXIS>::SIZE];
+    __shared__ float2 stw[N];
+    const int nwork = *nwork_p;
     for (int v = blockIdx.x; v < xcd_span(nwork); v += gridDim.x) {
         const int w = xcd_item(v, nwork);
         if (w >= nwork) continue;
@@ -333,101 +443,58 @@ __global__ __launch_bounds__(PlanT<N>::NB) void k_fft(const Drop* __restrict__ d
         const Drop& D = drops[wk.d];
         if (kstep >= D.nsteps) continue;
         __syncthreads();  // the previous item has read sx and stw
-        // first element of line l
-        size_t base;
-        int lx = 0, ly = 0;  // for the Poisson factor: the line's fixed indices
-        if constexpr (AXIS == 0) {
-            ly = wk.a * L + l;
-            base = ((size_t)wk.b * N + ly) * N;
-        } else if constexpr (AXIS == 1) {
-            lx = wk.a * L + l;
-            base = (size_t)wk.b * N * N + lx;
-        } else {
-            lx = wk.a * L + l;
-            ly = wk.b;
-            base = (size_t)ly * N + lx;
-        }
-        const gptr<float2> c = glb(D.c);
+        fft_lines<N, AXIS, MODE>(D, wk, sx, stw);
+    }
+}
 
-        // the Poisson pass's work item holding kx = ky = 0 sets the k = 0
-        // coefficient from the FP64 sum of s (k_proj_stats)
-        const bool has0 = MODE == FFT_POISSON && wk.a == 0 && wk.b == 0;
-        // the first forward pass divides the imaginary part by sigma (a
-        // power of two: exact)
-        float isg = 1.f;
-        if constexpr (AXIS == 0 && MODE == FFT_FWD) isg = 1.f / glb(D.sigma)[0];
+// The largest work-group and exchange buffer over the size list.
+template <int AXIS, int I = 0>
+constexpr int fft_max_lds()
+{
+    if constexpr (I == kNumGridSizes) return 0;
+    else return std::max(Xch<kGridSizes[I], AXIS>::SIZE, fft_max_lds<AXIS, I + 1>());
+}
+template <int I = 0>
+constexpr int fft_max_threads()
+{
+    if constexpr (I == kNumGridSizes) return 0;
+    else return std::max(PlanT<kGridSizes[I]>::NB, fft_max_threads<I + 1>());
+}
 
-        constexpr int DIR0 = MODE == FFT_INV ? 1 : -1;
-        float2 u[R1 > R2 ? R1 : R2];
-        // ---- step A: R1 threads, length-R2 DFTs -----------------------------
-        // The line's loads are issued before the twiddle table's, so both
-        // are in flight together; the table's LDS stores wait for all of them.
-        if (active && t < R1) {
-#pragma unroll
-            for (int n2 = 0; n2 < R2; ++n2) u[n2] = ld2(c, base + (size_t)(t + R1 * n2) * es);
-        }
-        for (int i = tid; i < N; i += blockDim.x) stw[i] = ld2(glb(D.tw), i);
-        if (active && t < R1) {
-            if constexpr (AXIS == 0 && MODE == FFT_FWD) {
-#pragma unroll
-                for (int n2 = 0; n2 < R2; ++n2) u[n2].y *= isg;
-            }
-            Dft<R2, DIR0>::run(u);
-        }
-        __syncthreads();  // stw
-        if (active && t < R1) {
-#pragma unroll
-            for (int k2 = 0; k2 < R2; ++k2) {
-                const float2 wv = stw[(t * k2) % N];
-                const float2 w2 = f2(wv.x, DIR0 == -1 ? wv.y : -wv.y);
-                sx[X::at(l, t, k2)] = k2 == 0 ? u[0] : mul2(u[k2], w2);
-            }
-        }
-        __syncthreads();
-        // ---- step B: R2 threads, length-R1 DFTs -----------------------------
-        if (active && t < R2) {
-#pragma unroll
-            for (int n1 = 0; n1 < R1; ++n1) u[n1] = sx[X::at(l, n1, t)];
-            Dft<R1, DIR0>::run(u);
-        }
-        if constexpr (MODE != FFT_POISSON) {
-            if (active && t < R2) {
-#pragma unroll
-                for (int k1 = 0; k1 < R1; ++k1) st2(c, base + (size_t)(t + R2 * k1) * es, u[k1]);
-            }
-        } else {
-            // multiply by -1/(k^2 N^3); element index kz = t + R2 k1
-            if (active && t < R2) {
-                const Coef co = D.co;
-#pragma unroll
-                for (int k1 = 0; k1 < R1; ++k1) {
-                    const int kz = t + R2 * k1;
-                    float2 s = u[k1];
-                    if (has0 && l == 0 && kz == 0) s = f2((float)glb(D.stat)[0], (float)glb(D.stat)[1]);
-                    const float m = poisson_factor(co, N, lx, ly, kz);
-                    u[k1] = f2(s.x * m, s.y * m);
-                }
-                // inverse, roles swapped: n' = t + R2 k1, thread t = n1' < R2,
-                // length-R1 DFT over k1 in registers
-                Dft<R1, 1>::run(u);
-            }
-            __syncthreads();  // every thread has read sx in step B
-            if (active && t < R2) {
-#pragma unroll
-                for (int m2 = 0; m2 < R1; ++m2) {
-                    const float2 wv = stw[(t * m2) % N];
-                    sx[X::at(l, m2, t)] = m2 == 0 ? u[0] : mul2(u[m2], f2(wv.x, -wv.y));
-                }
-            }
-            __syncthreads();
-            if (active && t < R1) {
-#pragma unroll
-                for (int n1 = 0; n1 < R2; ++n1) u[n1] = sx[X::at(l, t, n1)];
-                Dft<R2, 1>::run(u);
-#pragma unroll
-                for (int m1 = 0; m1 < R2; ++m1) st2(c, base + (size_t)(t + R1 * m1) * es, u[m1]);
-            }
-        }
+// fft_lines for the droplet's N, one of the size list.
+template <int AXIS, int MODE, int I = 0>
+__device__ __forceinline__ void fft_any(int N, const Drop& D, const Work& wk, float2* sx, float2* stw)
+{
+    if constexpr (I < kNumGridSizes) {
+        if (N == kGridSizes[I]) fft_lines<kGridSizes[I], AXIS, MODE>(D, wk, sx, stw);
+        else fft_any<AXIS, MODE, I + 1>(N, D, wk, sx, stw);
+    }
+}
+
+// One pass over droplets of several sizes in one launch.  A launch of its own
+// per size costs a batch of small droplets more than the transforms: at sizes
+// up to 64^3 a pass takes 4.2 to 5.6 us whatever it holds (six droplets of
+// 32^3 to 64^3: five passes in 20 launches and 100 us, now 5 and 33; the 48^3
+// to 128^3 mix of 20: z pass 78 -> 69 us, the others 31 -> 22 each).  128
+// VGPRs (the z pass would take 142) keep four waves per SIMD.  Each line is
+// transformed by the same operations as in k_fft, so results do not depend on
+// which kernel ran it.
+template <int AXIS, int MODE>
+__global__ __launch_bounds__(fft_max_threads(), 4) void k_fft_sizes(const Drop* __restrict__ drops,
+                                                                const Work* __restrict__ work,
+                                                                const int* __restrict__ nwork_p, int kstep)
+{
+    __shared__ float2 sx[fft_max_lds<AXIS>()];
+    __shared__ float2 stw[kMaxN];
+    const int nwork = *nwork_p;
+    for (int v = blockIdx.x; v < xcd_span(nwork); v += gridDim.x) {
+        const int w = xcd_item(v, nwork);
+        if (w >= nwork) continue;
+        const Work wk = work[w];
+        const Drop& D = drops[wk.d];
+        if (kstep >= D.nsteps) continue;
+        __syncthreads();  // the previous item has read sx and stw
+        fft_any<AXIS, MODE>(D.N, D, wk, sx, stw);
     }
 }
 
@@ -624,6 +691,20 @@ hipError_t launch_fft(int N, int axis, int mode, const Drop* drops, const Work* 
     return with_size(N, [&](auto n) {
         return launch_fft_n<decltype(n)::value>(axis, mode, drops, work, nwork_p, kstep, grid, st);
     });
+}
+
+hipError_t launch_fft_sizes(int axis, int mode, const Drop* drops, const Work* work, const int* nwork_p, int kstep,
+                            int grid, hipStream_t st)
+{
+    if (grid <= 0) return hipSuccess;
+    const dim3 blk(fft_max_threads()), g(grid);
+    if (axis == 0 && mode == FFT_FWD) return launch_kernel(k_fft_sizes<0, FFT_FWD>, g, blk, st, drops, work, nwork_p, kstep);
+    if (axis == 0 && mode == FFT_INV) return launch_kernel(k_fft_sizes<0, FFT_INV>, g, blk, st, drops, work, nwork_p, kstep);
+    if (axis == 1 && mode == FFT_FWD) return launch_kernel(k_fft_sizes<1, FFT_FWD>, g, blk, st, drops, work, nwork_p, kstep);
+    if (axis == 1 && mode == FFT_INV) return launch_kernel(k_fft_sizes<1, FFT_INV>, g, blk, st, drops, work, nwork_p, kstep);
+    if (axis == 2 && mode == FFT_POISSON)
+        return launch_kernel(k_fft_sizes<2, FFT_POISSON>, g, blk, st, drops, work, nwork_p, kstep);
+    return hipErrorInvalidValue;
 }
 
 int fft_lines_per_group(int N)

@@ -52,10 +52,11 @@ enum { KK_RHS = 0, KK_DIV, KK_FX, KK_FY, KK_FZ, KK_FYI, KK_FXI, KK_CORR, KK_N };
 static const char* const kKindNames[KK_N] = {"K_rhs", "K_div", "K_fft_xy", "K_fft_y", "K_fft_z_poisson",
                                              "K_fft_y_inv", "K_fft_xy_inv", "K_corr"};
 
-// Work tables: rhs, div/corr (shared), one item per droplet (the projection's
-// sums), and per grid size the x/y-pass table, the z-pass table and the
-// z-plane table of the fused x+y pass.
-enum { T_RHS = 0, T_PROJ = 1, T_STAT = 2, T_CORR = 3, T_FFT0 = 4 };
+// Work tables: rhs, div, one item per droplet (the projection's sums), corr,
+// the x/y-pass and z-pass tables of a launch that covers several sizes, and
+// per grid size the x/y-pass table, the z-pass table and the z-plane table of
+// the fused x+y pass.
+enum { T_RHS = 0, T_PROJ = 1, T_STAT = 2, T_CORR = 3, T_MXY = 4, T_MZ = 5, T_FFT0 = 6 };
 constexpr int kNTables = T_FFT0 + 3 * kNumGridSizes;
 static_assert(kNumGridSizes <= 32, "sizes are kept as bits of a 32-bit mask");
 static inline int t_xy(int s) { return T_FFT0 + 3 * s; }      // line groups of x or y passes
@@ -147,9 +148,18 @@ struct Engine {
     // graphs, one per starting parity; the sizes present at capture
     hipGraphExec_t gexec[2] = {nullptr, nullptr};
     int ggrid[kNTables] = {};
-    unsigned gsizes = 0;
-    // sizes that run the fused x+y pass (current tables, and at capture)
-    unsigned xy_mask = 0, gxy_mask = 0;
+    // What the FFT launches cover: the sizes present, those that run the fused
+    // x+y pass, and whether the x and y passes of the other sizes, and the z
+    // passes of all, are one launch for several sizes (T_MXY, T_MZ).
+    struct FftLayout {
+        unsigned sizes = 0, xy_mask = 0;
+        bool mxy = false, mz = false;
+        bool covers(const FftLayout& o) const
+        {
+            return !(o.sizes & ~sizes) && xy_mask == o.xy_mask && mxy == o.mxy && mz == o.mz;
+        }
+    };
+    FftLayout fft, gfft;  // of the current tables, and at capture
     int engine_parity = 0;
     int last_chunk = -1;
     bool tables_dirty = true;
@@ -256,8 +266,7 @@ struct Engine {
     {
         for (int p = 0; p < 2; ++p)
             if (gexec[p]) { (void)hipGraphExecDestroy(gexec[p]); gexec[p] = nullptr; }
-        gsizes = 0;
-        gxy_mask = 0;
+        gfft = FftLayout();
     }
 
     void release()
@@ -459,7 +468,7 @@ struct Engine {
         co.gamma = (float)p.gamma;
         co.A = (float)p.A;
         const double kk = 6.283185307179586476925286766559 / (N * h);
-        co.k2s = (float)(kk * kk);
+        co.pk0 = (float)(-1.0 / (kk * kk * (double)N * N * N));
         co.inv_n3 = (float)(1.0 / ((double)N * N * N));
         co.anchoring = (p.A != 0.0) ? 1 : 0;
     }
@@ -681,23 +690,85 @@ struct Engine {
         return active >= 2 && items >= 2 * (int64_t)cus;
     }
 
-    // K_rhs variant of the launches when the batch layout does not apply: the
-    // engine's when a droplet asks for one, else the tuned one of the largest
-    // active droplet, which has most of the work.
-    int lone_variant() const
+    // Tile and z-depths of a launch sequence.  rhs_tz, corr_tz 0: each
+    // droplet's tuned depth.
+    struct Layout {
+        int variant = 0, rhs_tz = 0, corr_tz = 0;
+        bool deep = false;  // the device-filling batch layout: depths are minima
+    };
+
+    // Predicted time of z-chunks of depth d over the active droplets, in
+    // plane iterations of one work-group: `over` iterations of a chunk (planes
+    // beyond its own, loading, launch) come on top of d, `at_once` groups run
+    // together, and a last round that is partly empty counts whole while there
+    // are few rounds.
+    template <typename Tiles>
+    double chunk_time(int d, double over, double at_once, Tiles&& tiles) const
     {
-        int v = rhs_variant < 0 ? 0 : rhs_variant, N = 0;
+        double items = 0.0, deepest = 0.0;
         for (const Slot& s : slots) {
             if (!s.used || remaining(s) <= 0) continue;
-            if (s.prm.rhs_variant >= 0) return rhs_variant;
+            const int nz = (s.N + d - 1) / d;
+            items += (double)tiles(s.N) * nz;
+            deepest = std::max(deepest, (double)((s.N + nz - 1) / nz));
+        }
+        const double rounds = items / at_once;
+        return (rounds < 3.0 ? std::ceil(rounds) : rounds + 0.5) * (deepest + over);
+    }
+
+    // The layout of the next launches.  One droplet: its tuned tile and depths
+    // (the engine's tile if it asks for one).  Several that do not fill the
+    // device: each one's tuned depths would be cut for the whole device, so
+    // that the batch runs several rounds of shallow chunks (six droplets of
+    // 32^3 to 64^3: 62 us in K_rhs); instead the tile and one depth with the
+    // least predicted time (the same six: 36 us).  An iteration takes 3.6 us
+    // with 16 rows and 2.2 with 8, and a chunk about 3 more than it stores;
+    // K_div and K_corr run four groups per CU.
+    Layout layout() const
+    {
+        Layout l;
+        int active = 0, N = 0;
+        bool asked = false;
+        for (const Slot& s : slots) {
+            if (!s.used || remaining(s) <= 0) continue;
+            ++active;
+            asked = asked || s.prm.rhs_variant >= 0;
             if (s.N > N) {
                 N = s.N;
-                v = s.rhs_want;
+                l.variant = s.rhs_want;
             }
         }
-        for (const Slot& s : slots)
-            if (s.used && remaining(s) > 0 && !rhs_fits(v, s.N)) return RHS_16x16;
-        return v;
+        if (asked) l.variant = rhs_variant;
+        if (active < 2) return l;
+        if (batch_layout()) {
+            l.variant = batch_rhs_variant;
+            l.rhs_tz = batch_rhs_tz;
+            l.corr_tz = batch_corr_tz;
+            l.deep = true;
+            return l;
+        }
+        double best = 0.0;
+        for (int v : {(int)RHS_16x16, (int)RHS_16x8}) {
+            if (asked && rhs_rows(v) != rhs_rows(l.variant)) continue;
+            const double unit = rhs_rows(v) == 16 ? 3.6 : 2.2;
+            for (int d = 1; d <= N; ++d) {
+                const double t = unit * chunk_time(d, 3.0, cus, [&](int n) { return rhs_tiles(v, n); });
+                if (l.rhs_tz && t >= best) continue;
+                best = t;
+                l.rhs_tz = d;
+                if (!asked) l.variant = v;
+            }
+        }
+        best = 0.0;
+        for (int d = 1; d <= N; ++d) {
+            const double t = chunk_time(d, 3.0, 4.0 * cus, [&](int n) {
+                return ((n + kProjTX - 1) / kProjTX) * ((n + kProjTY - 1) / kProjTY);
+            });
+            if (l.corr_tz && t >= best) continue;
+            best = t;
+            l.corr_tz = d;
+        }
+        return l;
     }
 
     // Rebuild descriptor and work tables from the active slots.
@@ -708,11 +779,10 @@ struct Engine {
         HIPCHK(uploads_into_st());
         up_pending = false;
         std::vector<Work> w[kNTables];
-        const bool batch = batch_layout();
-        const int rv = batch ? batch_rhs_variant : lone_variant();
-        if (rv != rhs_active) {
+        const Layout lay = layout();
+        if (lay.variant != rhs_active) {
             HIPCHK(hipStreamSynchronize(st));
-            rhs_active = rv;
+            rhs_active = lay.variant;
             drop_graphs();  // captured launches name the tile's kernel
         }
         const int ty = rhs_rows(rhs_active);
@@ -728,7 +798,10 @@ struct Engine {
             if (rem <= 0) continue;
             const int N = s.N;
             // z is split into ceil(N/tz) chunks of near-equal depth
-            const int rtz = batch && !s.rhs_tz_set ? std::min(std::max(s.rhs_tz, batch_rhs_tz), N) : s.rhs_tz;
+            auto depth = [&](int own, int common) {
+                return common <= 0 ? own : std::min(lay.deep ? std::max(own, common) : common, N);
+            };
+            const int rtz = s.rhs_tz_set ? s.rhs_tz : depth(s.rhs_tz, lay.rhs_tz);
             const int nzr = (N + rtz - 1) / rtz;
             for (int k = 0; k < nzr; ++k) {
                 const int zb = k * N / nzr, ze = (k + 1) * N / nzr;
@@ -738,16 +811,17 @@ struct Engine {
             }
             // divergence: the droplet's tuned z-chunks are its reduction blocks
             // (Drop::part); an item covers g consecutive blocks of one tile
-            // (one, except in a device-filling batch)
+            // (one, except in a batch)
             const int ntile = ((N + kProjTX - 1) / kProjTX) * ((N + kProjTY - 1) / kProjTY);
             const int nzp = (N + s.proj_tz - 1) / s.proj_tz;
-            const int g = batch && s.prm.corr_tz <= 0 ? std::max(1, std::min(nzp, batch_corr_tz * nzp / N)) : 1;
+            const int pdepth = s.prm.corr_tz > 0 ? 0 : lay.corr_tz;
+            const int g = pdepth > 0 ? std::max(1, std::min(nzp, pdepth * nzp / N)) : 1;
             for (int k0 = 0; k0 < nzp; k0 += g) {
                 const int k1 = std::min(nzp, k0 + g);
                 const int zb = k0 * N / nzp, ze = k1 * N / nzp;
                 for (int t = 0; t < ntile; ++t) w[T_PROJ].push_back(Work{si, t, zb | (ze << 16), k0 * ntile + t});
             }
-            const int ctz = batch && s.prm.corr_tz <= 0 ? std::min(std::max(s.proj_tz, batch_corr_tz), N) : s.proj_tz;
+            const int ctz = depth(s.proj_tz, pdepth);
             const int nzc = (N + ctz - 1) / ctz;
             for (int k = 0; k < nzc; ++k) {
                 const int zb = k * N / nzc, ze = (k + 1) * N / nzc;
@@ -768,6 +842,29 @@ struct Engine {
                 }
             }
         }
+        // The fused x+y pass puts one work-group on each z-plane; it pays only
+        // when a size has enough planes to give every CU two of them (a
+        // batch), otherwise the per-plane transform work leaves CUs idle and
+        // the single-axis passes are faster.
+        fft = FftLayout();
+        for (int sz = 0; sz < kNumGridSizes; ++sz) {
+            if (!w[t_z(sz)].empty()) fft.sizes |= 1u << sz;
+            if (w[t_pl(sz)].size() >= 2 * (size_t)cus) fft.xy_mask |= 1u << sz;
+        }
+        // Several sizes share one launch per pass (k_fft_sizes), the largest
+        // first: a launch costs at least 4 us, as much as the pass itself for
+        // one small droplet.
+        auto several = [](unsigned m) { return (m & (m - 1)) != 0; };
+        fft.mxy = several(fft.sizes & ~fft.xy_mask);
+        fft.mz = several(fft.sizes);
+        auto merge = [&](int to, int from) {
+            w[to].insert(w[to].end(), w[from].begin(), w[from].end());
+            w[from].clear();
+        };
+        for (int sz = kNumGridSizes - 1; sz >= 0; --sz) {
+            if (fft.mxy && !((fft.xy_mask >> sz) & 1u)) merge(T_MXY, t_xy(sz));
+            if (fft.mz) merge(T_MZ, t_z(sz));
+        }
         for (int k = 0; k < kNTables; ++k) {
             const int cnt = (int)w[k].size();
             if (cnt > tab[k].cap) {
@@ -783,27 +880,12 @@ struct Engine {
             tab[k].n = cnt;
             h_counts[k] = cnt;
         }
-        // The fused x+y pass puts one work-group on each z-plane; it pays only
-        // when a size has enough planes to give every CU two of them (a
-        // batch), otherwise the per-plane transform work leaves CUs idle and
-        // the single-axis passes are faster.
-        xy_mask = 0;
-        for (int sz = 0; sz < kNumGridSizes; ++sz)
-            if (tab[t_pl(sz)].n >= 2 * cus) xy_mask |= 1u << sz;
         HIPCHK(hipMemcpyAsync(d_counts, h_counts, sizeof(int) * kNTables, hipMemcpyHostToDevice, st));
         HIPCHK(hipMemcpyAsync(d_drops, h_drops.data(), sizeof(Drop) * slots.size(), hipMemcpyHostToDevice, st));
         HIPCHK(hipStreamSynchronize(st));  // host tables must outlive the copies
         tables_dirty = false;
         last_chunk = steps_this_call;
         return TTSH_OK;
-    }
-
-    unsigned sizes_present() const
-    {
-        unsigned m = 0;
-        for (int s = 0; s < kNumGridSizes; ++s)
-            if (tab[t_z(s)].n > 0) m |= 1u << s;
-        return m;
     }
 
     // One step's launches.  graph: use the captured fixed grids.  ev (2*KK_N
@@ -815,14 +897,14 @@ struct Engine {
     {
         // plain launches: one work-group per visit of the XCD-blocked order
         auto grid = [&](int t) { return graph ? ggrid[t] : ((tab[t].n + kXcds - 1) / kXcds) * kXcds; };
-        auto on = [&](int s) { return graph ? ((gsizes >> s) & 1u) != 0 : tab[t_z(s)].n > 0; };
+        const FftLayout& fl = graph ? gfft : fft;
         const int* cnt = d_counts;
         // the launches of the step in order, with their kind
         struct L {
             int kind, what, s, t;
         };
-        enum { W_RHS, W_DIV, W_STAT, W_FFT, W_FFT_XY, W_CORR };
-        L list[4 + 5 * kNumGridSizes];
+        enum { W_RHS, W_DIV, W_STAT, W_FFT, W_FFT_SIZES, W_FFT_XY, W_CORR };
+        L list[4 + 5 * (kNumGridSizes + 1)];
         int nl = 0;
         auto add = [&](int kind, int what, int s, int t) {
             if (grid(t) > 0) list[nl++] = L{kind, what, s, t};
@@ -834,16 +916,18 @@ struct Engine {
         // pass do x+y in the x slots and nothing in the y slots
         const int axes[5] = {0, 1, 2, 1, 0};
         const int modes[5] = {FFT_MODE_FWD, FFT_MODE_FWD, FFT_MODE_POISSON, FFT_MODE_INV, FFT_MODE_INV};
-        for (int f = 0; f < 5; ++f)
+        for (int f = 0; f < 5; ++f) {
+            const bool z = axes[f] == 2;
+            if (z ? fl.mz : fl.mxy) add(KK_FX + f, W_FFT_SIZES, 0, z ? T_MZ : T_MXY);
             for (int s = 0; s < kNumGridSizes; ++s) {
-                if (!on(s)) continue;
-                const bool fused = (((graph ? gxy_mask : xy_mask) >> s) & 1u) != 0;
-                if (axes[f] != 2 && fused) {
+                if (!((fl.sizes >> s) & 1u)) continue;
+                if (!z && ((fl.xy_mask >> s) & 1u)) {
                     if (axes[f] == 0) add(KK_FX + f, W_FFT_XY, s, t_pl(s));
                     continue;
                 }
-                add(KK_FX + f, W_FFT, s, axes[f] == 2 ? t_z(s) : t_xy(s));
+                if (!(z ? fl.mz : fl.mxy)) add(KK_FX + f, W_FFT, s, z ? t_z(s) : t_xy(s));
             }
+        }
         add(KK_CORR, W_CORR, 0, T_CORR);
         if (launched)
             for (int k = 0; k < KK_N; ++k) launched[k] = false;
@@ -862,6 +946,7 @@ struct Engine {
             case W_DIV: e = launch_div(d_drops, tab[T_PROJ].d, cnt + T_PROJ, parity, kstep, grid(T_PROJ), st); break;
             case W_STAT: e = launch_proj_stats(d_drops, tab[T_STAT].d, cnt + T_STAT, kstep, grid(T_STAT), st); break;
             case W_FFT_XY: e = launch_fft_xy(N, modes[f], d_drops, tab[l.t].d, cnt + l.t, kstep, grid(l.t), st); break;
+            case W_FFT_SIZES: e = launch_fft_sizes(axes[f], modes[f], d_drops, tab[l.t].d, cnt + l.t, kstep, grid(l.t), st); break;
             case W_FFT: e = launch_fft(N, axes[f], modes[f], d_drops, tab[l.t].d, cnt + l.t, kstep, grid(l.t), st); break;
             default: e = launch_corr(d_drops, tab[T_CORR].d, cnt + T_CORR, parity, kstep, grid(T_CORR), st); break;
             }
@@ -876,12 +961,12 @@ struct Engine {
         // fixed grids: enough work-groups to fill the device, never more than
         // a table can hold
         for (int t = 0; t < kNTables; ++t) ggrid[t] = std::max(0, std::min(tab[t].cap, cus * 8));
-        // the stencil kernels' items differ in cost (z-depths, partial tiles):
-        // one work-group per table slot leaves their balance to the hardware
-        // dispatcher instead of a fixed stride over the items
-        for (int t : {T_RHS, T_PROJ, T_CORR}) ggrid[t] = ((tab[t].cap + kXcds - 1) / kXcds) * kXcds;
-        gsizes = sizes_present();
-        gxy_mask = xy_mask;
+        // the stencil kernels' items differ in cost (z-depths, partial tiles),
+        // as do FFT items of several sizes: one work-group per table slot
+        // leaves their balance to the hardware dispatcher instead of a fixed
+        // stride over the items
+        for (int t : {T_RHS, T_PROJ, T_CORR, T_MXY, T_MZ}) ggrid[t] = ((tab[t].cap + kXcds - 1) / kXcds) * kXcds;
+        gfft = fft;
         hipGraph_t graph = nullptr;
         HIPCHK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
         int rc = TTSH_OK;
@@ -965,12 +1050,10 @@ struct Engine {
                 if (rc) return rc;
             }
             if (g) {
-                if ((sizes_present() & ~gsizes) || xy_mask != gxy_mask) drop_graphs();
+                if (!gfft.covers(fft)) drop_graphs();
                 if (!gexec[engine_parity]) {
-                    const unsigned keep = gsizes;
                     int rc = capture(engine_parity);
                     if (rc) return rc;
-                    (void)keep;
                 }
                 HIPCHK(hipGraphLaunch(gexec[engine_parity], st));
             } else {

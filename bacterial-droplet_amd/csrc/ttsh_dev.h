@@ -44,7 +44,7 @@ struct Coef {
     // f(z-1)+f(z+1) = 6 S_z f - 4 f, so L = lcs*sum_corners S_z f + lcf*sum_corners f
     // + lf*sum_faces f + l0s*S_z f + l0f*f
     float lcs, lcf, l0s, l0f;
-    float k2s;        // (2 pi/(N h))^2: k2 = k2s*(mx^2+my^2+mz^2) (TTSH3D.cu:1094-1114)
+    float pk0;        // -1/(k2s N^3), k2 = k2s*(mx^2+my^2+mz^2), k2s = (2 pi/(N h))^2 (TTSH3D.cu:1094-1114)
     float inv_n3;     // 1/N^3, the type-2 divisor (TTSH3D.cu:687)
     int   anchoring;  // A != 0: evaluate the anchoring term
 };

@@ -71,6 +71,9 @@ hipError_t launch_corr(const Drop* drops, const Work* work, const int* nwork_p, 
 // FFT_MODE_POISSON (z only): forward, times -1/(k^2 N^3), inverse.
 hipError_t launch_fft(int N, int axis, int mode, const Drop* drops, const Work* work, const int* nwork_p, int kstep,
                       int grid, hipStream_t st);
+// The same pass for droplets of any planned sizes in one launch.
+hipError_t launch_fft_sizes(int axis, int mode, const Drop* drops, const Work* work, const int* nwork_p, int kstep,
+                            int grid, hipStream_t st);
 // Lines per FFT work item for size N (0 if N has no plan).
 int fft_lines_per_group(int N);
 // Sizes up to this have the fused x+y pass (one work-group per z-plane,
