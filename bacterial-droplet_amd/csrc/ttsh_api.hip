@@ -31,6 +31,7 @@
 
 #include "../../include/ttsh3d.h"
 #include "ttsh_dev.h"
+#include "ttsh_hostcopy.h"
 #include "ttsh_internal.h"
 #include "ttsh_kernels.h"
 
@@ -187,6 +188,7 @@ struct Engine {
     std::vector<Pooled> pool;
     size_t pooled = 0;
     Drop* d_rdrop = nullptr;  // descriptor of the droplet being reduced
+    HostCopier host_out;      // state out to host arrays
 
     hipStream_t side() const { return us ? us : st; }
 
@@ -290,6 +292,7 @@ struct Engine {
         dev_free(d_rdrop);
         d_rdrop = nullptr;
         if (us) (void)hipStreamSynchronize(us);
+        host_out.release();
         for (auto& b : pool) {
             dev_free(b.mem);
             if (b.ev) (void)hipEventDestroy(b.ev);
@@ -1224,22 +1227,30 @@ struct Engine {
         }
         HIPCHK(hipStreamSynchronize(side()));
         const size_t n = (size_t)s.N * s.N * s.N;
-        std::vector<float> tmp(n);
-        auto get = [&](const float* src, void* dst, size_t off) -> int {
-            if (!dst) return TTSH_OK;
-            if (dtype == TTSH_F32) {
-                HIPCHK(hipMemcpy(static_cast<float*>(dst) + off, src, n * sizeof(float), hipMemcpyDeviceToHost));
-            } else {
-                HIPCHK(hipMemcpy(tmp.data(), src, n * sizeof(float), hipMemcpyDeviceToHost));
-                double* d = static_cast<double*>(dst) + off;
-                for (size_t i = 0; i < n; ++i) d[i] = tmp[i];
-            }
-            return TTSH_OK;
+        const bool f64 = dtype == TTSH_F64;
+        std::vector<HostPiece> pieces;
+        auto want = [&](const float* src, void* dst, size_t off) {
+            if (dst) pieces.push_back(HostPiece{src, static_cast<char*>(dst) + off * (f64 ? 8 : 4), n});
         };
-        int rc = get(s.drop.phi[s.q], phi, 0);
-        for (int a = 0; a < 3 && !rc; ++a) rc = get(s.drop.P[a], P, a * n);
-        for (int a = 0; a < 3 && !rc; ++a) rc = get(s.drop.v[a], v, a * n);
-        return rc;
+        want(s.drop.phi[s.q], phi, 0);
+        for (int a = 0; a < 3; ++a) want(s.drop.P[a], P, a * n);
+        for (int a = 0; a < 3; ++a) want(s.drop.v[a], v, a * n);
+        if (!external && pieces.size() * n * sizeof(float) >= HostCopier::kMinBytes) {
+            bool started = false;
+            HIPCHK(host_out.copy(pieces, f64, side(), &started));
+            if (started) return TTSH_OK;
+        }
+        std::vector<float> tmp(f64 ? n : 0);
+        for (const HostPiece& p : pieces) {
+            if (!f64) {
+                HIPCHK(hipMemcpy(p.dst, p.src, n * sizeof(float), hipMemcpyDeviceToHost));
+                continue;
+            }
+            HIPCHK(hipMemcpy(tmp.data(), p.src, n * sizeof(float), hipMemcpyDeviceToHost));
+            double* d = static_cast<double*>(p.dst);
+            for (size_t i = 0; i < n; ++i) d[i] = tmp[i];
+        }
+        return TTSH_OK;
     }
 
     int reductions(int si, double out[3])
