@@ -19,12 +19,17 @@
 // gives both corrected fields the same relative share, rounded to 2^e,
 // |e| <= 30 (e = 0 when s has no imaginary part or a sum is undefined).
 //
-// Both are z-marching stencils: a work-group owns a TX x TY column and walks
-// a z-range, loading one plane (with a one-cell xy apron) per iteration into
-// LDS and adding the plane's contribution to the three output planes it
-// touches.  With D_a = 1/(2h) d_a (x) S (x) S, S = [1,4,1]/6 (TTSH3D.cu:3280-3328):
-//   D_x f (z) = sum_dz S(dz) [1/(2h) S_y d_x f](z+dz)
-//   D_z f (z) = [1/(2h) S_x S_y f](z+1) - [..](z-1)
+// K_div applies the stencils one axis at a time, like K_rhs (k_rhs.hip): a wave
+// is a row of cells, marching in z with three planes of every value in
+// registers.  With S = [1,4,1], d = [-1,0,1] and s = 1/(72 h),
+// D_x = s d_x S_y S_z, D_y = s S_x d_y S_z, D_z = s S_x S_y d_z
+// (TTSH3D.cu:3280-3328):
+//   z  a = S_z f, b = d_z f
+//   x  X = d_x a, A = S_x a, B = S_x b, by DPP wave shifts
+//   y  4 X + Xm + Xp, Ap - Am, 4 B + Bm + Bp with the rows at y-1 (m) and y+1
+//      (p), whose values come through LDS
+// so a plane costs one barrier (two LDS buffers) and no 2D neighbourhood is
+// read from LDS.  K_corr is a z-marching 2D tile.
 //
 // K_div reproduces the reference's stale halo: an apron or wrapped-plane
 // position, i.e. any position outside the box that the reference reads from
@@ -35,237 +40,196 @@
 
 namespace ttsh {
 
-
-template <int TX, int TY>
-__global__ __launch_bounds__(TX * TY) void k_div(const Drop* __restrict__ drops, const Work* __restrict__ work,
-                                                 const int* __restrict__ nwork_p, int parity, int kstep)
+// Adds to each value the one that DPP control CTRL brings, 0 where none comes.
+template <int CTRL, int N>
+__device__ __forceinline__ void dpp_add(double (&e)[N])
 {
-    constexpr int NT = TX * TY, W1 = TX + 2, A1 = W1 * (TY + 2);
-    __shared__ float sF[6][A1];
-    __shared__ double red[kPartSums * (NT / 64)];
-    const int tid = threadIdx.x, tx = tid % TX, ty = tid / TX;
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+        const unsigned long long b = __double_as_longlong(e[k]);
+        const unsigned lo = __builtin_amdgcn_update_dpp(0, (int)(unsigned)b, CTRL, 0xf, 0xf, false);
+        const unsigned hi = __builtin_amdgcn_update_dpp(0, (int)(unsigned)(b >> 32), CTRL, 0xf, 0xf, false);
+        e[k] += __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+    }
+}
+
+// Sums over a wave, complete in lane 63: row_shr 1, 2, 4, 8 and the two row
+// broadcasts.  Shuffles through LDS would take 72 ds_bpermute, 3 us for the 16
+// waves of a work-group; this takes 0.7.
+template <int N>
+__device__ __forceinline__ void wave_sum(double (&e)[N])
+{
+    dpp_add<0x111>(e);
+    dpp_add<0x112>(e);
+    dpp_add<0x114>(e);
+    dpp_add<0x118>(e);
+    dpp_add<0x142>(e);
+    dpp_add<0x143>(e);
+}
+
+// K_div.  The divergence needs X of the x field, A of the y field and B of the
+// z field; a row's part of its neighbours' sum is U = X + A + B for the row
+// below and W = X - A + B for the row above, so each of the two divergences
+// exchanges two values.
+//
+// Bound by HBM when the device is full.  The 32x8 tile it replaces read 3x3
+// neighbourhoods of six fields from LDS behind two barriers per plane and
+// fetched a 33% ring; here the apron is 64*16/(62*14), 18%.  Waves hold 64
+// VGPRs, so that two work-groups share a CU and one loads while the other
+// waits at its barrier.  Measured with the 4.7 us of k_proj_stats: 96^3 19.5
+// -> 15.8 us, 128^3 26.1 -> 23.1, 180^3 70 -> 53, 256^3 166 -> 149 (637 MB of
+// traffic in 144 us, 4.4 TB/s).
+__global__ __launch_bounds__(64 * kProjWaves, 8) void k_div(const Drop* __restrict__ drops,
+                                                            const Work* __restrict__ work,
+                                                            const int* __restrict__ nwork_p, int parity, int kstep)
+{
+    // every fused multiply-add is written out, so that a cell's result does not
+    // depend on how the loop was compiled
+#pragma clang fp contract(off)
+    __shared__ float4 rec[2][kProjWaves * 64];  // U_v, W_v, U_p, W_p of a row
+    __shared__ double red[kPartSums * kProjWaves];
+    const int lane = threadIdx.x & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int nwork = *nwork_p;
-    for (int v = blockIdx.x; v < xcd_span(nwork); v += gridDim.x) {
-        const int w = xcd_item(v, nwork);
+    for (int vi = blockIdx.x; vi < xcd_span(nwork); vi += gridDim.x) {
+        const int w = xcd_item(vi, nwork);
         if (w >= nwork) continue;
         const Work wk = work[w];
         const Drop& D = drops[wk.d];
         if (kstep >= D.nsteps) continue;
         const int N = D.N;
-        const Coef co = D.co;
-        const int nbx = (N + TX - 1) / TX;
-        const int x0 = (wk.a % nbx) * TX, y0 = (wk.a / nbx) * TY;
+        const int nbx = proj_tiles_x(N), TX = proj_tile_width(N);
+        const int x0 = (wk.a % nbx) * TX, y0 = (wk.a / nbx) * kProjRows;
         const int zb = wk.b & 0xffff, ze = wk.b >> 16;
         const int pp = D.faithful ? (parity ^ 1) : parity;
-        gptr<const float> cur[6], prv[6];
-#pragma unroll
-        for (int f = 0; f < 3; ++f) {
-            cur[f] = glb<const float>(D.vs[parity][f]);
-            cur[3 + f] = glb<const float>(D.ps[parity][f]);
-            prv[f] = glb<const float>(D.vs[pp][f]);
-            prv[3 + f] = glb<const float>(D.ps[pp][f]);
-        }
-        const int gx = x0 + tx, gy = y0 + ty;
-        const bool own = gx < N && gy < N;
-        const size_t NN = (size_t)N * N;
-        float am[2] = {0.f, 0.f}, ac[2] = {0.f, 0.f}, ap[2] = {0.f, 0.f};
-        // sums over this item's cells (see Drop::part): s in FP64 (the k = 0
-        // coefficient), the squares, which only set sigma, per thread in FP32
-        double q[kPartSums] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-        float q2 = 0.f, q3 = 0.f, q4 = 0.f, q5 = 0.f;
-        // Per field, the current and the previous-step buffer are addressed
-        // from the lower of the two (uniform base lo[f]) with a per-lane byte
-        // offset that adds the distance dh[f] to reach the higher one.  Every
-        // load is then one scalar-base load; the buffers of a droplet share
-        // one allocation, so the distance fits 32 bits.
-        gptr<const float> lo[6];
-        unsigned dh[6];
-        bool prv_hi[6];
+        const unsigned NN = (unsigned)N * (unsigned)N;  // 4 N^3 bytes of a field fit 32 bits
+        // Own cell: lanes 1 .. TX of waves 1 .. 14.  Lanes and rows past the
+        // tile load some cell of the box (x0 + 62 and y0 + 14 are below 2 N).
+        const int gx = x0 + lane - 1, gy = y0 + wv - 1;
+        const bool own = lane >= 1 && lane <= TX && gx < N && wv >= 1 && wv <= kProjRows && gy < N;
+        const bool outside = gx < 0 || gx >= N || gy < 0 || gy >= N;
+        const unsigned o = 4u * ((unsigned)wrapi(gy, N) * (unsigned)N + (unsigned)wrapi(gx, N));
+        // Per field, the current and the previous step's buffer are addressed
+        // from the lower of the two (scalar base) with a per-lane byte offset
+        // that adds the distance to reach the higher one; the buffers of a
+        // droplet share one allocation, so the distance fits 32 bits.  In the
+        // stale-halo mode, lanes outside the box in x read the previous step's
+        // x = 0 / x = N-1 columns from the edge buffer (same z-stride as a
+        // field, so the same scalar base serves; K_corr writes each step's
+        // columns).  A plane outside the box in z is read wholly from the
+        // previous step's buffers.
+        gptr<const float> lo[6], prv[6];
+        unsigned off[6];
+        const bool xedge = D.faithful != 0 && (gx < 0 || gx >= N);
+        const unsigned col = 4u * (unsigned)((D.eslot[pp] * 12 + (gx < 0 ? 1 : 0)) * N + wrapi(gy, N));
 #pragma unroll
         for (int f = 0; f < 6; ++f) {
-            prv_hi[f] = prv[f] > cur[f];
-            lo[f] = prv_hi[f] ? cur[f] : prv[f];
-            dh[f] = 4u * (unsigned)(prv_hi[f] ? prv[f] - cur[f] : cur[f] - prv[f]);
+            const gptr<const float> c = glb<const float>(f < 3 ? D.vs[parity][f] : D.ps[parity][f - 3]);
+            prv[f] = glb<const float>(f < 3 ? D.vs[pp][f] : D.ps[pp][f - 3]);
+            const bool hi = prv[f] > c;
+            lo[f] = hi ? c : prv[f];
+            const unsigned dist = 4u * (unsigned)(hi ? prv[f] - c : c - prv[f]);
+            off[f] = xedge ? 4u * (unsigned)(glb<const float>(D.edge) - lo[f]) + col + 8u * (unsigned)(f * N)
+                           : o + (outside == hi ? dist : 0u);
         }
-        // In the stale-halo mode, positions outside the box in x read the
-        // previous step's x = 0 / x = N-1 columns from the edge buffer (same
-        // z-stride as a field, so the same scalar base serves; K_corr writes
-        // each step's columns).
-        const bool xedge = D.faithful != 0;
-        const int eprev = D.eslot[pp];
-        // Loads: the thread's own cell, one per field (a wave loads two whole
-        // aligned rows), and the one-cell ring around the tile (top row,
-        // bottom row, left and right column) as RING x 6 (position, field)
-        // pairs spread over two loads per thread.  Ring loads address every
-        // field from gb, the lowest of the droplet's predictor buffers (one
-        // allocation, with the edge buffer after them: 32-bit offsets).
-        constexpr int RING = 2 * W1 + 2 * TY;
-        static_assert(A1 - NT == RING && 6 * RING <= 2 * NT, "two ring loads per thread");
-        gptr<const float> gb = lo[0];
+        float q[6][3];
+        auto fetch = [&](int slot, int z) {
+            const unsigned zo = (unsigned)wrapi(z, N) * NN;
+            if (z >= 0 && z < N) {
 #pragma unroll
-        for (int f = 1; f < 6; ++f) gb = lo[f] < gb ? lo[f] : gb;
-        auto pos = [&](int i, bool& sxy, int& ex, int& ey) {
-            ex = x0 - 1 + i % W1;
-            ey = y0 - 1 + i / W1;
-            sxy = ex < 0 || ex >= N || ey < 0 || ey >= N;
-            return 4u * ((unsigned)wrapi(ey, N) * (unsigned)N + (unsigned)wrapi(ex, N));
-        };
-        // byte offset of field f's value at position (ex, ey) from base b:
-        // the current or previous buffer (stale: outside the box, or the
-        // whole plane when wz), or the edge buffer for x outside the box
-        auto foff = [&](int f, gptr<const float> b, unsigned o, bool stale, int ex, int ey) {
-            if (xedge && (ex < 0 || ex >= N)) {
-                const int col = ((eprev * 6 + f) * 2 + (ex < 0 ? 1 : 0)) * N + wrapi(ey, N);
-                return 4u * (unsigned)(glb<const float>(D.edge) - b) + 4u * (unsigned)col;
-            }
-            return 4u * (unsigned)(lo[f] - b) + o + ((stale == prv_hi[f]) ? dh[f] : 0u);
-        };
-        unsigned own_o[6], own_w[6];  // own cell: normal plane, whole-plane-stale plane
-        bool own_in;
-        {
-            bool sxy;
-            int ex, ey;
-            const unsigned o = pos((ty + 1) * W1 + (tx + 1), sxy, ex, ey);
-            own_in = !sxy;
-#pragma unroll
-            for (int f = 0; f < 6; ++f) {
-                own_o[f] = foff(f, lo[f], o, sxy, ex, ey);
-                own_w[f] = foff(f, lo[f], o, true, ex, ey);
-            }
-        }
-        unsigned ring_o[2], ring_w[2];
-        int ring_l[2];  // flat LDS index f*A1 + i (-1: past the last pair)
-#pragma unroll
-        for (int m = 0; m < 2; ++m) {
-            const int j = min(tid + m * NT, 6 * RING - 1), f = j / RING, r = j % RING;
-            int i;
-            if (r < W1) i = r;                                      // row y0-1
-            else if (r < 2 * W1) i = (TY + 1) * W1 + (r - W1);      // row y0+TY
-            else if (r < 2 * W1 + TY) i = (r - 2 * W1 + 1) * W1;    // column x0-1
-            else i = (r - 2 * W1 - TY + 1) * W1 + (W1 - 1);         // column x0+TX
-            bool sxy;
-            int ex, ey;
-            const unsigned o = pos(i, sxy, ex, ey);
-            ring_o[m] = foff(f, gb, o, sxy, ex, ey);
-            ring_w[m] = foff(f, gb, o, true, ex, ey);
-            ring_l[m] = tid + m * NT < 6 * RING ? f * A1 + i : -1;
-        }
-        // planes are loaded two ahead, into two register slots; a plane
-        // outside the box (wrapped in z) is read wholly from the previous step
-        float pre[2][8];
-        auto fetch = [&](int slot, int zi) {
-            const size_t zo = (size_t)wrapi(zi, N) * NN;
-            if (zi >= 0 && zi < N) {
-#pragma unroll
-                for (int f = 0; f < 6; ++f) pre[slot][f] = ldb(lo[f] + zo, own_o[f]);
-#pragma unroll
-                for (int m = 0; m < 2; ++m) pre[slot][6 + m] = ldb(gb + zo, ring_o[m]);
+                for (int f = 0; f < 6; ++f) q[f][slot] = ldb(lo[f] + zo, opaque(off[f]));
             } else {
+                const unsigned oo = opaque(o);
 #pragma unroll
-                for (int f = 0; f < 6; ++f) pre[slot][f] = ldb(lo[f] + zo, own_w[f]);
-#pragma unroll
-                for (int m = 0; m < 2; ++m) pre[slot][6 + m] = ldb(gb + zo, ring_w[m]);
+                for (int f = 0; f < 6; ++f) q[f][slot] = ldb(prv[f] + zo, oo);
             }
         };
+        // sums over this item's cells (see Drop::part): s in FP64 (the k = 0
+        // coefficient), the squares, which only set sigma, per thread in FP32
+        double d0 = 0.0, d1 = 0.0;
+        float q2 = 0.f, q3 = 0.f, q4 = 0.f, q5 = 0.f;
         // The sums are written per reduction block (see Drop::part): the
         // item starts at block wk.c, and at the last plane of each block the
         // work-group reduces them in a fixed order and starts the next.  The
         // sums of a block are then the same whichever item covers it.
-        const int ntile = nbx * ((N + TY - 1) / TY);
+        const int ntile = proj_tiles(N);
         int ordb = wk.c;
         int zend = (wk.c / ntile + 1) * N / D.nzp;
         auto flush = [&]() {
-            q[2] = q2;
-            q[3] = q3;
-            q[4] = q4;
-            q[5] = q5;
+            double e[kPartSums] = {d0, d1, q2, q3, q4, q5};
+            wave_sum(e);
+            __syncthreads();  // the previous block's sums were read
+            if (lane == 63) {
 #pragma unroll
-            for (int off = 32; off > 0; off >>= 1) {
-#pragma unroll
-                for (int e = 0; e < kPartSums; ++e) q[e] += __shfl_down(q[e], off, 64);
+                for (int k = 0; k < kPartSums; ++k) red[kPartSums * wv + k] = e[k];
             }
             __syncthreads();
-            if ((tid & 63) == 0) {
-#pragma unroll
-                for (int e = 0; e < kPartSums; ++e) red[kPartSums * (tid >> 6) + e] = q[e];
-            }
-            __syncthreads();
-            if (tid < kPartSums) {
+            if (threadIdx.x < kPartSums) {
                 double a = 0.0;
-                for (int i = 0; i < NT / 64; ++i) a += red[kPartSums * i + tid];
-                glb(D.part)[(size_t)kPartSums * ordb + tid] = a;
-            }
 #pragma unroll
-            for (int e = 0; e < kPartSums; ++e) q[e] = 0.0;
+                for (int i = 0; i < kProjWaves; ++i) a += red[kPartSums * i + threadIdx.x];
+                glb(D.part)[(size_t)kPartSums * ordb + threadIdx.x] = a;
+            }
+            d0 = d1 = 0.0;
             q2 = q3 = q4 = q5 = 0.f;
             ordb += ntile;
             zend = (ordb / ntile + 1) * N / D.nzp;
         };
-        auto body = [&](auto ph, int zi) {
-            constexpr int S = decltype(ph)::value;
-            // squares of this plane's inputs, added after the block check below
-            float sq4 = 0.f, sq5 = 0.f;
-            const bool sq = zi >= zb && zi < ze && own_in;
-            if (sq) {
-                const float* u = pre[S];
-                sq4 = u[0] * u[0] + u[1] * u[1] + u[2] * u[2];
-                sq5 = u[3] * u[3] + u[4] * u[4] + u[5] * u[5];
-            }
-            __syncthreads();
-            {
-                const int i = (ty + 1) * W1 + (tx + 1);
-#pragma unroll
-                for (int f = 0; f < 6; ++f) sF[f][i] = pre[S][f];
-#pragma unroll
-                for (int m = 0; m < 2; ++m)
-                    if (ring_l[m] >= 0) (&sF[0][0])[ring_l[m]] = pre[S][6 + m];
-            }
-            fetch(S, min(zi + 2, ze));  // past ze: a redundant reload of plane ze
-            __syncthreads();
-            const int o = (ty + 1) * W1 + (tx + 1);
+        // D.v*/dt0 and D.P*/dt0 of a cell
+        const float scale = D.co.d1 * (1.f / 36.f) * D.co.inv_dt0;
+        const unsigned oc = 2u * o;
+        int buf = 0;
+        const int own_i = wv * 64 + lane;
+        const int below = max(wv - 1, 0) * 64 + lane, above = min(wv + 1, kProjWaves - 1) * 64 + lane;
+        auto body = [&](auto ph, int zm) {
+            constexpr int S0 = decltype(ph)::value, S1 = (S0 + 1) % 3, S2 = (S0 + 2) % 3;
+            float xb[2], u[2], v[2];
 #pragma unroll
             for (int F = 0; F < 2; ++F) {
-                const float* fx = sF[3 * F];
-                const float* fy = sF[3 * F + 1];
-                const float* fz = sF[3 * F + 2];
-                const float ax = co.sw0 * (fx[o + 1] - fx[o - 1])
-                               + co.sw1 * ((fx[o - W1 + 1] - fx[o - W1 - 1]) + (fx[o + W1 + 1] - fx[o + W1 - 1]));
-                const float ay = co.sw0 * (fy[o + W1] - fy[o - W1])
-                               + co.sw1 * ((fy[o + W1 - 1] - fy[o - W1 - 1]) + (fy[o + W1 + 1] - fy[o - W1 + 1]));
-                const float r0 = co.sw0 * fz[o] + co.sw1 * (fz[o - 1] + fz[o + 1]);
-                const float rm = co.sw0 * fz[o - W1] + co.sw1 * (fz[o - W1 - 1] + fz[o - W1 + 1]);
-                const float rp = co.sw0 * fz[o + W1] + co.sw1 * (fz[o + W1 - 1] + fz[o + W1 + 1]);
-                const float A = co.d1 * (ax + ay);
-                const float B = co.d1 * (co.sw0 * r0 + co.sw1 * (rm + rp));
-                am[F] += co.sw1 * A + B;
-                ac[F] += co.sw0 * A;
-                ap[F] += co.sw1 * A - B;
+                const float* fx = q[3 * F];
+                const float* fy = q[3 * F + 1];
+                const float* fz = q[3 * F + 2];
+                const float ax = fma_(4.f, fx[S1], fx[S0] + fx[S2]);
+                const float ay = fma_(4.f, fy[S1], fy[S0] + fy[S2]);
+                const float b = fz[S2] - fz[S0];
+                const float A = fma_(4.f, ay, xpair(ay));
+                xb[F] = xdiff(ax) + fma_(4.f, b, xpair(b));
+                u[F] = xb[F] + A;
+                v[F] = xb[F] - A;
             }
-            const int zo = zi - 1;
-            if (zo >= zb && own) {
-                const float2 sv = make_float2(am[0] * co.inv_dt0, am[1] * co.inv_dt0);
-                st2(glb(D.c), gidx(N, gx, gy, zo), sv);
-                q[0] += (double)sv.x;
-                q[1] += (double)sv.y;
-                q2 += sv.x * sv.x;
-                q3 += sv.y * sv.y;
+            rec[buf][own_i] = make_float4(u[0], v[0], u[1], v[1]);
+            if (own) {
+                q4 = fma_(q[0][S1], q[0][S1], fma_(q[1][S1], q[1][S1], fma_(q[2][S1], q[2][S1], q4)));
+                q5 = fma_(q[3][S1], q[3][S1], fma_(q[4][S1], q[4][S1], fma_(q[5][S1], q[5][S1], q5)));
             }
-            if (zo >= zb && zo == zend - 1) flush();  // uniform across the work-group
-            if (sq) {
-                q4 += sq4;
-                q5 += sq5;
+            fetch(S0, min(zm + 2, ze));  // past ze: a redundant reload of plane ze
+            __syncthreads();
+            const float4 m = rec[buf][below], p = rec[buf][above];
+            buf ^= 1;
+            if (own) {
+                fvec2 sv;
+                sv.x = scale * fma_(4.f, xb[0], m.y + p.x);
+                sv.y = scale * fma_(4.f, xb[1], m.w + p.z);
+                *(gptr<fvec2>)((gptr<char>)(D.c + (unsigned)zm * NN) + opaque(oc)) = sv;
+                d0 += (double)sv.x;
+                d1 += (double)sv.y;
+                q2 = fma_(sv.x, sv.x, q2);
+                q3 = fma_(sv.y, sv.y, q3);
             }
-#pragma unroll
-            for (int F = 0; F < 2; ++F) { am[F] = ac[F]; ac[F] = ap[F]; ap[F] = 0.f; }
+            if (zm == zend - 1) flush();  // uniform across the work-group
         };
         fetch(0, zb - 1);
         fetch(1, zb);
+        fetch(2, zb + 1);
         wait_vmem();
-        for (int zi = zb - 1;;) {
-            body(Ph<0>{}, zi);
-            if (++zi > ze) break;
-            body(Ph<1>{}, zi);
-            if (++zi > ze) break;
+        __syncthreads();  // the previous item has read both buffers
+        for (int zm = zb;;) {
+            body(Ph<0>{}, zm);
+            if (++zm >= ze) break;
+            body(Ph<1>{}, zm);
+            if (++zm >= ze) break;
+            body(Ph<2>{}, zm);
+            if (++zm >= ze) break;
         }
         // the item ends at a block end, so its last block was written above
     }
@@ -341,6 +305,13 @@ __global__ __launch_bounds__(kStatsThreads) void k_proj_stats(const Drop* __rest
     }
 }
 
+// K_corr: a work-group owns a TX x TY column and walks a z-range, loading one
+// plane of p (with a one-cell xy apron) per iteration into LDS and adding its
+// contribution to the three output planes it touches.  Bound by HBM: 4.8 TB/s
+// of traffic at 256^3, where a copy reaches 5.1.  K_div's row waves measured
+// 197 -> 231 us there (their 52-cell rows end inside cache lines, and six
+// output fields are then written in partial lines), 77 -> 75 at 180^3 and
+// 21 -> 22 at 128^3, so the corrector keeps its aligned 32x8 tile.
 template <int TX, int TY>
 __global__ __launch_bounds__(TX * TY) void k_corr(const Drop* __restrict__ drops, const Work* __restrict__ work,
                                                   const int* __restrict__ nwork_p, int parity, int kstep)
@@ -563,8 +534,7 @@ hipError_t launch_div(const Drop* drops, const Work* work, const int* nwork_p, i
                       hipStream_t st)
 {
     if (grid <= 0) return hipSuccess;
-    return launch_kernel(k_div<kProjTX, kProjTY>, dim3(grid), dim3(kProjTX * kProjTY), st, drops, work, nwork_p,
-                         parity, kstep);
+    return launch_kernel(k_div, dim3(grid), dim3(64 * kProjWaves), st, drops, work, nwork_p, parity, kstep);
 }
 
 hipError_t launch_proj_stats(const Drop* drops, const Work* work, const int* nwork_p, int kstep, int grid,
@@ -620,7 +590,7 @@ hipError_t launch_corr(const Drop* drops, const Work* work, const int* nwork_p, 
                        hipStream_t st)
 {
     if (grid <= 0) return hipSuccess;
-    return launch_kernel(k_corr<kProjTX, kProjTY>, dim3(grid), dim3(kProjTX * kProjTY), st, drops, work, nwork_p,
+    return launch_kernel(k_corr<kCorrTX, kCorrTY>, dim3(grid), dim3(kCorrTX * kCorrTY), st, drops, work, nwork_p,
                          parity, kstep);
 }
 

@@ -74,32 +74,9 @@ namespace ttsh {
 
 typedef float fvec4 __attribute__((ext_vector_type(4)));
 
-__device__ __forceinline__ float fma_(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
-
 // Keeps the compiler from sinking a value's computation past this point: sunk
 // past a barrier, all its inputs would stay live instead of the one value.
 __device__ __forceinline__ void pin(float& a) { asm volatile("" : "+v"(a)); }
-
-// A value that the compiler cannot derive, so that a global access keeps its
-// scalar base and 32-bit lane offset instead of a hoisted 64-bit address.
-__device__ __forceinline__ unsigned opaque(unsigned a)
-{
-    asm volatile("" : "+v"(a));
-    return a;
-}
-
-// The value of the lane at x-1 / x+1 (DPP wave_shr:1, wave_shl:1; 0 past the
-// ends of the wave, whose lanes are apron).
-__device__ __forceinline__ float from_left(float a)
-{
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(a), 0x138, 0xf, 0xf, true));
-}
-__device__ __forceinline__ float from_right(float a)
-{
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(a), 0x130, 0xf, 0xf, true));
-}
-__device__ __forceinline__ float xpair(float a) { return from_left(a) + from_right(a); }
-__device__ __forceinline__ float xdiff(float a) { return from_right(a) - from_left(a); }
 
 // A row of one field after its z and x stages; X, A, B, E are the record that
 // the neighbouring rows read.

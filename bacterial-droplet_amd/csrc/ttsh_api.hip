@@ -76,7 +76,7 @@ static inline size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 // Upper bound of divergence work items of one droplet (z-depth >= 1).
 static int proj_items_max(int N)
 {
-    return ((N + kProjTX - 1) / kProjTX) * ((N + kProjTY - 1) / kProjTY) * N;
+    return proj_tiles(N) * N;
 }
 
 size_t droplet_bytes(int N)
@@ -89,6 +89,9 @@ size_t droplet_bytes(int N)
 
 // K_rhs variant of a size without a tuning entry; 16x16 fits every supported N.
 static int default_rhs_variant(int) { return RHS_16x16; }
+
+// K_corr work items of one z-range.
+static int corr_tiles(int N) { return ((N + kCorrTX - 1) / kCorrTX) * ((N + kCorrTY - 1) / kCorrTY); }
 
 // K_rhs work items of one z-range.
 static int rhs_tiles(int variant, int N) { return rhs_tiles_x(N) * ((N + rhs_rows(variant) - 1) / rhs_rows(variant)); }
@@ -693,10 +696,10 @@ struct Engine {
         return active >= 2 && items >= 2 * (int64_t)cus;
     }
 
-    // Tile and z-depths of a launch sequence.  rhs_tz, corr_tz 0: each
-    // droplet's tuned depth.
+    // Tile and z-depths of a launch sequence.  Depth 0: each droplet's tuned
+    // depth.
     struct Layout {
-        int variant = 0, rhs_tz = 0, corr_tz = 0;
+        int variant = 0, rhs_tz = 0, div_tz = 0, corr_tz = 0;
         bool deep = false;  // the device-filling batch layout: depths are minima
     };
 
@@ -726,7 +729,7 @@ struct Engine {
     // 32^3 to 64^3: 62 us in K_rhs); instead the tile and one depth with the
     // least predicted time (the same six: 36 us).  An iteration takes 3.6 us
     // with 16 rows and 2.2 with 8, and a chunk about 3 more than it stores;
-    // K_div and K_corr run four groups per CU.
+    // K_div runs two groups per CU, K_corr four.
     Layout layout() const
     {
         Layout l;
@@ -746,7 +749,7 @@ struct Engine {
         if (batch_layout()) {
             l.variant = batch_rhs_variant;
             l.rhs_tz = batch_rhs_tz;
-            l.corr_tz = batch_corr_tz;
+            l.div_tz = l.corr_tz = batch_corr_tz;
             l.deep = true;
             return l;
         }
@@ -762,15 +765,14 @@ struct Engine {
                 if (!asked) l.variant = v;
             }
         }
-        best = 0.0;
-        for (int d = 1; d <= N; ++d) {
-            const double t = chunk_time(d, 3.0, 4.0 * cus, [&](int n) {
-                return ((n + kProjTX - 1) / kProjTX) * ((n + kProjTY - 1) / kProjTY);
-            });
-            if (l.corr_tz && t >= best) continue;
-            best = t;
-            l.corr_tz = d;
-        }
+        auto least = [&](double at_once, int (*tiles)(int)) {
+            int d = 1;
+            for (int k = 2; k <= N; ++k)
+                if (chunk_time(k, 3.0, at_once, tiles) < chunk_time(d, 3.0, at_once, tiles)) d = k;
+            return d;
+        };
+        l.div_tz = least(2.0 * cus, [](int n) { return proj_tiles(n); });
+        l.corr_tz = least(4.0 * cus, corr_tiles);
         return l;
     }
 
@@ -815,20 +817,26 @@ struct Engine {
             // divergence: the droplet's tuned z-chunks are its reduction blocks
             // (Drop::part); an item covers g consecutive blocks of one tile
             // (one, except in a batch)
-            const int ntile = ((N + kProjTX - 1) / kProjTX) * ((N + kProjTY - 1) / kProjTY);
+            const int ntile = proj_tiles(N);
             const int nzp = (N + s.proj_tz - 1) / s.proj_tz;
-            const int pdepth = s.prm.corr_tz > 0 ? 0 : lay.corr_tz;
-            const int g = pdepth > 0 ? std::max(1, std::min(nzp, pdepth * nzp / N)) : 1;
+            const int dtz = s.prm.corr_tz > 0 ? 0 : lay.div_tz;
+            const int g = dtz > 0 ? std::max(1, std::min(nzp, dtz * nzp / N)) : 1;
             for (int k0 = 0; k0 < nzp; k0 += g) {
                 const int k1 = std::min(nzp, k0 + g);
                 const int zb = k0 * N / nzp, ze = k1 * N / nzp;
                 for (int t = 0; t < ntile; ++t) w[T_PROJ].push_back(Work{si, t, zb | (ze << 16), k0 * ntile + t});
             }
-            const int ctz = depth(s.proj_tz, pdepth);
+            // K_corr gains little from chunks deeper than 8 to 16 planes (a
+            // chunk re-reads two planes of p, 16 of its 72 bytes per cell) and
+            // loses from their uneven end: 256^3 195 us at 8, 210 at 32, the
+            // 20-droplet sweep 255 at 12 to 16, 267 at 32
+            const int ctz = s.prm.corr_tz > 0 ? s.proj_tz
+                            : lay.deep        ? depth(std::min(s.proj_tz, 16), std::min(lay.corr_tz, 16))
+                                              : depth(std::min(s.proj_tz, 8), lay.corr_tz);
             const int nzc = (N + ctz - 1) / ctz;
             for (int k = 0; k < nzc; ++k) {
                 const int zb = k * N / nzc, ze = (k + 1) * N / nzc;
-                for (int t = 0; t < ntile; ++t) w[T_CORR].push_back(Work{si, t, zb | (ze << 16), 0});
+                for (int t = 0; t < corr_tiles(N); ++t) w[T_CORR].push_back(Work{si, t, zb | (ze << 16), 0});
             }
             // k_proj_stats sums the blocks' FP64 partial sums in block order
             h_drops[si].npart = nzp * ntile;

@@ -105,6 +105,16 @@ constexpr int kRhsMaxTX = 60;
 __host__ __device__ constexpr int rhs_tiles_x(int N) { return (N + kRhsMaxTX - 1) / kRhsMaxTX; }
 __host__ __device__ constexpr int rhs_tile_width(int N) { return (N + rhs_tiles_x(N) - 1) / rhs_tiles_x(N); }
 
+// Tiles of the divergence: a wave is a row whose 64 lanes
+// include one apron cell on each side, a work-group 16 rows of which the
+// first and last are apron.
+constexpr int kProjWaves = 16;
+constexpr int kProjRows = kProjWaves - 2;
+constexpr int kProjMaxTX = 62;
+__host__ __device__ constexpr int proj_tiles_x(int N) { return (N + kProjMaxTX - 1) / kProjMaxTX; }
+__host__ __device__ constexpr int proj_tile_width(int N) { return (N + proj_tiles_x(N) - 1) / proj_tiles_x(N); }
+__host__ __device__ constexpr int proj_tiles(int N) { return proj_tiles_x(N) * ((N + kProjRows - 1) / kProjRows); }
+
 // Work-groups are dispatched round-robin over the 8 XCDs, each with its own
 // L2.  Visit v of the grid-stride loop maps to work item
 //   (v mod 8) * chunk + v / 8,   chunk = ceil(nwork / 8),
@@ -160,6 +170,29 @@ __device__ __forceinline__ void stb(gptr<float> base, unsigned boff, float v)
 {
     *(gptr<float>)((gptr<char>)base + boff) = v;
 }
+
+// A value that the compiler cannot derive, so that a global access keeps its
+// scalar base and 32-bit lane offset instead of a hoisted 64-bit address.
+__device__ __forceinline__ unsigned opaque(unsigned a)
+{
+    asm volatile("" : "+v"(a));
+    return a;
+}
+
+__device__ __forceinline__ float fma_(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+
+// The value of the lane at x-1 / x+1 of a wave that is a row of cells (DPP
+// wave_shr:1, wave_shl:1; 0 past the ends of the wave, whose lanes are apron).
+__device__ __forceinline__ float from_left(float a)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(a), 0x138, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float from_right(float a)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(a), 0x130, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float xpair(float a) { return from_left(a) + from_right(a); }
+__device__ __forceinline__ float xdiff(float a) { return from_right(a) - from_left(a); }
 
 // Compile-time phase of an unrolled z-march (register slot rotation).
 template <int K>

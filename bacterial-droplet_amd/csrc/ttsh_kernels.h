@@ -37,9 +37,9 @@ enum RhsVariant { RHS_32x8 = 0, RHS_16x16 = 1, RHS_64x4 = 2, RHS_16x8 = 3, RHS_3
                   RHS_64x8 = 6, RHS_NVARIANTS = 7 };
 static_assert(RHS_NVARIANTS == kRhsVariants, "tile variant count");
 
-// Tile of the divergence and corrector stencils.
-constexpr int kProjTX = 32;
-constexpr int kProjTY = 8;
+// Tile of the corrector.
+constexpr int kCorrTX = 32;
+constexpr int kCorrTY = 8;
 
 // FFT pass kinds (k_fft.hip).
 enum { FFT_MODE_FWD = 0, FFT_MODE_INV = 1, FFT_MODE_POISSON = 2 };

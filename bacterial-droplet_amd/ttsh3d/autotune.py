@@ -2,7 +2,7 @@
 
 For each grid size N it times, with HIP events through ttsh_profile, the two
 K_rhs kernels (16 and 8 rows per work-group) at several z-depths, and several
-z-depths of the divergence/corrector stencils, on a droplet of that size; then
+z-depths of the divergence stencil, on a droplet of that size; then
 writes the fastest choices as the tuning table libttsh3d.so reads (tuned.txt
 beside the library, lines "N rhs_variant rhs_tz proj_tz").
 
@@ -73,11 +73,11 @@ def tune_size(N: int, steps: int = 30, log=print):
                 break  # too few chunks by now: deeper ones leave more of the device idle
     for ptz in [t for t in PROJ_DEPTHS if t <= N]:
         k = _time(default_params(rhs_variant=best_rhs[0], rhs_tz=best_rhs[1], corr_tz=ptz, **base), state, steps)
-        t = k["K_div"] + k["K_corr"]
+        t = k["K_div"]  # without corr_tz the corrector takes the same depth, or 8 if that is less
         results.append({"kind": "proj", "tz": ptz, "ms": t})
         if best_proj is None or t < best_proj[1]:
             best_proj = (ptz, t)
-        log(f"N={N} K_div+K_corr tz {ptz}: {t * 1e3:.1f} us")
+        log(f"N={N} K_div tz {ptz}: {t * 1e3:.1f} us")
     return (best_rhs[0], best_rhs[1], best_proj[0]), results
 
 
