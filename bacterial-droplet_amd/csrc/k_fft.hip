@@ -18,17 +18,23 @@
 // forward e^{-2 pi i jk/N}, inverse e^{+2 pi i jk/N}, both unnormalised, as
 // cufftExecZ2Z.
 //
-// The first forward pass (x, or the fused x+y) divides the imaginary part of
-// s by the droplet's power-of-two sigma and the z pass takes the k = 0
-// coefficient from the FP64 sum of s; both come from k_proj_stats
-// (Drop::sigma, Drop::stat).
+// Sizes above kMaxPlane run five passes in place: x, y, z (forward, solve,
+// inverse), y, x.  For sizes up to kMaxPlane a y-z plane of N x N complex
+// values fits the LDS of a CU, and one kernel does both y passes and the z
+// pass on it (k_fft_yz); the x passes then write and read a transposed copy
+// (Drop::ct, [x][z][y]), so that a plane is contiguous.  That is three round
+// trips through memory and three launches instead of five.
+//
+// The forward x pass divides the imaginary part of s by the droplet's
+// power-of-two sigma and the z stage takes the k = 0 coefficient from the
+// FP64 sum of s (Drop::sigma, Drop::stat).
 #include "ttsh_dev.h"
 #include "ttsh_kernels.h"
 
-// No multiply-add contraction in this file: every pass then performs the
-// same IEEE operations whichever kernel runs a line (single-axis passes or
-// the fused x+y pass), so a droplet's result does not depend on the batch
-// it runs in.
+// No multiply-add contraction in this file (complex products write theirs
+// out): every pass then performs the
+// same IEEE operations whichever kernel runs a line (that of one size or that
+// of several), so a droplet's result does not depend on the batch it runs in.
 #pragma clang fp contract(off)
 
 namespace ttsh {
@@ -47,7 +53,10 @@ __device__ constexpr float kSin48[12] = {
 __device__ __forceinline__ float2 f2(float a, float b) { return make_float2(a, b); }
 __device__ __forceinline__ float2 add2(float2 a, float2 b) { return f2(a.x + b.x, a.y + b.y); }
 __device__ __forceinline__ float2 sub2(float2 a, float2 b) { return f2(a.x - b.x, a.y - b.y); }
-__device__ __forceinline__ float2 mul2(float2 a, float2 w) { return f2(a.x * w.x - a.y * w.y, a.x * w.y + a.y * w.x); }
+__device__ __forceinline__ float2 mul2(float2 a, float2 w)
+{
+    return f2(__builtin_fmaf(a.x, w.x, -(a.y * w.y)), __builtin_fmaf(a.x, w.y, a.y * w.x));
+}
 
 // a * exp(i 2 pi m/48) for a compile-time m (quarter turns are exact swaps).
 template <int M>
@@ -135,7 +144,7 @@ struct Dft<3, DIR> {
     {
         constexpr float c3 = 0.86602540378443864676f;  // sin(2 pi/3)
         const float2 t1 = add2(v[1], v[2]), t2 = sub2(v[1], v[2]);
-        const float2 m = f2(v[0].x - 0.5f * t1.x, v[0].y - 0.5f * t1.y);
+        const float2 m = f2(__builtin_fmaf(-0.5f, t1.x, v[0].x), __builtin_fmaf(-0.5f, t1.y, v[0].y));
         // DIR * i * sin(2pi/3) * t2
         const float2 q = f2(-(float)DIR * c3 * t2.y, (float)DIR * c3 * t2.x);
         v[0] = add2(v[0], t1);
@@ -171,10 +180,11 @@ struct Dft<5, DIR> {
         constexpr float s1 = 0.95105651629515357212f, s2 = 0.58778525229247312917f;
         const float2 t1 = add2(v[1], v[4]), t2 = add2(v[2], v[3]);
         const float2 t3 = sub2(v[1], v[4]), t4 = sub2(v[2], v[3]);
-        const float2 a1 = f2(v[0].x + c1 * t1.x + c2 * t2.x, v[0].y + c1 * t1.y + c2 * t2.y);
-        const float2 a2 = f2(v[0].x + c2 * t1.x + c1 * t2.x, v[0].y + c2 * t1.y + c1 * t2.y);
-        const float2 b1 = f2(s1 * t3.x + s2 * t4.x, s1 * t3.y + s2 * t4.y);
-        const float2 b2 = f2(s2 * t3.x - s1 * t4.x, s2 * t3.y - s1 * t4.y);
+        auto f = [](float a, float b, float c) { return __builtin_fmaf(a, b, c); };
+        const float2 a1 = f2(f(c2, t2.x, f(c1, t1.x, v[0].x)), f(c2, t2.y, f(c1, t1.y, v[0].y)));
+        const float2 a2 = f2(f(c1, t2.x, f(c2, t1.x, v[0].x)), f(c1, t2.y, f(c2, t1.y, v[0].y)));
+        const float2 b1 = f2(f(s1, t3.x, s2 * t4.x), f(s1, t3.y, s2 * t4.y));
+        const float2 b2 = f2(f(s2, t3.x, -(s1 * t4.x)), f(s2, t3.y, -(s1 * t4.y)));
         // DIR * i * b
         const float2 j1 = f2(-(float)DIR * b1.y, (float)DIR * b1.x);
         const float2 j2 = f2(-(float)DIR * b2.y, (float)DIR * b2.x);
@@ -276,19 +286,21 @@ struct PlanT : Plan<N> {
 };
 
 // Pass kinds.
-enum { FFT_FWD = 0, FFT_INV = 1, FFT_POISSON = 2 };
+enum { FFT_FWD = 0, FFT_INV = 1, FFT_POISSON = 2, FFT_FWD_FOLD = 3 };
 
 // LDS layout of the exchange buffer (L lines x R1 x R2 complex).  For the x
-// pass lanes run along a line (index k2 fastest, padded); for y/z passes
+// pass lanes run along a line (index k2 fastest, padded), and across lines
+// where they access the transposed copy (odd line stride); for y/z passes
 // lanes run across lines (line fastest).
 template <int N, int AXIS>
 struct Xch {
     using P = PlanT<N>;
     static constexpr int R1 = P::R1, R2 = P::R2, L = P::L;
-    static constexpr int SIZE = AXIS == 0 ? L * R1 * (R2 + 1) : L * R1 * R2;
+    static constexpr int LS = (R1 * (R2 + 1)) | 1;  // line stride of the x pass
+    static constexpr int SIZE = AXIS == 0 ? L * LS : L * R1 * R2;
     __device__ __forceinline__ static int at(int l, int n1, int k2)
     {
-        if constexpr (AXIS == 0) return (l * R1 + n1) * (R2 + 1) + k2;
+        if constexpr (AXIS == 0) return l * LS + n1 * (R2 + 1) + k2;
         else return (n1 * R2 + k2) * L + l;
     }
 };
@@ -311,9 +323,10 @@ __device__ __forceinline__ float poisson_factor(const Coef& co, int N, int kx, i
 
 // Work item (d, a, b): droplet d; the pass's lines are the L consecutive
 // lines starting at line-block a of the plane b (x pass: rows y of plane z=b;
-// y pass: columns x of plane z=b; z pass: columns x of row y=b).  One
+// y pass: columns x of plane z=b; z pass: columns x of row y=b).  Sizes up to
+// kMaxPlane have only the x passes.  One
 // work-group of PlanT<N>::NB or more threads; sx holds Xch<N, AXIS>::SIZE and
-// stw N elements.
+// stw N + 1 elements.
 template <int N, int AXIS, int MODE>
 __device__ __forceinline__ void fft_lines(const Drop& D, const Work& wk, float2* __restrict__ sx,
                                           float2* __restrict__ stw)
@@ -327,35 +340,35 @@ __device__ __forceinline__ void fft_lines(const Drop& D, const Work& wk, float2*
     asm volatile("" : "+v"(tid));
     tid &= 0x3ff;
     const bool active = tid < NT;
-    // lane -> (line l, thread-in-line t)
-    int l, t;
-    if constexpr (AXIS == 0) { l = tid / T; t = tid % T; }
-    else { t = tid / L; l = tid % L; }
+    // The x passes of sizes up to kMaxPlane write (forward) and read (inverse)
+    // the transposed copy: lanes run across the lines there, so that a wave
+    // accesses L consecutive y.
+    constexpr bool kTrans = AXIS == 0 && N <= kMaxPlane;
+    constexpr bool kAcrossA = AXIS != 0 || (kTrans && MODE == FFT_INV);
+    constexpr bool kAcrossB = AXIS != 0 || (kTrans && MODE != FFT_INV);
+    // lane -> (line l, thread-in-line t) of steps A and B
+    int l = kAcrossA ? tid % L : tid / T, t = kAcrossA ? tid / L : tid % T;
     constexpr size_t es = AXIS == 0 ? 1 : (AXIS == 1 ? (size_t)N : (size_t)N * N);
-    // first element of line l
-    size_t base;
-    int lx = 0, ly = 0;  // for the Poisson factor: the line's fixed indices
-    if constexpr (AXIS == 0) {
-        ly = wk.a * L + l;
-        base = ((size_t)wk.b * N + ly) * N;
-    } else if constexpr (AXIS == 1) {
-        lx = wk.a * L + l;
-        base = (size_t)wk.b * N * N + lx;
-    } else {
-        lx = wk.a * L + l;
-        ly = wk.b;
-        base = (size_t)ly * N + lx;
-    }
-    const gptr<float2> c = glb(D.c);
+    // element stride and first element of line l, natural or transposed
+    auto first = [&](bool trans) {
+        if constexpr (AXIS == 0) {
+            const int y = wk.a * L + l;
+            return trans ? (size_t)wk.b * N + y : ((size_t)wk.b * N + y) * N;
+        } else if constexpr (AXIS == 1) {
+            return (size_t)wk.b * N * N + wk.a * L + l;
+        } else {
+            return (size_t)wk.b * N + wk.a * L + l;
+        }
+    };
+    constexpr size_t est = (size_t)N * N;
+    constexpr size_t esA = kTrans && MODE == FFT_INV ? est : es, esB = kTrans && MODE != FFT_INV ? est : es;
+    const gptr<float2> src = glb(kTrans && MODE == FFT_INV ? D.ct : D.c);
+    const gptr<float2> dst = glb(kTrans && MODE != FFT_INV ? D.ct : D.c);
+    size_t base = first(kTrans && MODE == FFT_INV);
 
     // the Poisson pass's work item holding kx = ky = 0 sets the k = 0
-    // coefficient from the FP64 sum of s (k_proj_stats)
+    // coefficient from the FP64 sum of s
     const bool has0 = MODE == FFT_POISSON && wk.a == 0 && wk.b == 0;
-    // the first forward pass divides the imaginary part by sigma (a
-    // power of two: exact)
-    float isg = 1.f;
-    if constexpr (AXIS == 0 && MODE == FFT_FWD) isg = 1.f / glb(D.sigma)[0];
-
     constexpr int DIR0 = MODE == FFT_INV ? 1 : -1;
     float2 u[R1 > R2 ? R1 : R2];
     // ---- step A: R1 threads, length-R2 DFTs -----------------------------
@@ -363,17 +376,34 @@ __device__ __forceinline__ void fft_lines(const Drop& D, const Work& wk, float2*
     // are in flight together; the table's LDS stores wait for all of them.
     if (active && t < R1) {
 #pragma unroll
-        for (int n2 = 0; n2 < R2; ++n2) u[n2] = ld2(c, base + (size_t)(t + R1 * n2) * es);
+        for (int n2 = 0; n2 < R2; ++n2) u[n2] = ld2(src, base + (size_t)(t + R1 * n2) * esA);
+    }
+    // the forward x pass divides the imaginary part by sigma (a power of two:
+    // exact); where no launch before it worked that out, it does so, and the
+    // group of the droplet's first lines writes it down for the others
+    float isg = 1.f;
+    if constexpr (AXIS == 0 && MODE == FFT_FWD) isg = 1.f / glb(D.sigma)[0];
+    if constexpr (AXIS == 0 && MODE == FFT_FWD_FOLD) {
+        if (tid < 64) {
+            double q[kPartSums];
+            fold_proj_stats(D, tid, q);
+            const int e = proj_sigma_log2(q);
+            if (tid == 63) {
+                stw[N].x = ldexpf(1.f, -e);
+                if (wk.a == 0 && wk.b == 0) put_proj_stats(D, q, e);
+            }
+        }
     }
     for (int i = tid; i < N; i += blockDim.x) stw[i] = ld2(glb(D.tw), i);
+    __syncthreads();  // stw
     if (active && t < R1) {
-        if constexpr (AXIS == 0 && MODE == FFT_FWD) {
+        if constexpr (AXIS == 0 && MODE != FFT_INV) {
+            if constexpr (MODE == FFT_FWD_FOLD) isg = stw[N].x;
 #pragma unroll
             for (int n2 = 0; n2 < R2; ++n2) u[n2].y *= isg;
         }
         Dft<R2, DIR0>::run(u);
     }
-    __syncthreads();  // stw
     if (active && t < R1) {
 #pragma unroll
         for (int k2 = 0; k2 < R2; ++k2) {
@@ -384,6 +414,11 @@ __device__ __forceinline__ void fft_lines(const Drop& D, const Work& wk, float2*
     }
     __syncthreads();
     // ---- step B: R2 threads, length-R1 DFTs -----------------------------
+    if constexpr (kAcrossA != kAcrossB) {
+        l = kAcrossB ? tid % L : tid / T;
+        t = kAcrossB ? tid / L : tid % T;
+    }
+    base = first(kTrans && MODE != FFT_INV);
     if (active && t < R2) {
 #pragma unroll
         for (int n1 = 0; n1 < R1; ++n1) u[n1] = sx[X::at(l, n1, t)];
@@ -392,7 +427,7 @@ __device__ __forceinline__ void fft_lines(const Drop& D, const Work& wk, float2*
     if constexpr (MODE != FFT_POISSON) {
         if (active && t < R2) {
 #pragma unroll
-            for (int k1 = 0; k1 < R1; ++k1) st2(c, base + (size_t)(t + R2 * k1) * es, u[k1]);
+            for (int k1 = 0; k1 < R1; ++k1) st2(dst, base + (size_t)(t + R2 * k1) * esB, u[k1]);
         }
     } else {
         // multiply by -1/(k^2 N^3); element index kz = t + R2 k1
@@ -403,7 +438,7 @@ __device__ __forceinline__ void fft_lines(const Drop& D, const Work& wk, float2*
                 const int kz = t + R2 * k1;
                 float2 s = u[k1];
                 if (has0 && l == 0 && kz == 0) s = f2((float)glb(D.stat)[0], (float)glb(D.stat)[1]);
-                const float m = poisson_factor(co, N, lx, ly, kz);
+                const float m = poisson_factor(co, N, wk.a * L + l, wk.b, kz);
                 u[k1] = f2(s.x * m, s.y * m);
             }
             // inverse, roles swapped: n' = t + R2 k1, thread t = n1' < R2,
@@ -424,7 +459,7 @@ __device__ __forceinline__ void fft_lines(const Drop& D, const Work& wk, float2*
             for (int n1 = 0; n1 < R2; ++n1) u[n1] = sx[X::at(l, t, n1)];
             Dft<R2, 1>::run(u);
 #pragma unroll
-            for (int m1 = 0; m1 < R2; ++m1) st2(c, base + (size_t)(t + R1 * m1) * es, u[m1]);
+            for (int m1 = 0; m1 < R2; ++m1) st2(dst, base + (size_t)(t + R1 * m1) * es, u[m1]);
         }
     }
 }
@@ -434,7 +469,7 @@ __global__ __launch_bounds__(PlanT<N>::NB) void k_fft(const Drop* __restrict__ d
                                                       const int* __restrict__ nwork_p, int kstep)
 {
     __shared__ float2 sx[Xch<N, AXIS>::SIZE];
-    __shared__ float2 stw[N];
+    __shared__ float2 stw[N + 1];
     const int nwork = *nwork_p;
     for (int v = blockIdx.x; v < xcd_span(nwork); v += gridDim.x) {
         const int w = xcd_item(v, nwork);
@@ -448,11 +483,16 @@ __global__ __launch_bounds__(PlanT<N>::NB) void k_fft(const Drop* __restrict__ d
 }
 
 // The largest work-group and exchange buffer over the size list.
+template <int N, int AXIS>
+constexpr bool fft_has_pass()
+{
+    return AXIS == 0 || N > kMaxPlane;
+}
 template <int AXIS, int I = 0>
 constexpr int fft_max_lds()
 {
     if constexpr (I == kNumGridSizes) return 0;
-    else return std::max(Xch<kGridSizes[I], AXIS>::SIZE, fft_max_lds<AXIS, I + 1>());
+    else return std::max(fft_has_pass<kGridSizes[I], AXIS>() ? Xch<kGridSizes[I], AXIS>::SIZE : 0, fft_max_lds<AXIS, I + 1>());
 }
 template <int I = 0>
 constexpr int fft_max_threads()
@@ -466,8 +506,13 @@ template <int AXIS, int MODE, int I = 0>
 __device__ __forceinline__ void fft_any(int N, const Drop& D, const Work& wk, float2* sx, float2* stw)
 {
     if constexpr (I < kNumGridSizes) {
-        if (N == kGridSizes[I]) fft_lines<kGridSizes[I], AXIS, MODE>(D, wk, sx, stw);
-        else fft_any<AXIS, MODE, I + 1>(N, D, wk, sx, stw);
+        if constexpr (fft_has_pass<kGridSizes[I], AXIS>()) {
+            if (N == kGridSizes[I]) {
+                fft_lines<kGridSizes[I], AXIS, MODE>(D, wk, sx, stw);
+                return;
+            }
+        }
+        fft_any<AXIS, MODE, I + 1>(N, D, wk, sx, stw);
     }
 }
 
@@ -485,7 +530,7 @@ __global__ __launch_bounds__(fft_max_threads(), 4) void k_fft_sizes(const Drop* 
                                                                 const int* __restrict__ nwork_p, int kstep)
 {
     __shared__ float2 sx[fft_max_lds<AXIS>()];
-    __shared__ float2 stw[kMaxN];
+    __shared__ float2 stw[kMaxN + 1];
     const int nwork = *nwork_p;
     for (int v = blockIdx.x; v < xcd_span(nwork); v += gridDim.x) {
         const int w = xcd_item(v, nwork);
@@ -499,86 +544,171 @@ __global__ __launch_bounds__(fft_max_threads(), 4) void k_fft_sizes(const Drop* 
 }
 
 // ===========================================================================
-// Fused x+y pass for N <= 128: one work-group per z-plane holds the N x N
-// complex plane in LDS (row pitch N+1) and transforms all rows and all
-// columns there, so the plane crosses HBM once per direction instead of
-// twice.  Forward: x then y (e^{-i...}); inverse: y then x (e^{+i...});
-// unnormalised like the single-axis passes.
+// y-z plane of sizes up to kMaxPlane: one work-group takes the plane x of the
+// transposed copy through the forward y and z transforms, the solve and the
+// inverse z and y transforms.  LDS holds the plane, [z][y] with a row pitch of
+// N + 1 complex elements.
+//
+// Every stage is a set of register DFTs whose inputs and outputs occupy the
+// same positions, so it works in place and needs one barrier.  With N = R1 R2
+// a line x is transformed forward by
+//   A  per n1: length-R2 DFT over n2 of x[n1 + R1 n2], times W_N^{n1 k2}, to n1 + R1 k2
+//   B  per k2: length-R1 DFT over n1, X[k2 + R2 k1] to position k1 + R1 k2
+// and inversely from that order by
+//   B' per k2: length-R1 inverse DFT over k1, times W_N^{-k2 m}, to m + R1 k2
+//   C  per n1: length-R2 inverse DFT over k2, x[n1 + R1 m1] to n1 + R1 m1
+// The z lines' B and B' are one stage, with the solve between them in
+// registers.  A of the y lines takes its inputs from memory and C of the y
+// lines leaves its outputs there: 6 passes over LDS for 4 transforms.
+//
+// What bounds it: VALU and LDS of the CUs that have a plane when there are
+// fewer planes than CUs (a lone droplet), which is still less than the
+// launches and hand-offs between XCDs of three passes: 64^3 13.4 -> 9.2 us,
+// 128^3 31.2 -> 26.
 // ===========================================================================
 template <int N>
-struct XyCfg {
-    static constexpr int NT = N >= 96 ? 1024 : 256;
+struct PlaneCfg {
+    static constexpr int NT = N >= 72 ? 1024 : N >= 40 ? 512 : 256;  // one or two DFTs per thread and stage
     static constexpr int P = N + 1;  // LDS row pitch in complex elements
 };
 
-typedef float fvec4 __attribute__((ext_vector_type(4)));
-
-// In-place DFT of the N lines of the plane along x (AX 0: line l is row y=l)
-// or y (AX 1: line l is column x=l), four-step as the single-axis passes.
-template <int N, int AX, int DIR, int NT>
-__device__ __forceinline__ void plane_dft(float2* __restrict__ pl, const float2* __restrict__ stw, int tid)
+// Work item (d, -, x): plane x of droplet d.  NT threads; pl holds N (N + 1)
+// and stw N elements.
+template <int N, int NT>
+__device__ __forceinline__ void yz_plane(const Drop& D, int x, float2* __restrict__ pl, float2* __restrict__ stw)
 {
     using PL = PlanT<N>;
-    constexpr int R1 = PL::R1, R2 = PL::R2, P = XyCfg<N>::P;
-    auto at = [](int l, int j) { return AX == 0 ? l * P + j : j * P + l; };
-    // A: task (l, n1): length-R2 DFT of x[n1 + R1 n2], twiddle W_N^{n1 k2},
-    // back to the same positions.  Lanes run along a row (x lines) or across
-    // columns (y lines), contiguous in LDS either way.
-    constexpr int TA = N * R1;
+    constexpr int R1 = PL::R1, R2 = PL::R2, P = PlaneCfg<N>::P;
+    constexpr int TA = N * R1, TB = N * R2;  // register DFTs of length R2, of length R1
+    int tid = threadIdx.x;  // opaque: see fft_lines
+    asm volatile("" : "+v"(tid));
+    tid &= 0x3ff;
+    const gptr<float2> c = glb(D.ct) + (size_t)x * N * N;
+    for (int i = tid; i < N; i += NT) stw[i] = ld2(glb(D.tw), i);
+    constexpr int KA = (TA + NT - 1) / NT;
+    // ---- y lines, A: lanes along y, the loads of every task first ----------
+    {
+        float2 u[KA][R2];
+#pragma unroll
+        for (int k = 0; k < KA; ++k) {
+            const int task = tid + k * NT, z = task / R1, n1 = task % R1;
+            if (task < TA) {
+#pragma unroll
+                for (int n2 = 0; n2 < R2; ++n2) u[k][n2] = ld2(c, (unsigned)(z * N + n1 + R1 * n2));
+            }
+        }
+        __syncthreads();  // stw
+#pragma unroll
+        for (int k = 0; k < KA; ++k) {
+            const int task = tid + k * NT, z = task / R1, n1 = task % R1;
+            if (task < TA) {
+                Dft<R2, -1>::run(u[k]);
+#pragma unroll
+                for (int k2 = 0; k2 < R2; ++k2)
+                    pl[z * P + n1 + R1 * k2] = k2 == 0 ? u[k][0] : mul2(u[k][k2], stw[(n1 * k2) % N]);
+            }
+        }
+    }
+    __syncthreads();
+    // ---- y lines, B: lanes across the lines ---------------------------------
+    for (int task = tid; task < TB; task += NT) {
+        const int z = task % N, k2 = task / N;
+        float2 u[R1];
+        float2* const q = pl + z * P + R1 * k2;
+#pragma unroll
+        for (int n1 = 0; n1 < R1; ++n1) u[n1] = q[n1];
+        Dft<R1, -1>::run(u);
+#pragma unroll
+        for (int k1 = 0; k1 < R1; ++k1) q[k1] = u[k1];
+    }
+    __syncthreads();
+    // ---- z lines, A ---------------------------------------------------------
     for (int task = tid; task < TA; task += NT) {
-        const int l = AX == 0 ? task / R1 : task % N;
-        const int n1 = AX == 0 ? task % R1 : task / N;
+        const int py = task % N, n1 = task / N;
+        float2 u[R2];
+        float2* const q = pl + n1 * P + py;
+#pragma unroll
+        for (int n2 = 0; n2 < R2; ++n2) u[n2] = q[R1 * n2 * P];
+        Dft<R2, -1>::run(u);
+#pragma unroll
+        for (int k2 = 0; k2 < R2; ++k2) q[R1 * k2 * P] = k2 == 0 ? u[0] : mul2(u[k2], stw[(n1 * k2) % N]);
+    }
+    __syncthreads();
+    // ---- z lines, B, the solve, B' ------------------------------------------
+    {
+        const Coef co = D.co;
+        for (int task = tid; task < TB; task += NT) {
+            const int py = task % N, k2 = task / N;
+            float2 u[R1];
+            float2* const q = pl + R1 * k2 * P + py;
+#pragma unroll
+            for (int n1 = 0; n1 < R1; ++n1) u[n1] = q[n1 * P];
+            Dft<R1, -1>::run(u);
+            const int ky = py / R1 + R2 * (py % R1);
+#pragma unroll
+            for (int k1 = 0; k1 < R1; ++k1) {
+                const int kz = k2 + R2 * k1;
+                float2 s = u[k1];
+                // the k = 0 coefficient from the FP64 sum of s
+                if (k1 == 0 && x == 0 && ky == 0 && kz == 0) s = f2((float)glb(D.stat)[0], (float)glb(D.stat)[1]);
+                const float m = poisson_factor(co, N, x, ky, kz);
+                u[k1] = f2(s.x * m, s.y * m);
+            }
+            Dft<R1, 1>::run(u);
+#pragma unroll
+            for (int m = 0; m < R1; ++m) {
+                const float2 w = stw[(k2 * m) % N];
+                q[m * P] = m == 0 ? u[0] : mul2(u[m], f2(w.x, -w.y));
+            }
+        }
+    }
+    __syncthreads();
+    // ---- z lines, C ---------------------------------------------------------
+    for (int task = tid; task < TA; task += NT) {
+        const int py = task % N, n1 = task / N;
+        float2 u[R2];
+        float2* const q = pl + n1 * P + py;
+#pragma unroll
+        for (int k2 = 0; k2 < R2; ++k2) u[k2] = q[R1 * k2 * P];
+        Dft<R2, 1>::run(u);
+#pragma unroll
+        for (int m1 = 0; m1 < R2; ++m1) q[R1 * m1 * P] = u[m1];
+    }
+    __syncthreads();
+    // ---- y lines, B' --------------------------------------------------------
+    for (int task = tid; task < TB; task += NT) {
+        const int z = task % N, k2 = task / N;
+        float2 u[R1];
+        float2* const q = pl + z * P + R1 * k2;
+#pragma unroll
+        for (int k1 = 0; k1 < R1; ++k1) u[k1] = q[k1];
+        Dft<R1, 1>::run(u);
+#pragma unroll
+        for (int m = 0; m < R1; ++m) {
+            const float2 w = stw[(k2 * m) % N];
+            q[m] = m == 0 ? u[0] : mul2(u[m], f2(w.x, -w.y));
+        }
+    }
+    __syncthreads();
+    // ---- y lines, C: to memory, lanes along y -------------------------------
+    for (int task = tid; task < TA; task += NT) {
+        const int z = task / R1, n1 = task % R1;
         float2 u[R2];
 #pragma unroll
-        for (int n2 = 0; n2 < R2; ++n2) u[n2] = pl[at(l, n1 + R1 * n2)];
-        Dft<R2, DIR>::run(u);
+        for (int k2 = 0; k2 < R2; ++k2) u[k2] = pl[z * P + n1 + R1 * k2];
+        Dft<R2, 1>::run(u);
 #pragma unroll
-        for (int k2 = 0; k2 < R2; ++k2) {
-            const float2 wv = stw[(n1 * k2) % N];
-            const float2 w2 = f2(wv.x, DIR == -1 ? wv.y : -wv.y);
-            pl[at(l, n1 + R1 * k2)] = k2 == 0 ? u[0] : mul2(u[k2], w2);
-        }
+        for (int m1 = 0; m1 < R2; ++m1) st2(c, (unsigned)(z * N + n1 + R1 * m1), u[m1]);
     }
-    __syncthreads();
-    // B: task (l, k2): length-R1 DFT over n1, result X[k2 + R2 k1]; all reads
-    // precede all writes (same plane)
-    constexpr int TB = N * R2, KB = (TB + NT - 1) / NT;
-    float2 v[KB][R1];
-#pragma unroll
-    for (int k = 0; k < KB; ++k) {
-        const int task = tid + k * NT;
-        if (task < TB) {
-            const int l = AX == 0 ? task / R2 : task % N;
-            const int k2 = AX == 0 ? task % R2 : task / N;
-#pragma unroll
-            for (int n1 = 0; n1 < R1; ++n1) v[k][n1] = pl[at(l, n1 + R1 * k2)];
-            Dft<R1, DIR>::run(v[k]);
-        }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < KB; ++k) {
-        const int task = tid + k * NT;
-        if (task < TB) {
-            const int l = AX == 0 ? task / R2 : task % N;
-            const int k2 = AX == 0 ? task % R2 : task / N;
-#pragma unroll
-            for (int k1 = 0; k1 < R1; ++k1) pl[at(l, k2 + R2 * k1)] = v[k][k1];
-        }
-    }
-    __syncthreads();
 }
 
-// Work item (d, -, z): plane z of droplet d.
-template <int N, int MODE>
-__global__ __launch_bounds__(XyCfg<N>::NT) void k_fft_xy(const Drop* __restrict__ drops, const Work* __restrict__ work,
-                                                        const int* __restrict__ nwork_p, int kstep)
+template <int N>
+__global__ __launch_bounds__(PlaneCfg<N>::NT) void k_fft_yz(const Drop* __restrict__ drops,
+                                                            const Work* __restrict__ work,
+                                                            const int* __restrict__ nwork_p, int kstep)
 {
-    constexpr int NT = XyCfg<N>::NT, P = XyCfg<N>::P;
-    constexpr int DIR = MODE == FFT_INV ? 1 : -1;
-    __shared__ float2 pl[N * P];
+    __shared__ float2 pl[N * PlaneCfg<N>::P];
     __shared__ float2 stw[N];
-    const int tid = threadIdx.x;
     const int nwork = *nwork_p;
     for (int v = blockIdx.x; v < xcd_span(nwork); v += gridDim.x) {
         const int w = xcd_item(v, nwork);
@@ -586,66 +716,45 @@ __global__ __launch_bounds__(XyCfg<N>::NT) void k_fft_xy(const Drop* __restrict_
         const Work wk = work[w];
         const Drop& D = drops[wk.d];
         if (kstep >= D.nsteps) continue;
-        const gptr<fvec4> cp = (gptr<fvec4>)(glb(D.c) + (size_t)wk.b * N * N);
-        __syncthreads();  // the previous item's stores have read the plane
-        // load: two complex elements of one row per 16-byte access, all of
-        // the thread's accesses issued before the twiddle table's and sigma's
-        // so that they are in flight together; the forward pass divides the
-        // imaginary part by sigma (a power of two)
-        constexpr int NQ = (N * N / 2 + NT - 1) / NT;
-        fvec4 q[NQ];
-#pragma unroll
-        for (int k = 0; k < NQ; ++k) {
-            const int i = tid + k * NT;
-            if (i < N * N / 2) q[k] = cp[i];
-        }
-        for (int i = tid; i < N; i += NT) stw[i] = ld2(glb(D.tw), i);
-        const float isg = MODE == FFT_FWD ? 1.f / glb(D.sigma)[0] : 1.f;
-#pragma unroll
-        for (int k = 0; k < NQ; ++k) {
-            const int i = tid + k * NT;
-            if (i < N * N / 2) {
-                if constexpr (MODE == FFT_FWD) {
-                    q[k].y *= isg;
-                    q[k].w *= isg;
-                }
-                const int y = (2 * i) / N, x = (2 * i) % N;
-                pl[y * P + x] = f2(q[k].x, q[k].y);
-                pl[y * P + x + 1] = f2(q[k].z, q[k].w);
-            }
-        }
-        __syncthreads();
-        if constexpr (MODE == FFT_INV) {
-            plane_dft<N, 1, DIR, NT>(pl, stw, tid);
-            plane_dft<N, 0, DIR, NT>(pl, stw, tid);
-        } else {
-            plane_dft<N, 0, DIR, NT>(pl, stw, tid);
-            plane_dft<N, 1, DIR, NT>(pl, stw, tid);
-        }
-        for (int i = tid; i < N * N / 2; i += NT) {
-            const int y = (2 * i) / N, x = (2 * i) % N;
-            const float2 a = pl[y * P + x], b = pl[y * P + x + 1];
-            fvec4 q;
-            q.x = a.x;
-            q.y = a.y;
-            q.z = b.x;
-            q.w = b.y;
-            cp[i] = q;
-        }
+        __syncthreads();  // the previous item has read pl and stw
+        yz_plane<N, PlaneCfg<N>::NT>(D, wk.b, pl, stw);
     }
 }
 
-template <int N>
-static hipError_t launch_fft_xy_n(int mode, const Drop* drops, const Work* work, const int* nwork_p, int kstep,
-                                  int grid, hipStream_t st)
+// yz_plane for the droplet's N, one of the sizes in (LO, HI].
+template <int LO, int HI, int NT, int I = 0>
+__device__ __forceinline__ void yz_any(int N, const Drop& D, int x, float2* pl, float2* stw)
 {
-    const dim3 blk(XyCfg<N>::NT);
-    if (mode == FFT_FWD) return launch_kernel(k_fft_xy<N, FFT_FWD>, dim3(grid), blk, st, drops, work, nwork_p, kstep);
-    if (mode == FFT_INV) return launch_kernel(k_fft_xy<N, FFT_INV>, dim3(grid), blk, st, drops, work, nwork_p, kstep);
-    return hipErrorInvalidValue;
+    if constexpr (I < kNumGridSizes) {
+        if constexpr (kGridSizes[I] > LO && kGridSizes[I] <= HI) {
+            if (N == kGridSizes[I]) {
+                yz_plane<kGridSizes[I], NT>(D, x, pl, stw);
+                return;
+            }
+        }
+        yz_any<LO, HI, NT, I + 1>(N, D, x, pl, stw);
+    }
 }
 
-bool fft_xy_fused(int N) { return N <= kMaxFusedXy; }
+// Planes of several sizes in (LO, HI], HI one of them, in one launch.
+template <int LO, int HI>
+__global__ __launch_bounds__(PlaneCfg<HI>::NT) void k_fft_yz_sizes(const Drop* __restrict__ drops,
+                                                                  const Work* __restrict__ work,
+                                                                  const int* __restrict__ nwork_p, int kstep)
+{
+    __shared__ float2 pl[HI * PlaneCfg<HI>::P];
+    __shared__ float2 stw[HI];
+    const int nwork = *nwork_p;
+    for (int v = blockIdx.x; v < xcd_span(nwork); v += gridDim.x) {
+        const int w = xcd_item(v, nwork);
+        if (w >= nwork) continue;
+        const Work wk = work[w];
+        const Drop& D = drops[wk.d];
+        if (kstep >= D.nsteps) continue;
+        __syncthreads();  // the previous item has read pl and stw
+        yz_any<LO, HI, PlaneCfg<HI>::NT>(D.N, D, wk.b, pl, stw);
+    }
+}
 
 // f(std::integral_constant<int, N>) for the grid size N of the size list.
 template <int I = 0, class F>
@@ -659,28 +768,45 @@ static hipError_t with_size(int N, F&& f)
     }
 }
 
-hipError_t launch_fft_xy(int N, int mode, const Drop* drops, const Work* work, const int* nwork_p, int kstep, int grid,
+hipError_t launch_fft_yz(int N, const Drop* drops, const Work* work, const int* nwork_p, int kstep, int grid,
                          hipStream_t st)
 {
     if (grid <= 0) return hipSuccess;
     return with_size(N, [&](auto n) {
         constexpr int NS = decltype(n)::value;
-        if constexpr (NS <= kMaxFusedXy) return launch_fft_xy_n<NS>(mode, drops, work, nwork_p, kstep, grid, st);
+        if constexpr (NS <= kMaxPlane)
+            return launch_kernel(k_fft_yz<NS>, dim3(grid), dim3(PlaneCfg<NS>::NT), st, drops, work, nwork_p, kstep);
         else return hipErrorInvalidValue;
     });
+}
+
+hipError_t launch_fft_yz_sizes(int group, const Drop* drops, const Work* work, const int* nwork_p, int kstep, int grid,
+                               hipStream_t st)
+{
+    if (grid <= 0) return hipSuccess;
+    if (group == 0)
+        return launch_kernel(k_fft_yz_sizes<0, kSmallPlane>, dim3(grid), dim3(PlaneCfg<kSmallPlane>::NT), st, drops,
+                             work, nwork_p, kstep);
+    return launch_kernel(k_fft_yz_sizes<kSmallPlane, kMaxPlane>, dim3(grid), dim3(PlaneCfg<kMaxPlane>::NT), st, drops,
+                         work, nwork_p, kstep);
 }
 
 template <int N>
 static hipError_t launch_fft_n(int axis, int mode, const Drop* drops, const Work* work, const int* nwork_p,
                                int kstep, int grid, hipStream_t st)
 {
-    const dim3 blk(PlanT<N>::NB);
-    if (axis == 0 && mode == FFT_FWD) return launch_kernel(k_fft<N, 0, FFT_FWD>, dim3(grid), blk, st, drops, work, nwork_p, kstep);
-    if (axis == 0 && mode == FFT_INV) return launch_kernel(k_fft<N, 0, FFT_INV>, dim3(grid), blk, st, drops, work, nwork_p, kstep);
-    if (axis == 1 && mode == FFT_FWD) return launch_kernel(k_fft<N, 1, FFT_FWD>, dim3(grid), blk, st, drops, work, nwork_p, kstep);
-    if (axis == 1 && mode == FFT_INV) return launch_kernel(k_fft<N, 1, FFT_INV>, dim3(grid), blk, st, drops, work, nwork_p, kstep);
-    if (axis == 2 && mode == FFT_POISSON)
-        return launch_kernel(k_fft<N, 2, FFT_POISSON>, dim3(grid), blk, st, drops, work, nwork_p, kstep);
+    const dim3 blk(PlanT<N>::NB), g(grid);
+    if (axis == 0 && mode == FFT_FWD) return launch_kernel(k_fft<N, 0, FFT_FWD>, g, blk, st, drops, work, nwork_p, kstep);
+    if (axis == 0 && mode == FFT_INV) return launch_kernel(k_fft<N, 0, FFT_INV>, g, blk, st, drops, work, nwork_p, kstep);
+    if constexpr (N <= kMaxPlane) {
+        if (axis == 0 && mode == FFT_FWD_FOLD)
+            return launch_kernel(k_fft<N, 0, FFT_FWD_FOLD>, g, blk, st, drops, work, nwork_p, kstep);
+    } else {
+        if (axis == 1 && mode == FFT_FWD) return launch_kernel(k_fft<N, 1, FFT_FWD>, g, blk, st, drops, work, nwork_p, kstep);
+        if (axis == 1 && mode == FFT_INV) return launch_kernel(k_fft<N, 1, FFT_INV>, g, blk, st, drops, work, nwork_p, kstep);
+        if (axis == 2 && mode == FFT_POISSON)
+            return launch_kernel(k_fft<N, 2, FFT_POISSON>, g, blk, st, drops, work, nwork_p, kstep);
+    }
     return hipErrorInvalidValue;
 }
 
@@ -699,6 +825,8 @@ hipError_t launch_fft_sizes(int axis, int mode, const Drop* drops, const Work* w
     if (grid <= 0) return hipSuccess;
     const dim3 blk(fft_max_threads()), g(grid);
     if (axis == 0 && mode == FFT_FWD) return launch_kernel(k_fft_sizes<0, FFT_FWD>, g, blk, st, drops, work, nwork_p, kstep);
+    if (axis == 0 && mode == FFT_FWD_FOLD)
+        return launch_kernel(k_fft_sizes<0, FFT_FWD_FOLD>, g, blk, st, drops, work, nwork_p, kstep);
     if (axis == 0 && mode == FFT_INV) return launch_kernel(k_fft_sizes<0, FFT_INV>, g, blk, st, drops, work, nwork_p, kstep);
     if (axis == 1 && mode == FFT_FWD) return launch_kernel(k_fft_sizes<1, FFT_FWD>, g, blk, st, drops, work, nwork_p, kstep);
     if (axis == 1 && mode == FFT_INV) return launch_kernel(k_fft_sizes<1, FFT_INV>, g, blk, st, drops, work, nwork_p, kstep);

@@ -40,33 +40,6 @@
 
 namespace ttsh {
 
-// Adds to each value the one that DPP control CTRL brings, 0 where none comes.
-template <int CTRL, int N>
-__device__ __forceinline__ void dpp_add(double (&e)[N])
-{
-#pragma unroll
-    for (int k = 0; k < N; ++k) {
-        const unsigned long long b = __double_as_longlong(e[k]);
-        const unsigned lo = __builtin_amdgcn_update_dpp(0, (int)(unsigned)b, CTRL, 0xf, 0xf, false);
-        const unsigned hi = __builtin_amdgcn_update_dpp(0, (int)(unsigned)(b >> 32), CTRL, 0xf, 0xf, false);
-        e[k] += __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
-    }
-}
-
-// Sums over a wave, complete in lane 63: row_shr 1, 2, 4, 8 and the two row
-// broadcasts.  Shuffles through LDS would take 72 ds_bpermute, 3 us for the 16
-// waves of a work-group; this takes 0.7.
-template <int N>
-__device__ __forceinline__ void wave_sum(double (&e)[N])
-{
-    dpp_add<0x111>(e);
-    dpp_add<0x112>(e);
-    dpp_add<0x114>(e);
-    dpp_add<0x118>(e);
-    dpp_add<0x142>(e);
-    dpp_add<0x143>(e);
-}
-
 // K_div.  The divergence needs X of the x field, A of the y field and B of the
 // z field; a row's part of its neighbours' sum is U = X + A + B for the row
 // below and W = X - A + B for the row above, so each of the two divergences
@@ -87,7 +60,7 @@ __global__ __launch_bounds__(64 * kProjWaves, 8) void k_div(const Drop* __restri
     // depend on how the loop was compiled
 #pragma clang fp contract(off)
     __shared__ float4 rec[2][kProjWaves * 64];  // U_v, W_v, U_p, W_p of a row
-    __shared__ double red[kPartSums * kProjWaves];
+    __shared__ double red[2][kPartSums * kProjWaves];
     const int lane = threadIdx.x & 63;
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int nwork = *nwork_p;
@@ -148,30 +121,38 @@ __global__ __launch_bounds__(64 * kProjWaves, 8) void k_div(const Drop* __restri
         // coefficient), the squares, which only set sigma, per thread in FP32
         double d0 = 0.0, d1 = 0.0;
         float q2 = 0.f, q3 = 0.f, q4 = 0.f, q5 = 0.f;
-        // The sums are written per reduction block (see Drop::part): the
-        // item starts at block wk.c, and at the last plane of each block the
-        // work-group reduces them in a fixed order and starts the next.  The
-        // sums of a block are then the same whichever item covers it.
+        // The sums are written per reduction block (see Drop::part): the item
+        // starts at block wk.c, and at the last plane of each block every wave
+        // reduces its sums and starts the next.  The sums of a block are then
+        // the same whichever item covers it.  The waves' sums are added, in
+        // order, behind the next plane's barrier (or the one after the last
+        // plane), so that a block costs no barrier of its own; two buffers
+        // keep them until then.
         const int ntile = proj_tiles(N);
         int ordb = wk.c;
         int zend = (wk.c / ntile + 1) * N / D.nzp;
+        bool pending = false;  // uniform across the work-group, as is rb
+        int rb = 0;
         auto flush = [&]() {
             double e[kPartSums] = {d0, d1, q2, q3, q4, q5};
             wave_sum(e);
-            __syncthreads();  // the previous block's sums were read
             if (lane == 63) {
 #pragma unroll
-                for (int k = 0; k < kPartSums; ++k) red[kPartSums * wv + k] = e[k];
-            }
-            __syncthreads();
-            if (threadIdx.x < kPartSums) {
-                double a = 0.0;
-#pragma unroll
-                for (int i = 0; i < kProjWaves; ++i) a += red[kPartSums * i + threadIdx.x];
-                glb(D.part)[(size_t)kPartSums * ordb + threadIdx.x] = a;
+                for (int k = 0; k < kPartSums; ++k) red[rb][kPartSums * wv + k] = e[k];
             }
             d0 = d1 = 0.0;
             q2 = q3 = q4 = q5 = 0.f;
+            pending = true;
+        };
+        auto finish = [&]() {
+            if (threadIdx.x < kPartSums) {
+                double a = 0.0;
+#pragma unroll
+                for (int i = 0; i < kProjWaves; ++i) a += red[rb][kPartSums * i + threadIdx.x];
+                glb(D.part)[(size_t)kPartSums * ordb + threadIdx.x] = a;
+            }
+            pending = false;
+            rb ^= 1;
             ordb += ntile;
             zend = (ordb / ntile + 1) * N / D.nzp;
         };
@@ -206,6 +187,7 @@ __global__ __launch_bounds__(64 * kProjWaves, 8) void k_div(const Drop* __restri
             __syncthreads();
             const float4 m = rec[buf][below], p = rec[buf][above];
             buf ^= 1;
+            if (pending) finish();
             if (own) {
                 fvec2 sv;
                 sv.x = scale * fma_(4.f, xb[0], m.y + p.x);
@@ -231,25 +213,18 @@ __global__ __launch_bounds__(64 * kProjWaves, 8) void k_div(const Drop* __restri
             body(Ph<2>{}, zm);
             if (++zm >= ze) break;
         }
-        // the item ends at a block end, so its last block was written above
+        // the item ends at a block end
+        __syncthreads();
+        if (pending) finish();
     }
 }
 
-// One work-group per droplet (work item (d, -, -)): the sums of the
-// divergence items in item order, then the k = 0 coefficient of s/sigma and
-// this step's sigma (derivation at the top of this file).
+// One work-group per droplet (work item (d, -, -)): the sums of its reduction
+// blocks, then the k = 0 coefficient of s/sigma and this step's sigma
+// (derivation at the top of this file).  Up to kFoldedParts blocks one wave
+// adds them as the forward x pass would (fold_proj_stats), so that the result
+// is the same where that does it.
 constexpr int kStatsThreads = 256;
-
-// log2 x for x >= 0 (-inf at 0, +inf at inf): exponent plus the FP32 log2 of
-// the mantissa, enough for a rounded power of two
-__device__ __forceinline__ double log2_coarse(double x)
-{
-    if (!(x > 0.0)) return -INFINITY;
-    if (x == INFINITY) return INFINITY;
-    int ex;
-    const double m = frexp(x, &ex);
-    return (double)ex + (double)log2f((float)m);
-}
 
 __global__ __launch_bounds__(kStatsThreads) void k_proj_stats(const Drop* __restrict__ drops,
                                                               const Work* __restrict__ work,
@@ -264,6 +239,14 @@ __global__ __launch_bounds__(kStatsThreads) void k_proj_stats(const Drop* __rest
         const Drop& D = drops[work[w].d];
         if (kstep >= D.nsteps) continue;
         const int np = D.npart;
+        if (np <= kFoldedParts) {
+            if (tid < 64) {
+                double t[kPartSums];
+                fold_proj_stats(D, tid, t);
+                if (tid == 63) put_proj_stats(D, t, proj_sigma_log2(t));
+            }
+            continue;
+        }
         const gptr<const double> pt = glb<const double>(D.part);
         double q[kPartSums] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
 #pragma unroll 4
@@ -293,25 +276,11 @@ __global__ __launch_bounds__(kStatsThreads) void k_proj_stats(const Drop* __rest
             double t[kPartSums];
 #pragma unroll
             for (int e = 0; e < kPartSums; ++e) t[e] = tot[e];
-            // log2 of 0 is -inf, of inf +inf; -inf + inf is NaN
-            const double l = 0.25 * ((log2_coarse(t[3]) + log2_coarse(t[5])) - (log2_coarse(t[2]) + log2_coarse(t[4])));
-            int e = 0;
-            if (t[3] > 0.0 && l == l) e = (int)rint(fmin(fmax(l, -30.0), 30.0));
-            const float sig = ldexpf(1.f, e);
-            glb(D.sigma)[0] = sig;
-            glb(D.stat)[0] = t[0];
-            glb(D.stat)[1] = ldexp(t[1], -e);
+            put_proj_stats(D, t, proj_sigma_log2(t));
         }
     }
 }
 
-// K_corr: a work-group owns a TX x TY column and walks a z-range, loading one
-// plane of p (with a one-cell xy apron) per iteration into LDS and adding its
-// contribution to the three output planes it touches.  Bound by HBM: 4.8 TB/s
-// of traffic at 256^3, where a copy reaches 5.1.  K_div's row waves measured
-// 197 -> 231 us there (their 52-cell rows end inside cache lines, and six
-// output fields are then written in partial lines), 77 -> 75 at 180^3 and
-// 21 -> 22 at 128^3, so the corrector keeps its aligned 32x8 tile.
 template <int TX, int TY>
 __global__ __launch_bounds__(TX * TY) void k_corr(const Drop* __restrict__ drops, const Work* __restrict__ work,
                                                   const int* __restrict__ nwork_p, int parity, int kstep)

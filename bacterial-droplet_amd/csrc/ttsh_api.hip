@@ -3,11 +3,11 @@
 //
 // An Engine owns a set of droplet slots on one device and one stream.  One
 // step of the engine is eight kernel kinds, each launched once per step (the
-// FFT passes once per grid size present), each covering every active
+// FFT passes once per kind of size present), each covering every active
 // droplet through a work table (see ttsh_dev.h):
-//   K_rhs, K_div (with k_proj_stats, the per-droplet sums behind it), FFT x
+//   K_rhs, K_div (for large droplets with k_proj_stats, the sums behind it), FFT x
 //   fwd, FFT y fwd, FFT z (fwd, -1/k^2, inv), FFT y inv, FFT x inv, K_corr
-// standing in for the reference's EEuler (TTSH3D.cu:347-359: 107 kernel
+// (sizes up to kMaxPlane do y, z and y in the z slot) standing in for the reference's EEuler (TTSH3D.cu:347-359: 107 kernel
 // launches and 4 cuFFT transforms per step).
 //
 // ttsh_sim is an engine with one slot stepped with plain launches.  A
@@ -46,23 +46,28 @@ thread_local LaunchEvents g_launch_ev;
             return fail(TTSH_EHIP, std::string(#expr " failed: ") + hipGetErrorString(e_));           \
     } while (0)
 
-// Kernel kinds of one step, in launch order.  K_fft_xy is the x pass, or the
-// fused x+y pass for sizes N <= 128 of which the batch holds at least two
-// z-planes per CU (those sizes then have no work in K_fft_y, K_fft_y_inv).
+// Kernel kinds of one step, in launch order.  K_fft_xy and K_fft_xy_inv are
+// the x passes; K_fft_z_poisson is the z pass, or for sizes up to kMaxPlane
+// the plane kernel that does both y passes too (those sizes then have no work
+// in K_fft_y, K_fft_y_inv).
 enum { KK_RHS = 0, KK_DIV, KK_FX, KK_FY, KK_FZ, KK_FYI, KK_FXI, KK_CORR, KK_N };
 static const char* const kKindNames[KK_N] = {"K_rhs", "K_div", "K_fft_xy", "K_fft_y", "K_fft_z_poisson",
                                              "K_fft_y_inv", "K_fft_xy_inv", "K_corr"};
 
-// Work tables: rhs, div, one item per droplet (the projection's sums), corr,
-// the x/y-pass and z-pass tables of a launch that covers several sizes, and
-// per grid size the x/y-pass table, the z-pass table and the z-plane table of
-// the fused x+y pass.
-enum { T_RHS = 0, T_PROJ = 1, T_STAT = 2, T_CORR = 3, T_MXY = 4, T_MZ = 5, T_FFT0 = 6 };
+// Work tables: rhs, div, one item per droplet (the projection's sums), corr;
+// of FFT launches that cover several sizes, the x, y and z passes and the y-z
+// planes of the two plane groups; per grid size the line groups of x or y
+// passes, of the z pass, and the y-z planes.
+enum { T_RHS = 0, T_PROJ = 1, T_STAT = 2, T_CORR = 3, T_MX = 4, T_MY = 5, T_MZ = 6, T_MP = 7, T_FFT0 = 9 };
 constexpr int kNTables = T_FFT0 + 3 * kNumGridSizes;
 static_assert(kNumGridSizes <= 32, "sizes are kept as bits of a 32-bit mask");
-static inline int t_xy(int s) { return T_FFT0 + 3 * s; }      // line groups of x or y passes
-static inline int t_z(int s) { return T_FFT0 + 3 * s + 1; }   // line groups of the z pass
-static inline int t_pl(int s) { return T_FFT0 + 3 * s + 2; }  // z-planes of the fused x+y pass
+static inline int t_xy(int s) { return T_FFT0 + 3 * s; }
+static inline int t_z(int s) { return T_FFT0 + 3 * s + 1; }
+static inline int t_pl(int s) { return T_FFT0 + 3 * s + 2; }
+
+// Sizes whose y and z transforms run on y-z planes, and their plane group.
+static inline bool has_planes(int s) { return kGridSizes[s] <= kMaxPlane; }
+static inline int plane_group(int s) { return kGridSizes[s] <= kSmallPlane ? 0 : 1; }
 
 static int size_index(int N)
 {
@@ -73,6 +78,13 @@ static int size_index(int N)
 
 static inline size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
+// Bytes from one field to the next.  Fields whose distance is a power of two
+// put the same cell of every field on the same memory channels; a shift of 17
+// times 256 bytes per field took K_corr at 256^3 from 196 to 188 us, K_div from
+// 147 to 143 and the step of the 20-droplet sweep from 1201 to 1173 (256 bytes
+// do most of it, 129 times 256 no more).
+static inline size_t falign(size_t b) { return align256(b) + 17 * 256; }
+
 // Upper bound of divergence work items of one droplet (z-depth >= 1).
 static int proj_items_max(int N)
 {
@@ -82,9 +94,9 @@ static int proj_items_max(int N)
 size_t droplet_bytes(int N)
 {
     const size_t n = (size_t)N * N * N;
-    return 20 * align256(n * sizeof(float)) + align256(n * sizeof(float2)) +
+    return 20 * falign(n * sizeof(float)) + align256(n * sizeof(float2)) +
            align256((size_t)proj_items_max(N) * kPartSums * sizeof(double)) + align256(2 * sizeof(double)) +
-           align256(sizeof(float)) + align256(n * sizeof(float));
+           align256(sizeof(float)) + falign(n * sizeof(float));
 }
 
 // K_rhs variant of a size without a tuning entry; 16x16 fits every supported N.
@@ -152,15 +164,16 @@ struct Engine {
     // graphs, one per starting parity; the sizes present at capture
     hipGraphExec_t gexec[2] = {nullptr, nullptr};
     int ggrid[kNTables] = {};
-    // What the FFT launches cover: the sizes present, those that run the fused
-    // x+y pass, and whether the x and y passes of the other sizes, and the z
-    // passes of all, are one launch for several sizes (T_MXY, T_MZ).
+    // What the FFT launches cover: the sizes present, and which launches serve
+    // several sizes: x passes (T_MX), y and z passes (T_MY, T_MZ), planes of
+    // each group (T_MP).
     struct FftLayout {
-        unsigned sizes = 0, xy_mask = 0;
-        bool mxy = false, mz = false;
+        unsigned sizes = 0;
+        bool mx = false, mz = false, mp[2] = {false, false};
+        bool fold = false;  // the x pass does k_proj_stats' work
         bool covers(const FftLayout& o) const
         {
-            return !(o.sizes & ~sizes) && xy_mask == o.xy_mask && mxy == o.mxy && mz == o.mz;
+            return !(o.sizes & ~sizes) && mx == o.mx && mz == o.mz && fold == o.fold && mp[0] == o.mp[0] && mp[1] == o.mp[1];
         }
     };
     FftLayout fft, gfft;  // of the current tables, and at capture
@@ -541,7 +554,7 @@ struct Engine {
         char* b = static_cast<char*>(mem);
         auto take = [&](size_t sz) {
             char* r = b;
-            b += align256(sz);
+            b += sz == n * 4 ? falign(sz) : align256(sz);
             return r;
         };
         Drop& D = s.drop;
@@ -561,6 +574,7 @@ struct Engine {
         for (int q = 0; q < 2; ++q)
             for (int a = 0; a < 3; ++a) D.ps[q][a] = (float*)take(n * 4);
         D.c = (float2*)take(n * 8);
+        D.ct = (float2*)D.P[0];  // 12 n bytes in a row, of which it takes 8 n
         D.part = (double*)take((size_t)proj_items_max(N) * kPartSums * sizeof(double));
         D.stat = (double*)take(2 * sizeof(double));
         D.sigma = (float*)take(sizeof(float));
@@ -722,6 +736,40 @@ struct Engine {
         return (rounds < 3.0 ? std::ceil(rounds) : rounds + 0.5) * (deepest + over);
     }
 
+    // Reduction blocks of a divergence item: items of about d planes, and at
+    // most eight blocks, since a block's sums cost about half a plane and
+    // droplets with blocks of one plane would hold up the launch.
+    static int div_blocks(const Slot& s, int d)
+    {
+        const int nzp = (s.N + s.proj_tz - 1) / s.proj_tz;
+        return std::max(1, std::min({nzp, 8, d * nzp / s.N}));
+    }
+
+    // Depth (at most `most`) of K_div's items with the least predicted time
+    // over the active droplets: all items over two groups per CU, and half of
+    // the longest item for the end.
+    int div_depth(int most) const
+    {
+        int depth = 1;
+        double best = 0.0;
+        for (int d = 1; d <= most; ++d) {
+            double all = 0.0, longest = 0.0;
+            for (const Slot& s : slots) {
+                if (!s.used || remaining(s) <= 0) continue;
+                const int nzp = (s.N + s.proj_tz - 1) / s.proj_tz, g = div_blocks(s, d);
+                const double c = (double)s.N * g / nzp + 3.0 + 0.5 * g;
+                all += c * proj_tiles(s.N) * ((nzp + g - 1) / g);
+                longest = std::max(longest, c);
+            }
+            const double rounds = all / (2.0 * cus * longest);
+            const double t = rounds < 1.0 ? longest : all / (2.0 * cus) + 0.5 * longest;
+            if (d > 1 && t >= best) continue;
+            best = t;
+            depth = d;
+        }
+        return depth;
+    }
+
     // The layout of the next launches.  One droplet: its tuned tile and depths
     // (the engine's tile if it asks for one).  Several that do not fill the
     // device: each one's tuned depths would be cut for the whole device, so
@@ -749,7 +797,8 @@ struct Engine {
         if (batch_layout()) {
             l.variant = batch_rhs_variant;
             l.rhs_tz = batch_rhs_tz;
-            l.div_tz = l.corr_tz = batch_corr_tz;
+            l.corr_tz = batch_corr_tz;
+            l.div_tz = div_depth(batch_corr_tz);
             l.deep = true;
             return l;
         }
@@ -771,7 +820,7 @@ struct Engine {
                 if (chunk_time(k, 3.0, at_once, tiles) < chunk_time(d, 3.0, at_once, tiles)) d = k;
             return d;
         };
-        l.div_tz = least(2.0 * cus, [](int n) { return proj_tiles(n); });
+        l.div_tz = div_depth(N);
         l.corr_tz = least(4.0 * cus, corr_tiles);
         return l;
     }
@@ -784,6 +833,8 @@ struct Engine {
         HIPCHK(uploads_into_st());
         up_pending = false;
         std::vector<Work> w[kNTables];
+        size_t xgroups = 0;  // work-groups of an x pass
+        bool foldable = true;
         const Layout lay = layout();
         if (lay.variant != rhs_active) {
             HIPCHK(hipStreamSynchronize(st));
@@ -819,8 +870,7 @@ struct Engine {
             // (one, except in a batch)
             const int ntile = proj_tiles(N);
             const int nzp = (N + s.proj_tz - 1) / s.proj_tz;
-            const int dtz = s.prm.corr_tz > 0 ? 0 : lay.div_tz;
-            const int g = dtz > 0 ? std::max(1, std::min(nzp, dtz * nzp / N)) : 1;
+            const int g = s.prm.corr_tz <= 0 && lay.div_tz > 0 ? div_blocks(s, lay.div_tz) : 1;
             for (int k0 = 0; k0 < nzp; k0 += g) {
                 const int k1 = std::min(nzp, k0 + g);
                 const int zb = k0 * N / nzp, ze = k1 * N / nzp;
@@ -838,43 +888,62 @@ struct Engine {
                 const int zb = k * N / nzc, ze = (k + 1) * N / nzc;
                 for (int t = 0; t < corr_tiles(N); ++t) w[T_CORR].push_back(Work{si, t, zb | (ze << 16), 0});
             }
-            // k_proj_stats sums the blocks' FP64 partial sums in block order
+            // the blocks' FP64 partial sums are added by k_proj_stats or the x pass
             h_drops[si].npart = nzp * ntile;
             h_drops[si].nzp = nzp;
             w[T_STAT].push_back(Work{si, 0, 0, 0});
+            xgroups += (size_t)N * (N / fft_lines_per_group(N));
+            foldable = foldable && N <= kMaxPlane && nzp * ntile <= kFoldedParts;
             const int sidx = size_index(N);
             const int L = fft_lines_per_group(N);
-            const bool planes = fft_xy_fused(N);
             for (int b = 0; b < N; ++b) {
-                if (planes) w[t_pl(sidx)].push_back(Work{si, 0, b, 0});
+                if (has_planes(sidx)) w[t_pl(sidx)].push_back(Work{si, 0, b, 0});
                 for (int a = 0; a < N / L; ++a) {
                     w[t_xy(sidx)].push_back(Work{si, a, b, 0});
-                    w[t_z(sidx)].push_back(Work{si, a, b, 0});
+                    if (!has_planes(sidx)) w[t_z(sidx)].push_back(Work{si, a, b, 0});
                 }
             }
         }
-        // The fused x+y pass puts one work-group on each z-plane; it pays only
-        // when a size has enough planes to give every CU two of them (a
-        // batch), otherwise the per-plane transform work leaves CUs idle and
-        // the single-axis passes are faster.
+        // Several sizes share one launch per pass (k_fft_sizes, k_fft_yz_sizes),
+        // the largest first: a launch costs at least 4 us, as much as the pass
+        // itself for one small droplet.  A plane group's launch has the LDS of
+        // its largest size, so its sizes share one only while the planes do
+        // not fill the device anyway.
         fft = FftLayout();
+        size_t planes[2] = {0, 0};
+        int nsz = 0, nlarge = 0, npl[2] = {0, 0};
         for (int sz = 0; sz < kNumGridSizes; ++sz) {
-            if (!w[t_z(sz)].empty()) fft.sizes |= 1u << sz;
-            if (w[t_pl(sz)].size() >= 2 * (size_t)cus) fft.xy_mask |= 1u << sz;
+            if (w[t_xy(sz)].empty()) continue;
+            fft.sizes |= 1u << sz;
+            ++nsz;
+            if (has_planes(sz)) {
+                ++npl[plane_group(sz)];
+                planes[plane_group(sz)] += w[t_pl(sz)].size();
+            } else {
+                ++nlarge;
+            }
         }
-        // Several sizes share one launch per pass (k_fft_sizes), the largest
-        // first: a launch costs at least 4 us, as much as the pass itself for
-        // one small droplet.
-        auto several = [](unsigned m) { return (m & (m - 1)) != 0; };
-        fft.mxy = several(fft.sizes & ~fft.xy_mask);
-        fft.mz = several(fft.sizes);
-        auto merge = [&](int to, int from) {
-            w[to].insert(w[to].end(), w[from].begin(), w[from].end());
-            w[from].clear();
-        };
+        // few groups: the x pass adds up the projection's sums by itself
+        fft.fold = foldable && xgroups <= 4 * (size_t)cus;
+        if (fft.fold) w[T_STAT].clear();
+        fft.mx = nsz > 1;
+        fft.mz = nlarge > 1;
+        for (int g = 0; g < 2; ++g) fft.mp[g] = npl[g] > 1 && (g == 0 || planes[g] < 2 * (size_t)cus);
+        auto merge = [&](int to, int from) { w[to].insert(w[to].end(), w[from].begin(), w[from].end()); };
         for (int sz = kNumGridSizes - 1; sz >= 0; --sz) {
-            if (fft.mxy && !((fft.xy_mask >> sz) & 1u)) merge(T_MXY, t_xy(sz));
-            if (fft.mz) merge(T_MZ, t_z(sz));
+            const bool pl = has_planes(sz);
+            if (fft.mx) merge(T_MX, t_xy(sz));
+            if (!pl && fft.mz) {
+                merge(T_MY, t_xy(sz));
+                merge(T_MZ, t_z(sz));
+                w[t_z(sz)].clear();
+            }
+            if (pl && fft.mp[plane_group(sz)]) {
+                merge(T_MP + plane_group(sz), t_pl(sz));
+                w[t_pl(sz)].clear();
+            }
+            // a lone large size still runs its y passes from its own table
+            if (fft.mx && (pl || fft.mz)) w[t_xy(sz)].clear();
         }
         for (int k = 0; k < kNTables; ++k) {
             const int cnt = (int)w[k].size();
@@ -914,29 +983,33 @@ struct Engine {
         struct L {
             int kind, what, s, t;
         };
-        enum { W_RHS, W_DIV, W_STAT, W_FFT, W_FFT_SIZES, W_FFT_XY, W_CORR };
-        L list[4 + 5 * (kNumGridSizes + 1)];
+        enum { W_RHS, W_DIV, W_STAT, W_FFT, W_FFT_SIZES, W_YZ, W_YZ_SIZES, W_CORR };
+        L list[4 + 5 * (kNumGridSizes + 2)];
         int nl = 0;
         auto add = [&](int kind, int what, int s, int t) {
             if (grid(t) > 0) list[nl++] = L{kind, what, s, t};
         };
         add(KK_RHS, W_RHS, 0, T_RHS);
         add(KK_DIV, W_DIV, 0, T_PROJ);
-        add(KK_DIV, W_STAT, 0, T_STAT);
-        // x, y, z-Poisson, y inverse, x inverse; sizes with the fused x+y
-        // pass do x+y in the x slots and nothing in the y slots
+        if (!fl.fold) add(KK_DIV, W_STAT, 0, T_STAT);
+        // x, y, z-Poisson, y inverse, x inverse; sizes with planes do the middle
+        // three in the z slot
         const int axes[5] = {0, 1, 2, 1, 0};
-        const int modes[5] = {FFT_MODE_FWD, FFT_MODE_FWD, FFT_MODE_POISSON, FFT_MODE_INV, FFT_MODE_INV};
+        const int modes[5] = {fl.fold ? FFT_MODE_FWD_FOLD : FFT_MODE_FWD, FFT_MODE_FWD, FFT_MODE_POISSON, FFT_MODE_INV, FFT_MODE_INV};
         for (int f = 0; f < 5; ++f) {
-            const bool z = axes[f] == 2;
-            if (z ? fl.mz : fl.mxy) add(KK_FX + f, W_FFT_SIZES, 0, z ? T_MZ : T_MXY);
-            for (int s = 0; s < kNumGridSizes; ++s) {
+            const int ax = axes[f];
+            const bool all = ax == 0 ? fl.mx : fl.mz;
+            if (all) add(KK_FX + f, W_FFT_SIZES, 0, ax == 0 ? T_MX : ax == 1 ? T_MY : T_MZ);
+            if (ax == 2)
+                for (int g = 0; g < 2; ++g)
+                    if (fl.mp[g]) add(KK_FX + f, W_YZ_SIZES, g, T_MP + g);
+            for (int s = kNumGridSizes - 1; s >= 0; --s) {
                 if (!((fl.sizes >> s) & 1u)) continue;
-                if (!z && ((fl.xy_mask >> s) & 1u)) {
-                    if (axes[f] == 0) add(KK_FX + f, W_FFT_XY, s, t_pl(s));
-                    continue;
+                if (ax != 0 && has_planes(s)) {
+                    if (ax == 2 && !fl.mp[plane_group(s)]) add(KK_FX + f, W_YZ, s, t_pl(s));
+                } else if (!all) {
+                    add(KK_FX + f, W_FFT, s, ax == 2 ? t_z(s) : t_xy(s));
                 }
-                if (!(z ? fl.mz : fl.mxy)) add(KK_FX + f, W_FFT, s, z ? t_z(s) : t_xy(s));
             }
         }
         add(KK_CORR, W_CORR, 0, T_CORR);
@@ -956,7 +1029,8 @@ struct Engine {
             case W_RHS: e = launch_rhs(rhs_active, d_drops, tab[T_RHS].d, cnt + T_RHS, parity, kstep, grid(T_RHS), st); break;
             case W_DIV: e = launch_div(d_drops, tab[T_PROJ].d, cnt + T_PROJ, parity, kstep, grid(T_PROJ), st); break;
             case W_STAT: e = launch_proj_stats(d_drops, tab[T_STAT].d, cnt + T_STAT, kstep, grid(T_STAT), st); break;
-            case W_FFT_XY: e = launch_fft_xy(N, modes[f], d_drops, tab[l.t].d, cnt + l.t, kstep, grid(l.t), st); break;
+            case W_YZ: e = launch_fft_yz(N, d_drops, tab[l.t].d, cnt + l.t, kstep, grid(l.t), st); break;
+            case W_YZ_SIZES: e = launch_fft_yz_sizes(l.s, d_drops, tab[l.t].d, cnt + l.t, kstep, grid(l.t), st); break;
             case W_FFT_SIZES: e = launch_fft_sizes(axes[f], modes[f], d_drops, tab[l.t].d, cnt + l.t, kstep, grid(l.t), st); break;
             case W_FFT: e = launch_fft(N, axes[f], modes[f], d_drops, tab[l.t].d, cnt + l.t, kstep, grid(l.t), st); break;
             default: e = launch_corr(d_drops, tab[T_CORR].d, cnt + T_CORR, parity, kstep, grid(T_CORR), st); break;
@@ -976,7 +1050,7 @@ struct Engine {
         // as do FFT items of several sizes: one work-group per table slot
         // leaves their balance to the hardware dispatcher instead of a fixed
         // stride over the items
-        for (int t : {T_RHS, T_PROJ, T_CORR, T_MXY, T_MZ}) ggrid[t] = ((tab[t].cap + kXcds - 1) / kXcds) * kXcds;
+        for (int t : {(int)T_RHS, (int)T_PROJ, (int)T_CORR, (int)T_MX, (int)T_MY, (int)T_MZ, (int)T_MP, T_MP + 1}) ggrid[t] = ((tab[t].cap + kXcds - 1) / kXcds) * kXcds;
         gfft = fft;
         hipGraph_t graph = nullptr;
         HIPCHK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));

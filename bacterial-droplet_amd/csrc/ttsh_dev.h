@@ -62,6 +62,9 @@ struct Drop {
     float* vs[2][3];
     float* ps[2][3];
     float2* c;
+    // transposed copy of c, [x][z][y], of sizes up to kMaxPlane: the memory of
+    // P and v, whose values are not used between K_rhs and K_corr
+    float2* ct;
     // FP64 sums per reduction block, kPartSums each: s.x, s.y, s.x^2, s.y^2
     // over the block's cells and |v*|^2, |P*|^2 over the same cells.  A block
     // is one divergence tile over one of nzp z-ranges (the droplet's tuned
@@ -193,6 +196,81 @@ __device__ __forceinline__ float from_right(float a)
 }
 __device__ __forceinline__ float xpair(float a) { return from_left(a) + from_right(a); }
 __device__ __forceinline__ float xdiff(float a) { return from_right(a) - from_left(a); }
+
+// Adds to each value the one that DPP control CTRL brings, 0 where none comes.
+template <int CTRL, int N>
+__device__ __forceinline__ void dpp_add(double (&e)[N])
+{
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+        const unsigned long long b = __double_as_longlong(e[k]);
+        const unsigned lo = __builtin_amdgcn_update_dpp(0, (int)(unsigned)b, CTRL, 0xf, 0xf, false);
+        const unsigned hi = __builtin_amdgcn_update_dpp(0, (int)(unsigned)(b >> 32), CTRL, 0xf, 0xf, false);
+        e[k] += __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+    }
+}
+
+// Sums over a wave, complete in lane 63: row_shr 1, 2, 4, 8 and the two row
+// broadcasts.  Shuffles through LDS would take 72 ds_bpermute, 3 us for the 16
+// waves of a work-group; this takes 0.7.
+template <int N>
+__device__ __forceinline__ void wave_sum(double (&e)[N])
+{
+    dpp_add<0x111>(e);
+    dpp_add<0x112>(e);
+    dpp_add<0x114>(e);
+    dpp_add<0x118>(e);
+    dpp_add<0x142>(e);
+    dpp_add<0x143>(e);
+}
+
+// log2 x for x >= 0 (-inf at 0, +inf at inf): exponent plus the FP32 log2 of
+// the mantissa, enough for a rounded power of two
+__device__ __forceinline__ double log2_coarse(double x)
+{
+    if (!(x > 0.0)) return -INFINITY;
+    if (x == INFINITY) return INFINITY;
+    int ex;
+    const double m = frexp(x, &ex);
+    return (double)ex + (double)log2f((float)m);
+}
+
+// log2 of this step's sigma from the projection's sums (derivation in
+// k_proj.hip).  log2 of 0 is -inf, of inf +inf; -inf + inf is NaN.
+__device__ __forceinline__ int proj_sigma_log2(const double (&t)[kPartSums])
+{
+    const double l = 0.25 * ((log2_coarse(t[3]) + log2_coarse(t[5])) - (log2_coarse(t[2]) + log2_coarse(t[4])));
+    return t[3] > 0.0 && l == l ? (int)rint(fmin(fmax(l, -30.0), 30.0)) : 0;
+}
+__device__ __forceinline__ void put_proj_stats(const Drop& D, const double (&t)[kPartSums], int e)
+{
+    glb(D.sigma)[0] = ldexpf(1.f, e);
+    glb(D.stat)[0] = t[0];
+    glb(D.stat)[1] = ldexp(t[1], -e);
+}
+
+// The projection's sums of a droplet of at most kFoldedParts reduction blocks,
+// by one wave: lane l adds the blocks l, l + 64, ..., then the lanes are added;
+// t is complete in lane 63.  In a forward x pass of few work-groups every one
+// does this while its lines are on their way (FFT_MODE_FWD_FOLD), which saves
+// the launch of k_proj_stats: steps of 36.1 -> 34.8 us at 32^3, 51.4 -> 49.5 at
+// 64^3, 130 -> 128 at 128^3.  With many groups the repeated sums cost more
+// than the launch (the 20-droplet sweep: x pass 58 -> 87 us).  The order does
+// not depend on the work-group or the kernel, so all get the same sigma.
+constexpr int kFoldedParts = 512;
+__device__ __forceinline__ void fold_proj_stats(const Drop& D, int lane, double (&t)[kPartSums])
+{
+    const gptr<const double> pt = glb<const double>(D.part);
+    const int np = D.npart;
+#pragma unroll
+    for (int k = 0; k < kPartSums; ++k) t[k] = 0.0;
+#pragma unroll 4
+    for (int j = lane; j < np; j += 64) {
+#pragma unroll
+        for (int k = 0; k < kPartSums; ++k) t[k] += pt[(size_t)kPartSums * j + k];
+    }
+    wave_sum(t);
+}
 
 // Compile-time phase of an unrolled z-march (register slot rotation).
 template <int K>

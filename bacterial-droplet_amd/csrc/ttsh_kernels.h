@@ -42,7 +42,10 @@ constexpr int kCorrTX = 32;
 constexpr int kCorrTY = 8;
 
 // FFT pass kinds (k_fft.hip).
-enum { FFT_MODE_FWD = 0, FFT_MODE_INV = 1, FFT_MODE_POISSON = 2 };
+// FFT_MODE_FWD_FOLD: a forward x
+// pass that also does k_proj_stats' work (sizes up to kMaxPlane, droplets of at
+// most kFoldedParts reduction blocks).
+enum { FFT_MODE_FWD = 0, FFT_MODE_INV = 1, FFT_MODE_POISSON = 2, FFT_MODE_FWD_FOLD = 3 };
 
 hipError_t launch_rhs(int variant, const Drop* drops, const Work* work, const int* nwork_p, int parity, int kstep,
                       int grid, hipStream_t st);
@@ -67,8 +70,9 @@ hipError_t launch_fill_u32(void* p, uint32_t value, size_t n, hipStream_t st);
 // v = v* - Dt D p_v, P = P* - Dt D p_p from p_v + i p_p.
 hipError_t launch_corr(const Drop* drops, const Work* work, const int* nwork_p, int parity, int kstep, int grid,
                        hipStream_t st);
-// One FFT pass along axis (0 x, 1 y, 2 z) for droplets of size N.  mode
-// FFT_MODE_POISSON (z only): forward, times -1/(k^2 N^3), inverse.
+// One FFT pass along axis (0 x, 1 y, 2 z) for droplets of size N; x only for
+// N <= kMaxPlane.  mode FFT_MODE_POISSON (z only): forward, times
+// -1/(k^2 N^3), inverse.
 hipError_t launch_fft(int N, int axis, int mode, const Drop* drops, const Work* work, const int* nwork_p, int kstep,
                       int grid, hipStream_t st);
 // The same pass for droplets of any planned sizes in one launch.
@@ -76,14 +80,16 @@ hipError_t launch_fft_sizes(int axis, int mode, const Drop* drops, const Work* w
                             int grid, hipStream_t st);
 // Lines per FFT work item for size N (0 if N has no plan).
 int fft_lines_per_group(int N);
-// Sizes up to this have the fused x+y pass (one work-group per z-plane,
-// the plane in LDS).
-constexpr int kMaxFusedXy = 128;
-bool fft_xy_fused(int N);
-// Fused x and y passes over every z-plane (work item (d, -, z)): mode
-// FFT_MODE_FWD transforms x then y, FFT_MODE_INV y then x.
-hipError_t launch_fft_xy(int N, int mode, const Drop* drops, const Work* work, const int* nwork_p, int kstep, int grid,
+// Sizes up to kMaxPlane run their y and z transforms in one kernel, a y-z
+// plane in LDS per work-group (work item (d, -, x)): launch_fft_yz for one
+// size, launch_fft_yz_sizes for those of group 0 (up to kSmallPlane, 33 KB of
+// LDS) or group 1 (the others, 132 KB).
+constexpr int kMaxPlane = 128;
+constexpr int kSmallPlane = 64;
+hipError_t launch_fft_yz(int N, const Drop* drops, const Work* work, const int* nwork_p, int kstep, int grid,
                          hipStream_t st);
+hipError_t launch_fft_yz_sizes(int group, const Drop* drops, const Work* work, const int* nwork_p, int kstep, int grid,
+                               hipStream_t st);
 // Diagnostics (k_diag.hip): FP64 sums of phi, phi*y, phi*x, phi*z -> out[4]
 // (part holds 4*nblk doubles); plane z of phi, v, P and the 4th-order
 // vorticities of v and P -> out[9][N][N] (out has 9*N*N+1 floats; z < 0 takes

@@ -35,7 +35,8 @@ TUNED_VARIANTS = (1, 3)
 # computes two planes more than it stores, and the number of chunks times the
 # tiles of a plane should come just below a multiple of the CUs
 RHS_DEPTHS = (1, 2, 3, 4, 5, 6, 8, 9, 10, 11, 13, 16, 18, 20, 22, 24, 26, 29, 32, 36, 40, 43, 48, 52, 60, 64, 86, 128)
-PROJ_DEPTHS = (1, 2, 3, 4, 6, 8, 11, 16, 22, 32)
+# not 1: a batch has to add up every one of its planes by itself
+PROJ_DEPTHS = (2, 3, 4, 6, 8, 11, 16, 22, 32)
 DEFAULT_TABLE = os.path.join(os.path.dirname(LIB_PATH), "tuned.txt")
 
 
