@@ -540,6 +540,31 @@ hipError_t launch_fill_edges(const float* const vs[3], const float* const ps[3],
     return hipGetLastError();
 }
 
+// Field blockIdx.y of a list, n elements each (floats, or groups of four where
+// every address is a multiple of 16 bytes).  One launch for the 13 fields of a
+// state: 13 copies of the runtime cost a call of one 32^3 step 70 us on each
+// side of the step, this 5.
+template <typename T>
+__global__ __launch_bounds__(256) void k_copy_fields(FieldList f, unsigned n)
+{
+    const gptr<const T> src = glb((const T*)f.src[blockIdx.y]);
+    const gptr<T> dst = glb((T*)f.dst[blockIdx.y]);
+    for (unsigned i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) dst[i] = src[i];
+}
+
+hipError_t launch_copy_fields(const FieldList& f, size_t n, hipStream_t st)
+{
+    if (f.count <= 0 || n == 0) return hipSuccess;
+    size_t bits = n * sizeof(float);
+    for (int k = 0; k < f.count; ++k) bits |= (size_t)f.src[k] | (size_t)f.dst[k];
+    const bool wide = bits % 16 == 0;
+    const unsigned m = (unsigned)(wide ? n / 4 : n);
+    const dim3 grid(std::min((m + 255) / 256, 64u), f.count);
+    if (wide) hipLaunchKernelGGL(k_copy_fields<fvec4>, grid, dim3(256), 0, st, f, m);
+    else hipLaunchKernelGGL(k_copy_fields<float>, grid, dim3(256), 0, st, f, m);
+    return hipGetLastError();
+}
+
 // Fill n 32-bit words with a value (vector stores; grid-stride).
 __global__ __launch_bounds__(256) void k_fill_u32(uint32_t* __restrict__ p, uint32_t value, size_t n)
 {

@@ -72,8 +72,6 @@
 
 namespace ttsh {
 
-typedef float fvec4 __attribute__((ext_vector_type(4)));
-
 // Keeps the compiler from sinking a value's computation past this point: sunk
 // past a barrier, all its inputs would stay live instead of the one value.
 __device__ __forceinline__ void pin(float& a) { asm volatile("" : "+v"(a)); }

@@ -1257,15 +1257,17 @@ struct Engine {
         Slot& s = slots[si];
         HIPCHK(hipSetDevice(device));
         normalise_parity();
-        const size_t n = (size_t)s.N * s.N * s.N, b = n * sizeof(float);
+        const size_t n = (size_t)s.N * s.N * s.N;
         const int q = s.q;
-        HIPCHK(hipMemcpyAsync(s.drop.phi[q], phi, b, hipMemcpyDeviceToDevice, st));
+        FieldList f{};
+        f.add(phi, s.drop.phi[q]);
         for (int a = 0; a < 3; ++a) {
-            HIPCHK(hipMemcpyAsync(s.drop.P[a], P + a * n, b, hipMemcpyDeviceToDevice, st));
-            HIPCHK(hipMemcpyAsync(s.drop.v[a], v + a * n, b, hipMemcpyDeviceToDevice, st));
-            HIPCHK(hipMemcpyAsync(s.drop.vs[q ^ 1][a], vsp + a * n, b, hipMemcpyDeviceToDevice, st));
-            HIPCHK(hipMemcpyAsync(s.drop.ps[q ^ 1][a], psp + a * n, b, hipMemcpyDeviceToDevice, st));
+            f.add(P + a * n, s.drop.P[a]);
+            f.add(v + a * n, s.drop.v[a]);
+            f.add(vsp + a * n, s.drop.vs[q ^ 1][a]);
+            f.add(psp + a * n, s.drop.ps[q ^ 1][a]);
         }
+        HIPCHK(launch_copy_fields(f, n, st));
         const float* vs[3] = {s.drop.vs[q ^ 1][0], s.drop.vs[q ^ 1][1], s.drop.vs[q ^ 1][2]};
         const float* ps[3] = {s.drop.ps[q ^ 1][0], s.drop.ps[q ^ 1][1], s.drop.ps[q ^ 1][2]};
         HIPCHK(launch_fill_edges(vs, ps, s.drop.edge, s.drop.eslot[q ^ 1], s.N, st));
@@ -1280,15 +1282,17 @@ struct Engine {
     {
         Slot& s = slots[si];
         HIPCHK(hipSetDevice(device));
-        const size_t n = (size_t)s.N * s.N * s.N, b = n * sizeof(float);
+        const size_t n = (size_t)s.N * s.N * s.N;
         const int last = s.q ^ 1;  // parity of the last step's predictors
-        HIPCHK(hipMemcpyAsync(phi, s.drop.phi[s.q], b, hipMemcpyDeviceToDevice, st));
+        FieldList f{};
+        f.add(s.drop.phi[s.q], phi);
         for (int a = 0; a < 3; ++a) {
-            HIPCHK(hipMemcpyAsync(P + a * n, s.drop.P[a], b, hipMemcpyDeviceToDevice, st));
-            HIPCHK(hipMemcpyAsync(v + a * n, s.drop.v[a], b, hipMemcpyDeviceToDevice, st));
-            HIPCHK(hipMemcpyAsync(vs_out + a * n, s.drop.vs[last][a], b, hipMemcpyDeviceToDevice, st));
-            HIPCHK(hipMemcpyAsync(ps_out + a * n, s.drop.ps[last][a], b, hipMemcpyDeviceToDevice, st));
+            f.add(s.drop.P[a], P + a * n);
+            f.add(s.drop.v[a], v + a * n);
+            f.add(s.drop.vs[last][a], vs_out + a * n);
+            f.add(s.drop.ps[last][a], ps_out + a * n);
         }
+        HIPCHK(launch_copy_fields(f, n, st));
         return TTSH_OK;
     }
 

@@ -150,6 +150,7 @@ __device__ __forceinline__ gptr<T> glb(T* p)
 // HIP float2 class has no assignment operators for an address-space-qualified
 // object.
 typedef float fvec2 __attribute__((ext_vector_type(2)));
+typedef float fvec4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ float2 ld2(gptr<const float2> p, size_t i)
 {
     const fvec2 t = *(gptr<const fvec2>)(p + i);
