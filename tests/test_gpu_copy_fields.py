@@ -1,34 +1,52 @@
 """ttsh_step_noalloc copies a state in and out with one kernel each, 16 bytes at
 a time where every array begins on a 16-byte boundary and 4 otherwise.  Caller
 arrays at offsets of 0 to 3 floats: the state and predictors equal ttsh_step's
-bitwise, and the floats around each array stay as they were."""
+bitwise, and the floats around each array stay as they were.  Device memory
+comes from the HIP runtime that the library itself loads, through ctypes."""
+import ctypes
+
 import numpy as np
 import pytest
 
 pytestmark = pytest.mark.gpu
 
+H2D, D2H = 1, 2  # hipMemcpyHostToDevice, hipMemcpyDeviceToHost
+
 
 @pytest.mark.parametrize("N,offset", [(32, 0), (32, 1), (36, 2), (50, 3), (64, 0), (64, 1)])
 def test_offsets(ttsh, N, offset):
-    import torch
     print(f"[copy_fields N={N} offset={offset}]", flush=True)
+    ttsh.lib()
+    hip = ctypes.CDLL("libamdhip64.so.7")
+    hip.hipMalloc.argtypes = [ctypes.POINTER(ctypes.c_void_p), ctypes.c_size_t]
+    hip.hipFree.argtypes = [ctypes.c_void_p]
+    hip.hipMemcpy.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_int]
     rng = np.random.default_rng(N + offset)
     r = lambda k: rng.uniform(-1, 1, (k, N, N, N)).astype(np.float32)
     state = (0.5 + 0.4 * r(1)[0], r(3), 0.1 * r(3))
     prev = (0.1 * r(3), r(3))
     p = ttsh.default_params(N=N, dt0=0.005)
+    begin = 4 + offset
     held = []
-    for a in (*state, *prev):
-        t = torch.full((a.size + 8,), 7.0, device="cuda")
-        t[4 + offset:4 + offset + a.size] = torch.from_numpy(a.reshape(-1)).cuda()
-        held.append((t, a.size))
-    torch.cuda.synchronize()
-    ttsh.step_noalloc(p, *(t.data_ptr() + 4 * (4 + offset) for t, _ in held), 3)
+    try:
+        for a in (*state, *prev):
+            host = np.full(a.size + 8, 7.0, np.float32)
+            host[begin:begin + a.size] = a.reshape(-1)
+            ptr = ctypes.c_void_p()
+            assert hip.hipMalloc(ctypes.byref(ptr), host.nbytes) == 0
+            held.append((ptr, host))
+            assert hip.hipMemcpy(ptr, host.ctypes.data, host.nbytes, H2D) == 0
+        assert hip.hipDeviceSynchronize() == 0
+        ttsh.step_noalloc(p, *(ptr.value + 4 * begin for ptr, _ in held), 3)
+        for ptr, host in held:
+            assert hip.hipMemcpy(host.ctypes.data, ptr, host.nbytes, D2H) == 0
+    finally:
+        for ptr, _ in held:
+            hip.hipFree(ptr)
     with ttsh.Simulation(p) as s:
         s.set_state(*state, *prev, dtype=ttsh.F32)
         s.step(3)
         want = (*s.get_state(), s.aux("vstar"), s.aux("pstar"))
-    for (t, n), b in zip(held, want):
-        got = t.cpu().numpy()
-        assert np.array_equal(got[4 + offset:4 + offset + n], b.reshape(-1))
-        assert (got[:4 + offset] == 7.0).all() and (got[4 + offset + n:] == 7.0).all()
+    for (_, got), b in zip(held, want):
+        assert np.array_equal(got[begin:begin + b.size], b.reshape(-1))
+        assert (got[:begin] == 7.0).all() and (got[begin + b.size:] == 7.0).all()
