@@ -563,8 +563,8 @@ __global__ __launch_bounds__(fft_max_threads(), 4) void k_fft_sizes(const Drop* 
 //
 // What bounds it: VALU and LDS of the CUs that have a plane when there are
 // fewer planes than CUs (a lone droplet), which is still less than the
-// launches and hand-offs between XCDs of three passes: 64^3 13.4 -> 9.2 us,
-// 128^3 31.2 -> 26.
+// launches and hand-offs between XCDs of three passes: 64^3 13.4 -> 6.7 us,
+// 128^3 31.2 -> 18.
 // ===========================================================================
 template <int N>
 struct PlaneCfg {

@@ -44,25 +44,31 @@
 // reads per field where the 2D stencils took 22 values, and each one-axis sum
 // is made once instead of by every neighbour: 44 LDS and 430 VALU
 // instructions per plane and wave.  Measured, same boxes, 16-row tiles
-// against the best of the former tiles: 64^3 37 -> 19 us (with the shallower
-// z-chunks below), 128^3 75 -> 55, 180^3 216 -> 119, 240^3 463 -> 234,
-// 256^3 498 -> 324.
+// against the best of the former tiles: 64^3 37 -> 19 us (in z-chunks of two
+// planes instead of eight), 128^3 75 -> 55 (47 with the flattened tile),
+// 180^3 216 -> 119, 240^3 463 -> 234, 256^3 498 -> 324.
 //
-// Tile: one wave per row of TX <= 60 cells, whose 64 lanes include the 2-cell
-// x apron; NW rows per work-group (8 or 16), one cell per lane.  N is cut
-// into ceil(N/60) tiles of equal width.  Wider tiles would need the apron
-// columns from other waves; two rows per wave (213 VGPRs, two waves per SIMD)
-// measured 4% slower at 128^3 and equal at 240^3 and 256^3.  The rows above
-// and below the tile are staged by all waves, one or two (row, field) pairs
-// each, and the first eight waves compute the intermediates of the two rows
-// next to the tile.
+// Tiles.  W = 64: one wave per row of TX <= 60 cells, whose 64 lanes include
+// the 2-cell x apron; 8 or 16 rows per work-group.  N is cut into ceil(N/60)
+// tiles of equal width.  W = 36: TX <= 32 cells and 26 rows, the tile's rows
+// one after another over 16 waves, each of which holds 60 positions of them
+// and two of its neighbours' on either side.  A wave of a 60-wide tile is
+// idle in part where 60 does not divide N well (64^3, 128^3: a third to a
+// half), a wave of the flattened tile only at its ends.  At 128^3 that makes
+// 20 tiles of 24 and 47 us of 52; where the counts are equal the flattened
+// tile is 3% (96^3) to 11% (256^3, its rows end inside cache lines more often)
+// slower, so the tuning table chooses per size.  Two rows per wave (213
+// VGPRs, two waves per SIMD) measured 4% slower at 128^3 and equal at 240^3
+// and 256^3.  The rows above and below the tile are staged by all waves, one
+// or two (row, field) pairs each, and the first eight waves compute the
+// intermediates of the two rows next to the tile.
 //
-// 16 rows (1024 threads, 128 VGPRs, 160 KB of LDS: one group per CU, four
-// waves per SIMD) have the smaller share of apron rows and are faster
-// wherever the device is full: 240^3 234 against 317 us.  8 rows (98 KB) take
-// 2.1 us per plane instead of 3.2 when a CU holds one group, which wins for
-// small boxes.  Both do the same arithmetic in the same order (no contraction
-// in this file), so a droplet's result does not depend on the tile.
+// 16 waves (128 VGPRs, 160 KB of LDS: one group per CU, four waves per SIMD)
+// have the smaller share of apron rows and are faster wherever the device is
+// full: 240^3 234 against 317 us.  8 waves (98 KB) take 2.1 us per plane
+// instead of 3.2 when a CU holds one group, which wins for small boxes.  All
+// do the same arithmetic in the same order (no contraction in this file), so a
+// droplet's result does not depend on the tile.
 #include <type_traits>
 
 #include "ttsh_dev.h"
@@ -139,19 +145,27 @@ __device__ __forceinline__ float mu0_of(float ph, float l, float kl, float a2)
     return fma_(-kl, l, a2 * fma_(2.f * ph2, ph, fma_(-3.f, ph2, ph)));
 }
 
-template <int NW>
+// NW waves, W records per tile row.  W = 64: a wave is a row.  W < 64: the
+// tile's rows lie one after another and wave w holds the positions 60 w - 2 ..
+// 60 w + 61 of that sequence; the two positions at each end are also those of
+// its neighbours, which store them.
+template <int NW, int W>
 __global__ __launch_bounds__(64 * NW, NW / 4) void k_rhs(const Drop* __restrict__ drops, const Work* __restrict__ work,
                                                          const int* __restrict__ nwork_p, int parity, int kstep)
 {
-    constexpr int HP = NW + 4, HV = NW + 2;  // rows of phi, P records; of v records and intermediates
+    constexpr int TY = rhs_tile_rows(NW, W);
+    // Records of a field: rows -2 .. TY+1 of phi and P; rows -1 .. TY of v and
+    // of the intermediates; with W < 64, 64 more that take what lanes without
+    // a position of their own would store.
+    constexpr int FP = (TY + 4) * W + (W < 64 ? 64 : 0), FV = (TY + 2) * W + (W < 64 ? W + 64 : 0);
     // Two buffers of BUF records.  A plane uses them as: phi, P -> X; the
     // intermediates -> Y; v -> X; then X and Y swap.  Each exchange then
     // writes the buffer whose readers passed the previous barrier.
-    constexpr int BUF = 4 * HP * 64;
-    // intermediates: per component (U, W, B, pm), then (m_0, m_1, m_2, mu0),
-    // then mu0's pm
-    constexpr int IM = 3 * HV * 64, IP = 4 * HV * 64;
-    static_assert(IP + HV * 16 <= BUF, "the intermediates fit a buffer");
+    // Intermediates: per component (U, W, B, pm), then (m_0, m_1, m_2, mu0),
+    // then mu0's pm.
+    constexpr int IM = 3 * FV, IP = 4 * FV;
+    constexpr int BUF = W == 64 ? 4 * FP : IP + (FV + 3) / 4;
+    static_assert(4 * FP <= BUF && IP + (FV + 3) / 4 <= BUF && 32 * BUF <= 160 * 1024, "buffers");
     // apron rows of phi, P staged per wave: (field, inner row) and (field,
     // outer row) for 8 waves, one of them for 16
     constexpr int NT = NW == 8 ? 2 : 1;
@@ -171,8 +185,8 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void k_rhs(const Drop* __restrict_
         const Coef co = D.co;
         const int N = D.N;
         const unsigned NN = (unsigned)N * (unsigned)N;
-        const int TX = rhs_tile_width(N);
-        const int x0 = wk.a * TX, y0 = wk.b * NW;
+        const int TX = rhs_tile_width(N, W);
+        const int x0 = wk.a * TX, y0 = wk.b * TY;
         const int zb = wk.c & 0xffff;
         const int ze = wk.c >> 16;
         const gptr<const float> gin[4] = {glb<const float>(D.phi[parity]), glb<const float>(D.P[0]),
@@ -183,36 +197,51 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void k_rhs(const Drop* __restrict_
         const gptr<float> ovs[3] = {glb(D.vs[parity][0]), glb(D.vs[parity][1]), glb(D.vs[parity][2])};
         const gptr<float> ops[3] = {glb(D.ps[parity][0]), glb(D.ps[parity][1]), glb(D.ps[parity][2])};
 
-        // own cell: lanes 2 .. TX+1 of the row; the other lanes load the
-        // apron (or, past it, any cell: x0 + lane - 2 < 2 N since N >= 32)
-        const int gx = x0 + lane - 2, gy = y0 + wv;
+        // own cell: columns 2 .. TX+1 of a row; the other columns are apron
+        // (or, past it, any cell: x0 + 61 < 2 N since N >= 32)
+        int row = wv, col = lane;
+        bool mine = true;
+        if constexpr (W < 64) {
+            const int q = wv * 60 + lane - 2;
+            mine = lane >= 2 && lane < 62 && q < TY * W;
+            row = min(max(q, 0), TY * W - 1) / W;
+            col = min(max(q, 0), TY * W - 1) % W;
+        }
+        const int gx = x0 + col - 2, gy = y0 + row;
         const int cx = wrapi(gx, N);
-        const bool own = lane >= 2 && lane < 2 + TX && gx < N && gy < N;
-        auto row_off = [&](int y) { return 4u * ((unsigned)wrapi(y, N) * (unsigned)N + (unsigned)cx); };
-        const unsigned off = row_off(gy);
+        const bool own = mine && col >= 2 && col < 2 + TX && gx < N && gy < N;
+        auto row_off = [&](int y, int c) { return 4u * ((unsigned)wrapi(y, N) * (unsigned)N + (unsigned)c); };
+        const unsigned off = row_off(gy, cx);
         // Apron rows: field `part` (phi, P_x, P_y, P_z) at the row next to the
-        // tile (inner: -1 or NW) or beyond it (-2 or NW+1), side 0 below and 1
+        // tile (inner: -1 or TY) or beyond it (-2 or TY+1), side 0 below and 1
         // above.  Waves 0..7 stage an inner row and compute its intermediates;
         // the outer rows go to the same waves (8 rows) or to waves 8..15, and
         // with them v_x, v_y, v_z of the inner rows.
         const int part = (wv & 7) >> 1, side = wv & 1;
         const bool inner = wv < 8;
         const bool vrow = part < 3 && (NW == 8 || !inner);
-        const int ri = side ? NW : -1, ro = side ? NW + 1 : -2;
+        const int ri = side ? TY : -1, ro = side ? TY + 1 : -2;
         const int r0 = inner ? ri : ro;  // first staged row; the second is ro
-        const unsigned off0 = row_off(y0 + r0), off1 = row_off(y0 + ro), offv = row_off(y0 + ri);
+        const int ac = W == 64 ? cx : wrapi(x0 + min(lane, W - 1) - 2, N);
+        const unsigned off0 = row_off(y0 + r0, ac), off1 = row_off(y0 + ro, ac), offv = row_off(y0 + ri, ac);
         const gptr<const float> gp = part == 0 ? gin[0] : part == 1 ? gin[1] : part == 2 ? gin[2] : gin[3];
         const gptr<const float> gpv = part == 0 ? gv[0] : part == 1 ? gv[1] : gv[2];
 
-        // record indices: row q of a field at (q - first row)*64 + lane
-        const int lp = (wv + 2) * 64 + lane;
-        const int lv = (wv + 1) * 64 + lane;
-        const int l0 = (part * HP + r0 + 2) * 64 + lane, l1 = (part * HP + ro + 2) * 64 + lane;
-        const int lvr = (part * HV + ri + 1) * 64 + lane;
-        const int lir = (ri + 1) * 64 + lane;
+        // record indices: column c of row q of a field at (q - first row) W + c.
+        // lp, lv: the own cell's, which the rows above and below are read from;
+        // wp, wv_: where its records go
+        constexpr int LP = (TY + 4) * W;  // the first record of no position, of phi and P
+        const int lp = (row + 2) * W + col, lv = lp - W;
+        const int wp = mine ? lp : LP + lane, wv_ = wp - W;
+        const int la = W == 64 || lane < W ? lane : -1;
+        const int l0 = part * FP + (la < 0 ? LP + lane : (r0 + 2) * W + la);
+        const int l1 = part * FP + (la < 0 ? LP + lane : (ro + 2) * W + la);
+        const int lvr = part * FV + (la < 0 ? LP - W + lane : (ri + 1) * W + la);
+        const int lir = la < 0 ? LP - W + lane : (ri + 1) * W + la;
+        const int lri = part * FP + (r0 + 2) * W + min(lane, W - 1);  // the staged inner row, to read beside it
 
         auto put_i = [&](fvec4* y, int b, int i, const IRow& o) {
-            y[b * HV * 64 + i] = fvec4{o.U, o.W, o.B, o.pm};
+            y[b * FV + i] = fvec4{o.U, o.W, o.B, o.pm};
             ((float*)(y + IM + i))[b] = o.m;
         };
         auto put_m = [&](fvec4* y, int i, float pm, float m) {
@@ -268,14 +297,17 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void k_rhs(const Drop* __restrict_
         auto body = [&](auto ph_, int zm) {
             constexpr int S0 = decltype(ph_)::value, S1 = (S0 + 1) % 3, S2 = (S0 + 2) % 3;
             // ---- a: y stage of v of plane zm-1 (records in Y), which ends its
-            // update terms; z and x stages of phi, P of plane zm
-            {
+            // update terms; z and x stages of phi, P of plane zm.  The 8-wave
+            // kernel, whose chunks are shallow, leaves v out where the plane
+            // is not stored (32^3 10.9 -> 10.4 us); with 16 waves the branch
+            // costs 16 spilled registers.
+            if (NW == 16 || zm > zb) {
                 const float mulc = co.mu * lc;
                 const float vx = vf[0][S0] * s, vy = vf[1][S0] * s, vz = vf[2][S0] * s;
 #pragma unroll
                 for (int b = 0; b < 3; ++b) {
-                    const fvec4* q = by + b * HV * 64 + lv;
-                    const Der d = yder(xv[b], q[-64], q[64]);
+                    const fvec4* q = by + b * FV + lv;
+                    const Der d = yder(xv[b], q[-W], q[W]);
                     const float adv = fma_(vx, d.dx, fma_(vy, d.dy, vz * d.dz));
                     nx[S0][b] = fma_(co.Dt, fma_(mulc, d.l, nx[S0][b]) - adv, vf[b][S0]);
                     pin(nx[S0][b]);
@@ -289,7 +321,7 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void k_rhs(const Drop* __restrict_
             for (int k = 0; k < 4; ++k) {
                 xp[k] = xrow(f[k][S0], f[k][S1], f[k][S2]);
                 pin(xp[k].O);
-                bx[k * HP * 64 + lp] = xp[k].record();
+                bx[k * FP + wp] = xp[k].record();
                 __builtin_amdgcn_sched_barrier(0);
             }
             XRow xi = xrow(tf[0][S0], tf[0][S1], tf[0][S2]);
@@ -312,10 +344,10 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void k_rhs(const Drop* __restrict_
                 float w0, w1, w2, q1, an[3] = {0.f, 0.f, 0.f};
                 {
                     const fvec4* q = bx + lp;
-                    const Der d = yder(xp[0], q[-64], q[64]);
+                    const Der d = yder(xp[0], q[-W], q[W]);
                     m0 = mu0_of(ph, d.l, co.kPhi * lc, co.aPhi2);
                     pm0 = xpair(m0);
-                    put_m(by, lv, pm0, m0);
+                    put_m(by, wv_, pm0, m0);
                     const float P0 = f[1][S1], P1 = f[2][S1], P2 = f[3][S1];
                     const float v0 = vf[0][S1], v1 = vf[1][S1], v2 = vf[2][S1];
                     const float pp = fma_(P0, P0, fma_(P1, P1, P2 * P2));
@@ -346,19 +378,19 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void k_rhs(const Drop* __restrict_
                 const float phs = ph * s, la = co.La2 * lc;
 #pragma unroll
                 for (int b = 0; b < 3; ++b) {
-                    const fvec4* q = bx + (1 + b) * HP * 64 + lp;
-                    const Der d = yder(xp[1 + b], q[-64], q[64]);
+                    const fvec4* q = bx + (1 + b) * FP + lp;
+                    const Der d = yder(xp[1 + b], q[-W], q[W]);
                     const float Pb = f[1 + b][S1];
                     const float dt = fma_(q1, Pb, fma_(w0, d.dx, fma_(w1, d.dy, w2 * d.dz))) + an[b];
                     nx[S1][3 + b] = fma_(-co.Dt, dt, Pb);
                     pin(nx[S1][3 + b]);
                     im[b] = irow(phs * d.dx, phs * d.dy, phs * d.dz, fma_(la, d.l, ph * Pb));
-                    put_i(by, b, lv, im[b]);
+                    put_i(by, b, wv_, im[b]);
                     __builtin_amdgcn_sched_barrier(0);
                 }
             }
             if (NW == 8 || inner) {
-                const Der d = yder(xi, bx[l0 - 64], bx[l0 + 64]);
+                const Der d = yder(xi, bx[lri - W], bx[lri + W]);
                 if (part == 0) {
                     const float m = mu0_of(phr, d.l, co.kPhi * lc, co.aPhi2);
                     put_m(by, lir, xpair(m), m);
@@ -374,11 +406,11 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void k_rhs(const Drop* __restrict_
             // zm+1; store plane zm-1; z and x stages of v of plane zm
             __builtin_amdgcn_sched_barrier(0);
             {
-                const fvec4 mm = by[IM + lv - 64], mp = by[IM + lv + 64];
+                const fvec4 mm = by[IM + lv - W], mp = by[IM + lv + W];
 #pragma unroll
                 for (int b = 0; b < 3; ++b) {
-                    const fvec4* q = by + b * HV * 64 + lv;
-                    const fvec4 im_ = q[-64], ip_ = q[64];
+                    const fvec4* q = by + b * FV + lv;
+                    const fvec4 im_ = q[-W], ip_ = q[W];
                     const IRow& o = im[b];
                     const float A = fma_(4.f, o.X, ip_.x + im_.y);
                     const float B = fma_(4.f, o.B, im_.z + ip_.z);
@@ -395,7 +427,7 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void k_rhs(const Drop* __restrict_
                     __builtin_amdgcn_sched_barrier(0);
                 }
                 const float* const q = (const float*)(by + IP) + lv;
-                const float E = fma_(8.f, m0, q[-64] + q[64]);
+                const float E = fma_(8.f, m0, q[-W] + q[W]);
                 const float F = fma_(-7.f, m0, (mm.w + mp.w) + pm0);
                 aL0[S0] += E;
                 aL0[S1] = fma_(8.f, F, aL0[S1]);
@@ -415,14 +447,16 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void k_rhs(const Drop* __restrict_
                 }
             }
             __builtin_amdgcn_sched_barrier(0);
+            if (NW == 16 || (zm >= zb && zm < ze)) {
 #pragma unroll
-            for (int b = 0; b < 3; ++b) {
-                xv[b] = xrow(vf[b][S0], vf[b][S1], vf[b][S2]);
-                pin(xv[b].O);
-                bx[b * HV * 64 + lv] = xv[b].record();
-                __builtin_amdgcn_sched_barrier(0);
+                for (int b = 0; b < 3; ++b) {
+                    xv[b] = xrow(vf[b][S0], vf[b][S1], vf[b][S2]);
+                    pin(xv[b].O);
+                    bx[b * FV + wv_] = xv[b].record();
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                if (vrow) bx[lvr] = xrow(tv[S0], tv[S1], tv[S2]).record();
             }
-            if (vrow) bx[lvr] = xrow(tv[S0], tv[S1], tv[S2]).record();
             load_v(S0, min(zm + 2, ze));
             __syncthreads();
             fvec4* const t = bx;
@@ -442,13 +476,13 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void k_rhs(const Drop* __restrict_
 }
 
 // ---------------------------------------------------------------------------
-// Tile variants: the nominal tile a box has to hold, and the rows of the
-// kernel that runs it.
+// Tile variants: the nominal tile a box has to hold, and the waves and records
+// per row of the kernel that runs it.
 struct RhsVar {
-    int tx, ty, rows;
+    int tx, ty, nw, w;
 };
 static const RhsVar kRhsVars[RHS_NVARIANTS] = {
-    {32, 8, 8}, {16, 16, 16}, {64, 4, 8}, {16, 8, 8}, {32, 8, 8}, {32, 16, 16}, {64, 8, 8},
+    {32, 8, 8, 64}, {16, 16, 16, 64}, {64, 4, 8, 64}, {16, 8, 8, 64}, {32, 8, 8, 64}, {32, 16, 16, 36}, {64, 8, 8, 64},
 };
 
 hipError_t launch_rhs(int variant, const Drop* drops, const Work* work, const int* nwork_p, int parity, int kstep,
@@ -456,12 +490,23 @@ hipError_t launch_rhs(int variant, const Drop* drops, const Work* work, const in
 {
     if (grid <= 0) return hipSuccess;
     if (variant < 0 || variant >= RHS_NVARIANTS) return hipErrorInvalidValue;
-    if (kRhsVars[variant].rows == 8)
-        return launch_kernel(k_rhs<8>, dim3(grid), dim3(512), st, drops, work, nwork_p, parity, kstep);
-    return launch_kernel(k_rhs<16>, dim3(grid), dim3(1024), st, drops, work, nwork_p, parity, kstep);
+    const RhsVar& v = kRhsVars[variant];
+    if (v.nw == 8)
+        return launch_kernel(k_rhs<8, 64>, dim3(grid), dim3(512), st, drops, work, nwork_p, parity, kstep);
+    if (v.w == 36)
+        return launch_kernel(k_rhs<16, 36>, dim3(grid), dim3(1024), st, drops, work, nwork_p, parity, kstep);
+    return launch_kernel(k_rhs<16, 64>, dim3(grid), dim3(1024), st, drops, work, nwork_p, parity, kstep);
 }
 
-int rhs_rows(int variant) { return variant >= 0 && variant < RHS_NVARIANTS ? kRhsVars[variant].rows : 0; }
+int rhs_rows(int variant)
+{
+    return variant >= 0 && variant < RHS_NVARIANTS ? rhs_tile_rows(kRhsVars[variant].nw, kRhsVars[variant].w) : 0;
+}
+
+int rhs_cols(int variant, int N)
+{
+    return variant >= 0 && variant < RHS_NVARIANTS ? rhs_tiles_x(N, kRhsVars[variant].w) : 0;
+}
 
 bool rhs_fits(int variant, int N)
 {

@@ -106,7 +106,7 @@ static int default_rhs_variant(int) { return RHS_16x16; }
 static int corr_tiles(int N) { return ((N + kCorrTX - 1) / kCorrTX) * ((N + kCorrTY - 1) / kCorrTY); }
 
 // K_rhs work items of one z-range.
-static int rhs_tiles(int variant, int N) { return rhs_tiles_x(N) * ((N + rhs_rows(variant) - 1) / rhs_rows(variant)); }
+static int rhs_tiles(int variant, int N) { return rhs_cols(variant, N) * ((N + rhs_rows(variant) - 1) / rhs_rows(variant)); }
 
 struct Slot {
     bool used = false;
@@ -664,7 +664,7 @@ struct Engine {
     // a size are chosen for that droplet alone, with enough z-chunks to fill
     // the device; each chunk computes two more planes than it stores.  A batch
     // that fills the device by itself runs every droplet's K_rhs with one tile
-    // (the batch entry of the tuning table; by default 16 rows) and chunks of
+    // (the batch entry of the tuning table) and chunks of
     // at least batch_rhs_tz planes, which cuts the share of those planes and
     // gives items of nearly equal cost.  It applies when at least two droplets
     // are active, none asks for a tile, every one fits the tile, and the items
@@ -776,7 +776,7 @@ struct Engine {
     // that the batch runs several rounds of shallow chunks (six droplets of
     // 32^3 to 64^3: 62 us in K_rhs); instead the tile and one depth with the
     // least predicted time (the same six: 36 us).  An iteration takes 3.6 us
-    // with 16 rows and 2.2 with 8, and a chunk about 3 more than it stores;
+    // with 16 waves and 2.2 with 8, and a chunk about 3 more than it stores;
     // K_div runs two groups per CU, K_corr four.
     Layout layout() const
     {
@@ -803,9 +803,12 @@ struct Engine {
             return l;
         }
         double best = 0.0;
-        for (int v : {(int)RHS_16x16, (int)RHS_16x8}) {
-            if (asked && rhs_rows(v) != rhs_rows(l.variant)) continue;
-            const double unit = rhs_rows(v) == 16 ? 3.6 : 2.2;
+        for (int v : {(int)RHS_16x16, (int)RHS_32x16, (int)RHS_16x8}) {
+            // the 32 x 26 tile only where a droplet asks for it: 192^3 + 128^3 +
+            // 96^3 + 64^3 take 633 us a step with it, 621 without, and the
+            // 64-droplet sweep 1175 and 1135
+            if (asked ? rhs_rows(v) != rhs_rows(l.variant) : v == RHS_32x16) continue;
+            const double unit = v == RHS_16x8 ? 2.2 : 3.6;
             for (int d = 1; d <= N; ++d) {
                 const double t = unit * chunk_time(d, 3.0, cus, [&](int n) { return rhs_tiles(v, n); });
                 if (l.rhs_tz && t >= best) continue;
@@ -862,7 +865,7 @@ struct Engine {
             for (int k = 0; k < nzr; ++k) {
                 const int zb = k * N / nzr, ze = (k + 1) * N / nzr;
                 for (int by = 0; by < (N + ty - 1) / ty; ++by)
-                    for (int bx = 0; bx < rhs_tiles_x(N); ++bx)
+                    for (int bx = 0; bx < rhs_cols(rhs_active, N); ++bx)
                         w[T_RHS].push_back(Work{si, bx, by, zb | (ze << 16)});
             }
             // divergence: the droplet's tuned z-chunks are its reduction blocks

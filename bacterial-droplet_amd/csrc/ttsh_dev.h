@@ -102,11 +102,12 @@ struct Work {
     int d, a, b, c;
 };
 
-// Width of K_rhs's tiles for a box of N: a wave holds at most 60 cells of a
-// row beside the 2-cell apron, and the row is cut into equal parts.
-constexpr int kRhsMaxTX = 60;
-__host__ __device__ constexpr int rhs_tiles_x(int N) { return (N + kRhsMaxTX - 1) / kRhsMaxTX; }
-__host__ __device__ constexpr int rhs_tile_width(int N) { return (N + rhs_tiles_x(N) - 1) / rhs_tiles_x(N); }
+// K_rhs's tiles for a box of N.  A tile row has at most W records, four of
+// which are apron; the box's rows are cut into equal parts.  A tile has one
+// row per wave (W = 64), or as many as fit the waves' 60 positions each.
+__host__ __device__ constexpr int rhs_tiles_x(int N, int W) { return (N + W - 5) / (W - 4); }
+__host__ __device__ constexpr int rhs_tile_width(int N, int W) { return (N + rhs_tiles_x(N, W) - 1) / rhs_tiles_x(N, W); }
+__host__ __device__ constexpr int rhs_tile_rows(int NW, int W) { return W == 64 ? NW : NW * 60 / W; }
 
 // Tiles of the divergence: a wave is a row whose 64 lanes
 // include one apron cell on each side, a work-group 16 rows of which the

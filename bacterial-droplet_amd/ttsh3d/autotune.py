@@ -1,14 +1,14 @@
 """Autotuner for the TTSH3D step kernels.
 
-For each grid size N it times, with HIP events through ttsh_profile, the two
-K_rhs kernels (16 and 8 rows per work-group) at several z-depths, and several
+For each grid size N it times, with HIP events through ttsh_profile, the three
+K_rhs kernels (tiles of 60 x 16, 60 x 8 and 32 x 26) at several z-depths, and several
 z-depths of the divergence stencil, on a droplet of that size; then
 writes the fastest choices as the tuning table libttsh3d.so reads (tuned.txt
 beside the library, lines "N rhs_variant rhs_tz proj_tz").
 
 With --batch it tunes the layout of a batch that fills the device instead:
 on the 64-droplet sweep mix (L in {48, 64, 96, 128}) as one graph batch, it
-times whole batch steps for both K_rhs kernels, minimum
+times whole batch steps for each K_rhs kernel that fits all sizes, minimum
 K_rhs z-depth and divergence/corrector z-depth, through the table's "batch"
 line (re-read between candidates; the batch is laid out again at its next
 step), and keeps the fastest.  The FFT passes' lines per work-group are
@@ -29,8 +29,9 @@ from . import F64, TTSHError, Batch, Simulation, default_params, init_droplet, l
 
 # nominal tile of each variant: the box has to hold it
 RHS_VARIANTS = {0: (32, 8), 1: (16, 16), 2: (64, 4), 3: (16, 8), 4: (32, 8), 5: (32, 16), 6: (64, 8)}
-# one variant of each kernel, with the smallest nominal tile: 16 and 8 rows
-TUNED_VARIANTS = (1, 3)
+# one variant of each kernel, with the smallest nominal tile: tiles of up to
+# 60 x 16, 60 x 8 and 32 x 26 cells
+TUNED_VARIANTS = (1, 3, 5)
 # z-depths: the engine splits z into ceil(N/tz) near-equal chunks; a chunk
 # computes two planes more than it stores, and the number of chunks times the
 # tiles of a plane should come just below a multiple of the CUs
@@ -60,6 +61,8 @@ def tune_size(N: int, steps: int = 30, log=print):
             nz.add((N + tz - 1) // tz)
             depths.append(tz)
     for var in TUNED_VARIANTS:
+        if N < max(RHS_VARIANTS[var]) + 2:
+            continue
         for tz in depths:
             try:
                 k = _time(default_params(rhs_variant=var, rhs_tz=tz, corr_tz=8, **base), state, steps)

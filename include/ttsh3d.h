@@ -63,16 +63,18 @@ typedef struct ttsh_params {
     int32_t faithful_halo; /* 1 (default): div(v*), div(P*) read the previous step's
                               v*, P* across the periodic boundary, as the reference's
                               stale halo does (TTSH3D.cu:366-371,405-407,665-667) */
-    int32_t rhs_variant;   /* K_rhs tile: -1 = tuned default, else 0..6 (1 and 5
-                              run 16 rows of cells per work-group, the others 8);
-                              results do not depend on it */
+    int32_t rhs_variant;   /* K_rhs tile: -1 = tuned default, else 0..6 (1 runs
+                              tiles of up to 60 x 16 cells, 5 of up to 32 x 26,
+                              the others of up to 60 x 8); results do not depend
+                              on it */
     int32_t rhs_tz;        /* K_rhs z-range per work item, 0 = tuned default */
     int32_t corr_tz;       /* divergence and corrector z-range per work item,
                               0 = tuned default.  With the defaults, a batch
                               whose droplets fill the device runs K_rhs with
-                              16 rows and ranges of at least 32, and the
-                              divergence and corrector with ranges of about 32;
-                              results do not change. */
+                              the tile and minimum range of the tuning table's
+                              batch line, and other batches a tile and ranges
+                              chosen for all droplets together; results do not
+                              change. */
 } ttsh_params;
 
 typedef struct ttsh_sim ttsh_sim;
@@ -341,7 +343,7 @@ int ttsh_tuning_lookup(int N, int* rhs_variant, int* rhs_tz, int* corr_tz);
 /* New: the layout of a batch whose droplets fill the device (table line
  * "batch rhs_variant rhs_tz corr_tz"): the K_rhs tile every droplet then
  * runs, the minimum K_rhs z-range per work item and the divergence and
- * corrector z-range.  Without the line the engine uses 16 rows, 32 and 32.  A
+ * corrector z-range.  Without the line the engine uses variant 1, 32 and 32.  A
  * reload applies to running batches at their next step call. */
 int ttsh_tuning_lookup_batch(int* rhs_variant, int* rhs_tz, int* corr_tz);
 

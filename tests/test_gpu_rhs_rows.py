@@ -36,7 +36,7 @@ def test_rough_fields(ttsh, oracle_mod, N, A):
     o.step(1)
     want = [o.get_state()[0], o.aux("pstar"), o.aux("vstar")]
     first = None
-    for variant, tz in ((1, 7), (3, 7), (1, 1), (3, N), (1, N), (3, 1)):
+    for variant, tz in ((1, 7), (3, 7), (1, 1), (3, N), (1, N), (3, 1)) + (((5, 7), (5, 1), (5, N)) if N >= 34 else ()):
         q = p.copy()
         q.rhs_variant, q.rhs_tz = variant, tz
         with ttsh.Simulation(q) as sim:
