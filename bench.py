@@ -54,8 +54,8 @@ sys.path.insert(0, os.path.join(ROOT, "bacterial-droplet_amd"))
 # Algorithmic FP32 field traffic per cell of each kernel kind (reads + writes):
 # K_rhs reads phi, P, v and writes phi', v*, P*; K_div reads v*, P* and writes
 # the complex s; each FFT pass reads and writes the complex buffer (K_fft_xy
-# and K_fft_xy_inv are the x passes, or in large batches the fused x+y
-# passes); K_corr reads p (complex), v*, P* and writes v, P.
+# and K_fft_xy_inv are the x passes; up to 128^3 one y-z plane kernel, timed
+# under K_fft_z_poisson, does the work of the three between); K_corr reads p (complex), v*, P* and writes v, P.
 ALG_BYTES = {"K_rhs": 56, "K_div": 32, "K_fft_xy": 16, "K_fft_y": 16, "K_fft_z_poisson": 16,
              "K_fft_y_inv": 16, "K_fft_xy_inv": 16, "K_corr": 56}
 STEP_BYTES = sum(ALG_BYTES.values())  # bytes per cell-step this design moves (five FFT passes)
