@@ -306,9 +306,12 @@ struct Xch {
 };
 
 // -1/(k^2 N^3) at integer wavenumbers (fftfreq order), k2[0] = 1.  With
-// k^2 = k2s m2, m2 a whole number, it is pk0/m2; the reciprocal of m2 is the
-// hardware's (one unit in the last place) with one Newton step, so within one
-// unit, at a third of the instructions of an IEEE division.
+// k^2 = k2s m2, m2 a whole number, it is pk0/m2: the hardware's reciprocal of
+// m2 (one unit in the last place), one Newton step, and one step on the
+// quotient's remainder, which rounds it as a division does (all m2 of all
+// sizes, and reciprocals one unit off either way, give the rounded quotient)
+// at half the instructions of an IEEE division, whose scaling and special
+// cases a whole m2 does not need.
 __device__ __forceinline__ float poisson_factor(const Coef& co, int N, int kx, int ky, int kz)
 {
     const int mx = kx < N / 2 ? kx : kx - N;
@@ -318,7 +321,8 @@ __device__ __forceinline__ float poisson_factor(const Coef& co, int N, int kx, i
     const float x = (float)m2;
     float r = __builtin_amdgcn_rcpf(x);
     r = __builtin_fmaf(__builtin_fmaf(-x, r, 1.f), r, r);
-    return m2 == 0 ? -co.inv_n3 : co.pk0 * r;
+    const float q = co.pk0 * r;
+    return m2 == 0 ? -co.inv_n3 : __builtin_fmaf(__builtin_fmaf(-x, q, co.pk0), r, q);
 }
 
 // Work item (d, a, b): droplet d; the pass's lines are the L consecutive
