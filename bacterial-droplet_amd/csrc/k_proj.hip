@@ -551,7 +551,8 @@ hipError_t launch_fill_edges(const float* const vs[3], const float* const ps[3],
 }
 
 // Field blockIdx.y of a list, n elements each (floats, or groups of four where
-// every address is a multiple of 16 bytes).  One launch for the 13 fields of a
+// every address is a multiple of 16 bytes), in memory that the device reaches,
+// no destination overlapping another.  One launch for the 13 fields of a
 // state: 13 copies of the runtime cost a call of one 32^3 step 70 us on each
 // side of the step, this 5.
 template <typename T>

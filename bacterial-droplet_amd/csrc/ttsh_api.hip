@@ -20,9 +20,11 @@
 #include <algorithm>
 #include <cmath>
 #include <condition_variable>
+#include <cstdint>
 #include <cstdio>
 #include <cstring>
 #include <deque>
+#include <initializer_list>
 #include <map>
 #include <mutex>
 #include <string>
@@ -1252,10 +1254,24 @@ struct Engine {
         return TTSH_OK;
     }
 
-    // State in from device memory (FP32, same layouts as upload_state): phi,
-    // P, v and the previous step's predictors vsp, psp, copied on the
-    // engine's stream.
-    int upload_device(int si, const float* phi, const float* P, const float* v, const float* vsp, const float* psp)
+    // Copies a list of fields on st: one kernel, or the runtime's copies, which
+    // also take memory that a kernel does not reach.
+    int copy_fields(const FieldList& f, size_t n, bool kernel)
+    {
+        if (kernel) {
+            HIPCHK(launch_copy_fields(f, n, st));
+            return TTSH_OK;
+        }
+        for (int k = 0; k < f.count; ++k)
+            HIPCHK(hipMemcpyAsync(f.dst[k], f.src[k], n * sizeof(float), hipMemcpyDeviceToDevice, st));
+        return TTSH_OK;
+    }
+
+    // State in from the caller's memory (FP32, same layouts as upload_state):
+    // phi, P, v and the previous step's predictors vsp, psp, copied on the
+    // engine's stream; kernel: see copy_fields and caller_fields_on_device.
+    int upload_device(int si, const float* phi, const float* P, const float* v, const float* vsp, const float* psp,
+                      bool kernel)
     {
         Slot& s = slots[si];
         HIPCHK(hipSetDevice(device));
@@ -1270,7 +1286,7 @@ struct Engine {
             f.add(vsp + a * n, s.drop.vs[q ^ 1][a]);
             f.add(psp + a * n, s.drop.ps[q ^ 1][a]);
         }
-        HIPCHK(launch_copy_fields(f, n, st));
+        if (int rc = copy_fields(f, n, kernel)) return rc;
         const float* vs[3] = {s.drop.vs[q ^ 1][0], s.drop.vs[q ^ 1][1], s.drop.vs[q ^ 1][2]};
         const float* ps[3] = {s.drop.ps[q ^ 1][0], s.drop.ps[q ^ 1][1], s.drop.ps[q ^ 1][2]};
         HIPCHK(launch_fill_edges(vs, ps, s.drop.edge, s.drop.eslot[q ^ 1], s.N, st));
@@ -1280,8 +1296,8 @@ struct Engine {
         return TTSH_OK;
     }
 
-    // State out to device memory: phi, P, v and the last step's predictors.
-    int download_device(int si, float* phi, float* P, float* v, float* vs_out, float* ps_out)
+    // State out to the caller's memory: phi, P, v and the last step's predictors.
+    int download_device(int si, float* phi, float* P, float* v, float* vs_out, float* ps_out, bool kernel)
     {
         Slot& s = slots[si];
         HIPCHK(hipSetDevice(device));
@@ -1295,8 +1311,7 @@ struct Engine {
             f.add(s.drop.vs[last][a], vs_out + a * n);
             f.add(s.drop.ps[last][a], ps_out + a * n);
         }
-        HIPCHK(launch_copy_fields(f, n, st));
-        return TTSH_OK;
+        return copy_fields(f, n, kernel);
     }
 
     int download(int si, int dtype, void* phi, void* P, void* v)
@@ -1639,6 +1654,37 @@ int scratch_address(int dev, void** out)
     }
     *out = g_scratch_ptr[dev];
     return TTSH_OK;
+}
+
+struct CallerField {
+    const float* p;
+    size_t n;  // floats
+};
+
+// Whether one kernel may read and write the caller's arrays: each lies wholly
+// in one allocation of device memory of `dev`, on a float boundary, and no two
+// overlap (the kernel writes them in no order).  Anything else, host memory
+// and peers' memory among it, goes through the runtime's copies, which know
+// how to reach it or fail.
+bool caller_fields_on_device(std::initializer_list<CallerField> fields, int dev)
+{
+    for (const CallerField& f : fields) {
+        const uintptr_t b = (uintptr_t)f.p, e = b + f.n * sizeof(float);
+        hipPointerAttribute_t at{};
+        hipDeviceptr_t base = nullptr;
+        size_t size = 0;
+        if (hipPointerGetAttributes(&at, f.p) != hipSuccess || at.type != hipMemoryTypeDevice || at.device != dev ||
+            hipMemGetAddressRange(&base, &size, (hipDeviceptr_t)f.p) != hipSuccess) {
+            (void)hipGetLastError();  // not a pointer the runtime knows: not an error of this call
+            return false;
+        }
+        if (b % sizeof(float) || b < (uintptr_t)base || e > (uintptr_t)base + size) return false;
+        for (const CallerField& g : fields) {
+            const uintptr_t gb = (uintptr_t)g.p, ge = gb + g.n * sizeof(float);
+            if (&g != &f && b < ge && gb < e) return false;
+        }
+    }
+    return true;
 }
 }  // namespace
 
@@ -1985,9 +2031,12 @@ int ttsh_step_noalloc(const ttsh_params* p, float* phi, float* P, float* v, floa
     Engine e;
     rc = e.init_external(dev, static_cast<hipStream_t>(stream), base, kScratchBytes);
     if (!rc) rc = e.alloc_slot(0, *p);
-    if (!rc) rc = e.upload_device(0, phi, P, v, vstar_prev, pstar_prev);
+    const size_t n1 = (size_t)p->Nx * p->Nx * p->Nx, n3 = 3 * n1;
+    const bool kernel =
+        caller_fields_on_device({{phi, n1}, {P, n3}, {v, n3}, {vstar_prev, n3}, {pstar_prev, n3}}, dev);
+    if (!rc) rc = e.upload_device(0, phi, P, v, vstar_prev, pstar_prev, kernel);
     if (!rc) rc = e.step(n, false);
-    if (!rc) rc = e.download_device(0, phi, P, v, vstar_prev, pstar_prev);
+    if (!rc) rc = e.download_device(0, phi, P, v, vstar_prev, pstar_prev, kernel);
     if (!rc) HIPCHK(hipStreamSynchronize(e.st));
     return rc;
 }

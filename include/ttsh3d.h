@@ -312,7 +312,9 @@ int ttsh_batch_ready(ttsh_batch* b, int slot, int* ready);
  * vstar_prev, pstar_prev (3*N^3 each) in: the predictors the first step's
  * stale-halo divergence reads (the reference's initial v*, P*; pass copies
  * of v and P for a fresh state), out: the last step's predictors, so
- * consecutive calls continue one run exactly.  n steps as ttsh_step with
+ * consecutive calls continue one run exactly.  Arrays in other memory that
+ * hipMemcpyAsync takes (the host's, another GPU's) work too, with slower
+ * copies.  n steps as ttsh_step with
  * the same kernels, tiles and results; stream is a hipStream_t (NULL: the
  * null stream); the call returns when the steps are done.
  * Every other buffer of the step lives in one device array of 32 MiB per

@@ -50,3 +50,63 @@ def test_offsets(ttsh, N, offset):
     for (_, got), b in zip(held, want):
         assert np.array_equal(got[begin:begin + b.size], b.reshape(-1))
         assert (got[:begin] == 7.0).all() and (got[begin + b.size:] == 7.0).all()
+
+
+@pytest.mark.parametrize("memory", ["pageable", "pinned", "phi pageable", "v* is v"])
+def test_memory_that_the_copy_kernel_may_not_touch(ttsh, memory):
+    """Host arrays, and arrays of which two are the same memory, take the
+    runtime's copies: a kernel would fault on the first and write the second in
+    no order.  The state equals ttsh_step's bitwise; of one array given twice
+    the later copy, the predictor, is what remains."""
+    print(f"[copy_fields {memory}]", flush=True)
+    ttsh.lib()
+    hip = ctypes.CDLL("libamdhip64.so.7")
+    hip.hipMalloc.argtypes = [ctypes.POINTER(ctypes.c_void_p), ctypes.c_size_t]
+    hip.hipHostMalloc.argtypes = [ctypes.POINTER(ctypes.c_void_p), ctypes.c_size_t, ctypes.c_uint]
+    hip.hipFree.argtypes = hip.hipHostFree.argtypes = [ctypes.c_void_p]
+    hip.hipMemcpy.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_int]
+    N = 36
+    rng = np.random.default_rng(5)
+    r = lambda k: rng.uniform(-1, 1, (k, N, N, N)).astype(np.float32)
+    phi, P, v = 0.5 + 0.4 * r(1)[0], r(3), 0.1 * r(3)
+    p = ttsh.default_params(N=N, dt0=0.005)
+    begin = [phi, P, v, v.copy(), P.copy()]
+    out = [a.copy() for a in begin]
+    ptrs, frees = [], []
+    try:
+        for k, a in enumerate(out):
+            ptr = ctypes.c_void_p()
+            if memory == "pageable" or (memory == "phi pageable" and k == 0):
+                ptr.value = a.ctypes.data
+            elif memory == "pinned":
+                assert hip.hipHostMalloc(ctypes.byref(ptr), a.nbytes, 0) == 0
+                frees.append((hip.hipHostFree, ptr))
+                ctypes.memmove(ptr, a.ctypes.data, a.nbytes)
+                out[k] = np.ctypeslib.as_array((ctypes.c_float * a.size).from_address(ptr.value))
+            else:
+                assert hip.hipMalloc(ctypes.byref(ptr), a.nbytes) == 0
+                frees.append((hip.hipFree, ptr))
+                assert hip.hipMemcpy(ptr, a.ctypes.data, a.nbytes, H2D) == 0
+                out[k] = None
+            ptrs.append(ptr)
+        if memory == "v* is v":
+            ptrs[3] = ptrs[2]
+        assert hip.hipDeviceSynchronize() == 0
+        ttsh.step_noalloc(p, *(q.value for q in ptrs), 3)
+        got = []
+        for q, a, b in zip(ptrs, out, begin):
+            if a is None:
+                a = np.empty(b.size, np.float32)
+                assert hip.hipMemcpy(a.ctypes.data, q, a.nbytes, D2H) == 0
+            got.append(a.reshape(-1).copy())
+    finally:
+        for free, q in frees:
+            free(q)
+    with ttsh.Simulation(p) as s:
+        s.set_state(*begin, dtype=ttsh.F32)
+        s.step(3)
+        want = [x.reshape(-1) for x in (*s.get_state(), s.aux("vstar"), s.aux("pstar"))]
+    if memory == "v* is v":
+        want[2] = want[3]
+    for a, b in zip(got, want):
+        assert np.array_equal(a, b)
