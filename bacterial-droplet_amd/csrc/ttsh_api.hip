@@ -1339,12 +1339,8 @@ struct Engine {
         want(s.drop.phi[s.q], phi, 0);
         for (int a = 0; a < 3; ++a) want(s.drop.P[a], P, a * n);
         for (int a = 0; a < 3; ++a) want(s.drop.v[a], v, a * n);
-        if (!external && pieces.size() * n * sizeof(float) >= HostCopier::kMinBytes) {
-            bool started = false;
-            HIPCHK(host_out.copy(pieces, f64, side(), &started));
-            if (started) return TTSH_OK;
-        }
-        std::vector<float> tmp(f64 ? n : 0);
+        if (!external) HIPCHK(host_out.copy(pieces, f64, side()));
+        std::vector<float> tmp(f64 && !pieces.empty() ? n : 0);
         for (const HostPiece& p : pieces) {
             if (!f64) {
                 HIPCHK(hipMemcpy(p.dst, p.src, n * sizeof(float), hipMemcpyDeviceToHost));

@@ -7,7 +7,9 @@
 // thread queues the copies and hands each finished chunk to worker threads,
 // which store it (widened to FP64 if asked) in the destination.  Four workers
 // take 56 GB/s with the page faults, one 16.  State of a 256^3 droplet (470
-// MB) 58 -> 11 ms, 128^3 (59 MB) 7.2 -> 1.7 ms.
+// MB) 58 -> 11 ms, 128^3 (59 MB) 7.2 -> 1.7 ms.  A destination that is pinned
+// already has nothing to gain: 128^3 takes 1.1 ms by hipMemcpy, 1.5 through
+// the ring.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -110,13 +112,17 @@ public:
         }
     }
 
-    // Copies the pieces on stream st and returns when they are in place.
-    // started = false: threads or pinned memory were not to be had and nothing
-    // was copied.
-    hipError_t copy(const std::vector<HostPiece>& pieces, bool f64, hipStream_t st, bool* started)
+    // Takes the pieces that go through the ring out of the list, copies them on
+    // stream st and returns when they are in place.  What stays is the caller's
+    // to copy: FP32 for destinations that are not pageable, less than kMinBytes
+    // altogether, or all if threads or pinned memory were not to be had.
+    hipError_t copy(std::vector<HostPiece>& pieces, bool f64, hipStream_t st)
     {
-        *started = false;
-        if (!events()) return hipSuccess;
+        const auto mine = std::stable_partition(pieces.begin(), pieces.end(),
+                                                [&](const HostPiece& p) { return !f64 && !pageable(p.dst); });
+        size_t bytes = 0;
+        for (auto p = mine; p != pieces.end(); ++p) bytes += p->n * sizeof(float);
+        if (bytes < kMinBytes || !events()) return hipSuccess;
         struct Loan {
             float* p = PinnedRings::get().borrow();
             ~Loan()
@@ -127,10 +133,10 @@ public:
         ring = loan.p;
         if (!ring) return hipSuccess;
         std::vector<HostPiece> chunk;
-        for (const HostPiece& p : pieces)
-            for (size_t o = 0; o < p.n; o += kChunk) {
-                const size_t n = std::min(kChunk, p.n - o);
-                chunk.push_back(HostPiece{p.src + o, static_cast<char*>(p.dst) + o * (f64 ? 8 : 4), n});
+        for (auto p = mine; p != pieces.end(); ++p)
+            for (size_t o = 0; o < p->n; o += kChunk) {
+                const size_t n = std::min(kChunk, p->n - o);
+                chunk.push_back(HostPiece{p->src + o, static_cast<char*>(p->dst) + o * (f64 ? 8 : 4), n});
             }
         head = tail = 0;
         for (bool& b : busy) b = false;
@@ -142,7 +148,7 @@ public:
         } catch (...) {
             if (th.empty()) return hipSuccess;  // with fewer workers it goes on
         }
-        *started = true;
+        pieces.erase(mine, pieces.end());
         hipError_t e = hipSuccess;
         size_t issued = 0;
         for (size_t i = 0; i < chunk.size() && e == hipSuccess; ++i) {
@@ -190,6 +196,14 @@ private:
         void* dst;
         size_t n;
     };
+
+    static bool pageable(const void* p)
+    {
+        hipPointerAttribute_t at{};
+        if (hipPointerGetAttributes(&at, p) == hipSuccess) return at.type == hipMemoryTypeUnregistered;
+        (void)hipGetLastError();  // memory that the runtime does not know
+        return true;
+    }
 
     float* slot(int s) const { return ring + (size_t)s * kChunk; }
 
