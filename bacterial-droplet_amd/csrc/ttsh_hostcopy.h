@@ -28,13 +28,16 @@ struct HostPiece {
     size_t n;
 };
 
-// Rings of pinned chunks, shared by the copiers of a process: at most kIdle
-// are kept while no copy uses them, and none once the last copier is gone.
+// A ring of pinned chunks.
+struct Ring {
+    float* p = nullptr;  // nullptr: no pinned memory to be had
+    size_t n = 0;        // floats
+};
+
+// Rings shared by the copiers of a process: at most kIdle are kept while no copy
+// uses them, the larger ones, and none once the last copier is gone.
 class PinnedRings {
 public:
-    static constexpr size_t kChunk = (size_t)1 << 20;  // floats: 4 MiB
-    static constexpr int kSlots = 8;
-
     static PinnedRings& get()
     {
         static PinnedRings* const r = new PinnedRings();  // never destroyed: copiers may outlive main
@@ -49,43 +52,47 @@ public:
     {
         std::lock_guard<std::mutex> lk(mu);
         if (--copiers > 0) return;
-        for (float* p : idle) (void)hipHostFree(p);
+        for (const Ring& r : idle) (void)hipHostFree(r.p);
         idle.clear();
     }
-    float* borrow()  // nullptr: no pinned memory to be had
+    // A ring of at least n floats.
+    Ring borrow(size_t n)
     {
         {
             std::lock_guard<std::mutex> lk(mu);
-            if (!idle.empty()) {
-                float* const p = idle.back();
-                idle.pop_back();
-                return p;
-            }
+            for (size_t k = 0; k < idle.size(); ++k)
+                if (idle[k].n >= n) {
+                    const Ring r = idle[k];
+                    idle.erase(idle.begin() + (long)k);
+                    return r;
+                }
         }
         void* p = nullptr;
-        if (hipHostMalloc(&p, sizeof(float) * kChunk * kSlots, hipHostMallocPortable) != hipSuccess) {
+        if (hipHostMalloc(&p, sizeof(float) * n, hipHostMallocPortable) != hipSuccess) {
             (void)hipGetLastError();
-            return nullptr;
+            return Ring{};
         }
-        return static_cast<float*>(p);
+        return Ring{static_cast<float*>(p), n};
     }
-    void give(float* p)
+    void give(Ring r)
     {
         {
             std::lock_guard<std::mutex> lk(mu);
             if (idle.size() < kIdle) {
-                idle.push_back(p);
+                idle.push_back(r);
                 return;
             }
+            for (Ring& k : idle)
+                if (k.n < r.n) std::swap(k, r);
         }
-        (void)hipHostFree(p);
+        (void)hipHostFree(r.p);
     }
 
 private:
     static constexpr size_t kIdle = 2;
     PinnedRings() { idle.reserve(kIdle); }
     std::mutex mu;
-    std::vector<float*> idle;
+    std::vector<Ring> idle;
     int copiers = 0;
 };
 
@@ -93,6 +100,13 @@ class HostCopier {
 public:
     // Below this the threads cost more than they save.
     static constexpr size_t kMinBytes = (size_t)8 << 20;
+    // States below kLargeBytes use 4 chunks of 2 MiB, larger ones 8 of 4 MiB.
+    // The first copy through a ring takes the page faults of its host mapping,
+    // about 0.13 ms per MiB.  A first read of a 72^3 or 96^3 state takes 1.2 and
+    // 2.5 ms with the small ring, 1.9 and 4.7 with the large one, later ones
+    // 0.44 and 0.79 against 0.43 and 0.75.  Where a plain copy takes 5 ms and
+    // more (128^3) the large ring's first read costs no more than that.
+    static constexpr size_t kLargeBytes = (size_t)32 << 20;
 
     HostCopier() { PinnedRings::get().join(); }
     HostCopier(const HostCopier&) = delete;
@@ -123,19 +137,21 @@ public:
         size_t bytes = 0;
         for (auto p = mine; p != pieces.end(); ++p) bytes += p->n * sizeof(float);
         if (bytes < kMinBytes || !events()) return hipSuccess;
+        slots = bytes < kLargeBytes ? kSlots / 2 : kSlots;
+        chunk_n = bytes < kLargeBytes ? kChunk / 2 : kChunk;
         struct Loan {
-            float* p = PinnedRings::get().borrow();
+            Ring r;
             ~Loan()
             {
-                if (p) PinnedRings::get().give(p);
+                if (r.p) PinnedRings::get().give(r);
             }
-        } loan;  // outlives the workers and every copy into it
-        ring = loan.p;
+        } loan{PinnedRings::get().borrow(chunk_n * slots)};  // outlives the workers and every copy into it
+        ring = loan.r.p;
         if (!ring) return hipSuccess;
         std::vector<HostPiece> chunk;
         for (auto p = mine; p != pieces.end(); ++p)
-            for (size_t o = 0; o < p->n; o += kChunk) {
-                const size_t n = std::min(kChunk, p->n - o);
+            for (size_t o = 0; o < p->n; o += chunk_n) {
+                const size_t n = std::min(chunk_n, p->n - o);
                 chunk.push_back(HostPiece{p->src + o, static_cast<char*>(p->dst) + o * (f64 ? 8 : 4), n});
             }
         head = tail = 0;
@@ -153,9 +169,9 @@ public:
         size_t issued = 0;
         for (size_t i = 0; i < chunk.size() && e == hipSuccess; ++i) {
             // keep every free slot's copy in flight; chunk i's slot frees up
-            // when the workers have stored chunk i - kSlots
-            while (issued < chunk.size() && issued < i + kSlots && e == hipSuccess) {
-                const int s = (int)(issued % kSlots);
+            // when the workers have stored chunk i - slots
+            while (issued < chunk.size() && issued < i + slots && e == hipSuccess) {
+                const int s = (int)(issued % slots);
                 {
                     std::unique_lock<std::mutex> lk(mu);
                     if (busy[s]) {
@@ -169,12 +185,12 @@ public:
                 ++issued;
             }
             if (e != hipSuccess) break;
-            const int s = (int)(i % kSlots);
+            const int s = (int)(i % slots);
             e = hipEventSynchronize(ev[s]);
             if (e != hipSuccess) break;
             {
                 std::lock_guard<std::mutex> lk(mu);
-                ready[tail++ % kSlots] = Job{s, chunk[i].dst, chunk[i].n};
+                ready[tail++ % slots] = Job{s, chunk[i].dst, chunk[i].n};
             }
             ready_cv.notify_one();
         }
@@ -189,8 +205,8 @@ public:
     }
 
 private:
-    static constexpr size_t kChunk = PinnedRings::kChunk;
-    static constexpr int kSlots = PinnedRings::kSlots, kWorkers = 4;
+    static constexpr size_t kChunk = (size_t)1 << 20;  // floats: 4 MiB
+    static constexpr int kSlots = 8, kWorkers = 4;
     struct Job {
         int slot;
         void* dst;
@@ -205,7 +221,7 @@ private:
         return true;
     }
 
-    float* slot(int s) const { return ring + (size_t)s * kChunk; }
+    float* slot(int s) const { return ring + (size_t)s * chunk_n; }
 
     bool events()
     {
@@ -226,7 +242,7 @@ private:
                 std::unique_lock<std::mutex> lk(mu);
                 ready_cv.wait(lk, [&] { return quit || head != tail; });
                 if (head == tail) return;
-                j = ready[head++ % kSlots];
+                j = ready[head++ % slots];
             }
             const float* s = slot(j.slot);
             if (f64) {
@@ -244,6 +260,7 @@ private:
     }
 
     float* ring = nullptr;
+    size_t slots = kSlots, chunk_n = kChunk;  // of the copy under way
     hipEvent_t ev[kSlots] = {};
     std::mutex mu;
     std::condition_variable ready_cv, free_cv;

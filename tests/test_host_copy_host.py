@@ -13,6 +13,7 @@ CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
 
 STUB = r"""
 #pragma once
+#include <atomic>
 #include <cstddef>
 #include <cstdlib>
 #include <cstring>
@@ -27,7 +28,8 @@ typedef void* hipEvent_t;
 struct hipPointerAttribute_t { hipMemoryType type; int device; };
 inline std::mutex g_mu;
 inline std::map<const char*, size_t> g_pinned;
-inline size_t g_pinned_bytes = 0, g_allocs = 0, g_async = 0;
+inline size_t g_pinned_bytes = 0, g_allocs = 0;
+inline std::atomic<size_t> g_async{0};
 inline bool g_no_memory = false;
 inline hipError_t hipHostMalloc(void** p, size_t n, unsigned)
 {
@@ -94,6 +96,7 @@ int main()
         // pageable: everything through the ring
         auto p = fields(src, n, (char*)a.data(), 4 * n);
         CHECK(hc.copy(p, false, nullptr) == hipSuccess && p.empty() && g_allocs == 1);
+        CHECK(g_pinned_bytes <= (size_t)8 << 20);  // a first read of a small state pins a small ring
         CHECK(std::memcmp(a.data(), src.data(), 28 * n) == 0);
         p = fields(src, n, (char*)b.data(), 8 * n);
         CHECK(hc.copy(p, true, nullptr) == hipSuccess && p.empty() && g_allocs == 1);
@@ -125,6 +128,37 @@ int main()
         (void)hipHostFree(pin);
     }
     CHECK(g_pinned_bytes == 0);  // given back with the last copier
+    {
+        // a large state takes a larger ring, which then serves small ones too
+        HostCopier hc;
+        const size_t m = 2500000;  // 70 MB
+        std::vector<float> big(7 * m), out(7 * m);
+        for (size_t i = 0; i < big.size(); ++i) big[i] = (float)(i % 99991);
+        auto p = fields(src, n, (char*)a.data(), 4 * n);
+        CHECK(hc.copy(p, false, nullptr) == hipSuccess && p.empty());
+        const size_t small = g_pinned_bytes;
+        p = fields(big, m, (char*)out.data(), 4 * m);
+        CHECK(hc.copy(p, false, nullptr) == hipSuccess && p.empty() && big == out);
+        CHECK(g_pinned_bytes > small);
+        const size_t allocs = g_allocs;
+        std::fill(a.begin(), a.end(), 0.f);
+        p = fields(src, n, (char*)a.data(), 4 * n);
+        CHECK(hc.copy(p, false, nullptr) == hipSuccess && p.empty() && a == src && g_allocs == allocs);
+        // three at once; two rings stay, the larger ones
+        HostCopier h3[3];
+        std::vector<float> o3[3];
+        std::vector<std::thread> th;
+        for (int k = 0; k < 3; ++k)
+            th.emplace_back([&, k] {
+                o3[k].resize(7 * m);
+                auto q = fields(big, m, (char*)o3[k].data(), 4 * m);
+                if (h3[k].copy(q, false, nullptr) != hipSuccess || !q.empty()) o3[k].clear();
+            });
+        for (auto& t : th) t.join();
+        for (auto& o : o3) CHECK(o == big);
+        CHECK(g_pinned_bytes <= (size_t)64 << 20);
+    }
+    CHECK(g_pinned_bytes == 0);
     {
         HostCopier hc;
         g_no_memory = true;
