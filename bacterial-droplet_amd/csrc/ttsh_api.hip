@@ -36,6 +36,7 @@
 #include "ttsh_hostcopy.h"
 #include "ttsh_internal.h"
 #include "ttsh_kernels.h"
+#include "ttsh_layout.h"
 
 namespace ttsh {
 
@@ -719,59 +720,6 @@ struct Engine {
         bool deep = false;  // the device-filling batch layout: depths are minima
     };
 
-    // Predicted time of z-chunks of depth d over the active droplets, in
-    // plane iterations of one work-group: `over` iterations of a chunk (planes
-    // beyond its own, loading, launch) come on top of d, `at_once` groups run
-    // together, and a last round that is partly empty counts whole while there
-    // are few rounds.
-    template <typename Tiles>
-    double chunk_time(int d, double over, double at_once, Tiles&& tiles) const
-    {
-        double items = 0.0, deepest = 0.0;
-        for (const Slot& s : slots) {
-            if (!s.used || remaining(s) <= 0) continue;
-            const int nz = (s.N + d - 1) / d;
-            items += (double)tiles(s.N) * nz;
-            deepest = std::max(deepest, (double)((s.N + nz - 1) / nz));
-        }
-        const double rounds = items / at_once;
-        return (rounds < 3.0 ? std::ceil(rounds) : rounds + 0.5) * (deepest + over);
-    }
-
-    // Reduction blocks of a divergence item: items of about d planes, and at
-    // most eight blocks, since a block's sums cost about half a plane and
-    // droplets with blocks of one plane would hold up the launch.
-    static int div_blocks(const Slot& s, int d)
-    {
-        const int nzp = (s.N + s.proj_tz - 1) / s.proj_tz;
-        return std::max(1, std::min({nzp, 8, d * nzp / s.N}));
-    }
-
-    // Depth (at most `most`) of K_div's items with the least predicted time
-    // over the active droplets: all items over two groups per CU, and half of
-    // the longest item for the end.
-    int div_depth(int most) const
-    {
-        int depth = 1;
-        double best = 0.0;
-        for (int d = 1; d <= most; ++d) {
-            double all = 0.0, longest = 0.0;
-            for (const Slot& s : slots) {
-                if (!s.used || remaining(s) <= 0) continue;
-                const int nzp = (s.N + s.proj_tz - 1) / s.proj_tz, g = div_blocks(s, d);
-                const double c = (double)s.N * g / nzp + 3.0 + 0.5 * g;
-                all += c * proj_tiles(s.N) * ((nzp + g - 1) / g);
-                longest = std::max(longest, c);
-            }
-            const double rounds = all / (2.0 * cus * longest);
-            const double t = rounds < 1.0 ? longest : all / (2.0 * cus) + 0.5 * longest;
-            if (d > 1 && t >= best) continue;
-            best = t;
-            depth = d;
-        }
-        return depth;
-    }
-
     // The layout of the next launches.  One droplet: its tuned tile and depths
     // (the engine's tile if it asks for one).  Several that do not fill the
     // device: each one's tuned depths would be cut for the whole device, so
@@ -785,9 +733,11 @@ struct Engine {
         Layout l;
         int active = 0, N = 0;
         bool asked = false;
+        std::vector<SizeCount> sizes;
         for (const Slot& s : slots) {
             if (!s.used || remaining(s) <= 0) continue;
             ++active;
+            count_size(sizes, s.N, s.proj_tz);
             asked = asked || s.prm.rhs_variant >= 0;
             if (s.N > N) {
                 N = s.N;
@@ -800,10 +750,11 @@ struct Engine {
             l.variant = batch_rhs_variant;
             l.rhs_tz = batch_rhs_tz;
             l.corr_tz = batch_corr_tz;
-            l.div_tz = div_depth(batch_corr_tz);
+            l.div_tz = div_depth(sizes, batch_corr_tz, cus, proj_tiles);
             l.deep = true;
             return l;
         }
+        const std::vector<int> depths = chunk_depths(sizes, N);
         double best = 0.0;
         for (int v : {(int)RHS_16x16, (int)RHS_32x16, (int)RHS_16x8}) {
             // the 32 x 26 tile only where a droplet asks for it: 192^3 + 128^3 +
@@ -811,22 +762,14 @@ struct Engine {
             // 64-droplet sweep 1175 and 1135
             if (asked ? rhs_rows(v) != rhs_rows(l.variant) : v == RHS_32x16) continue;
             const double unit = v == RHS_16x8 ? 2.2 : 3.6;
-            for (int d = 1; d <= N; ++d) {
-                const double t = unit * chunk_time(d, 3.0, cus, [&](int n) { return rhs_tiles(v, n); });
-                if (l.rhs_tz && t >= best) continue;
-                best = t;
-                l.rhs_tz = d;
-                if (!asked) l.variant = v;
-            }
+            const Depth d = least_depth(sizes, depths, 3.0, cus, [&](int n) { return rhs_tiles(v, n); });
+            if (l.rhs_tz && unit * d.time >= best) continue;
+            best = unit * d.time;
+            l.rhs_tz = d.d;
+            if (!asked) l.variant = v;
         }
-        auto least = [&](double at_once, int (*tiles)(int)) {
-            int d = 1;
-            for (int k = 2; k <= N; ++k)
-                if (chunk_time(k, 3.0, at_once, tiles) < chunk_time(d, 3.0, at_once, tiles)) d = k;
-            return d;
-        };
-        l.div_tz = div_depth(N);
-        l.corr_tz = least(4.0 * cus, corr_tiles);
+        l.div_tz = div_depth(sizes, N, cus, proj_tiles);
+        l.corr_tz = least_depth(sizes, depths, 3.0, 4.0 * cus, corr_tiles).d;
         return l;
     }
 
@@ -875,7 +818,7 @@ struct Engine {
             // (one, except in a batch)
             const int ntile = proj_tiles(N);
             const int nzp = (N + s.proj_tz - 1) / s.proj_tz;
-            const int g = s.prm.corr_tz <= 0 && lay.div_tz > 0 ? div_blocks(s, lay.div_tz) : 1;
+            const int g = s.prm.corr_tz <= 0 && lay.div_tz > 0 ? div_blocks(N, s.proj_tz, lay.div_tz) : 1;
             for (int k0 = 0; k0 < nzp; k0 += g) {
                 const int k1 = std::min(nzp, k0 + g);
                 const int zb = k0 * N / nzp, ze = k1 * N / nzp;

@@ -1,0 +1,110 @@
+// ttsh_layout.h -- z-depths of the step kernels' work items over the active
+// droplets of a batch, by predicted time.  Host code without HIP; the tile
+// counts of the kernels are passed in.
+#pragma once
+#include <algorithm>
+#include <cmath>
+#include <vector>
+
+namespace ttsh {
+
+// Active droplets of one size and one depth of reduction blocks.  The
+// predictions below run over these and not over the slots: at many depths each,
+// for a batch of 4,096 slots they took 1 to 1.5 ms of a table rebuild that way.
+struct SizeCount {
+    int N, proj_tz, n;
+};
+
+inline void count_size(std::vector<SizeCount>& sizes, int N, int proj_tz)
+{
+    for (SizeCount& s : sizes)
+        if (s.N == N && s.proj_tz == proj_tz) {
+            ++s.n;
+            return;
+        }
+    sizes.push_back(SizeCount{N, proj_tz, 1});
+}
+
+// z is split into ceil(N/d) chunks of near-equal depth.
+inline int z_chunks(int N, int d) { return (N + d - 1) / d; }
+
+// Depths 1 .. most that split some size differently from the depth before.
+inline std::vector<int> chunk_depths(const std::vector<SizeCount>& sizes, int most)
+{
+    std::vector<int> out;
+    for (int d = 1; d <= most; ++d) {
+        bool differs = d == 1;
+        for (const SizeCount& s : sizes) differs = differs || z_chunks(s.N, d) != z_chunks(s.N, d - 1);
+        if (differs) out.push_back(d);
+    }
+    return out;
+}
+
+// Predicted time of z-chunks of depth d, in plane iterations of one
+// work-group: `over` iterations of a chunk (planes beyond its own, loading,
+// launch) come on top of d, `at_once` groups run together, and a last round
+// that is partly empty counts whole while there are few rounds.
+template <typename Tiles>
+double chunk_time(const std::vector<SizeCount>& sizes, int d, double over, double at_once, Tiles&& tiles)
+{
+    double items = 0.0, deepest = 0.0;
+    for (const SizeCount& s : sizes) {
+        const int nz = z_chunks(s.N, d);
+        items += (double)tiles(s.N) * nz * s.n;
+        deepest = std::max(deepest, (double)((s.N + nz - 1) / nz));
+    }
+    const double rounds = items / at_once;
+    return (rounds < 3.0 ? std::ceil(rounds) : rounds + 0.5) * (deepest + over);
+}
+
+// The first of the depths with the least predicted time.
+struct Depth {
+    int d;
+    double time;
+};
+template <typename Tiles>
+Depth least_depth(const std::vector<SizeCount>& sizes, const std::vector<int>& depths, double over, double at_once,
+                  Tiles&& tiles)
+{
+    Depth best{0, 0.0};
+    for (int d : depths) {
+        const double t = chunk_time(sizes, d, over, at_once, tiles);
+        if (!best.d || t < best.time) best = Depth{d, t};
+    }
+    return best;
+}
+
+// Reduction blocks of a divergence item: items of about d planes, and at most
+// eight blocks, since a block's sums cost about half a plane and droplets with
+// blocks of one plane would hold up the launch.
+inline int div_blocks(int N, int proj_tz, int d)
+{
+    const int nzp = z_chunks(N, proj_tz);
+    return std::max(1, std::min({nzp, 8, d * nzp / N}));
+}
+
+// Depth (at most `most`) of K_div's items with the least predicted time: all
+// items over two groups per CU, and half of the longest item for the end.
+template <typename Tiles>
+int div_depth(const std::vector<SizeCount>& sizes, int most, int cus, Tiles&& tiles)
+{
+    int depth = 1;
+    double best = 0.0;
+    for (int d = 1; d <= most; ++d) {
+        double all = 0.0, longest = 0.0;
+        for (const SizeCount& s : sizes) {
+            const int nzp = z_chunks(s.N, s.proj_tz), g = div_blocks(s.N, s.proj_tz, d);
+            const double c = (double)s.N * g / nzp + 3.0 + 0.5 * g;
+            all += c * tiles(s.N) * ((nzp + g - 1) / g) * s.n;
+            longest = std::max(longest, c);
+        }
+        const double rounds = all / (2.0 * cus * longest);
+        const double t = rounds < 1.0 ? longest : all / (2.0 * cus) + 0.5 * longest;
+        if (d > 1 && t >= best) continue;
+        best = t;
+        depth = d;
+    }
+    return depth;
+}
+
+}  // namespace ttsh
