@@ -81,25 +81,42 @@ static int size_index(int N)
 
 static inline size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
-// Bytes from one field to the next.  Fields whose distance is a power of two
-// put the same cell of every field on the same memory channels; a shift of 17
-// times 256 bytes per field took K_corr at 256^3 from 196 to 188 us, K_div from
-// 147 to 143 and the step of the 20-droplet sweep from 1201 to 1173 (256 bytes
-// do most of it, 129 times 256 no more).
-static inline size_t falign(size_t b) { return align256(b) + 17 * 256; }
-
 // Upper bound of divergence work items of one droplet (z-depth >= 1).
 static int proj_items_max(int N)
 {
     return proj_tiles(N) * N;
 }
 
+constexpr int kFields = 21;  // 20 FP32 fields and the edge columns
+
+// Bytes of a droplet without the fields' shift, with room for the sums of
+// `tiles` divergence tiles on every plane.
+static size_t packed_bytes(int N, int tiles)
+{
+    const size_t n = (size_t)N * N * N;
+    return kFields * align256(n * sizeof(float)) + align256(n * sizeof(float2)) +
+           align256((size_t)tiles * N * kPartSums * sizeof(double)) + align256(2 * sizeof(double)) +
+           align256(sizeof(float));
+}
+
+// Bytes from one field to the next.  Fields whose distance is a power of two
+// put the same cell of every field on the same memory channels; a shift of 17
+// times 256 bytes per field took K_corr at 256^3 from 196 to 188 us, K_div from
+// 147 to 143 and the step of the 20-droplet sweep from 1201 to 1173 (256 bytes
+// do most of it, 129 times 256 no more).  The shift takes no more than what the
+// sums leave of the room of a 32 x 8 tile's, by which budgets were sized: 17
+// from 90^3 on, 2 to 12 below, none at 32^3, whose state stays in the caches.
+static size_t field_bytes(int N)
+{
+    const size_t n = (size_t)N * N * N;
+    const size_t room = packed_bytes(N, ((N + 31) / 32) * ((N + 7) / 8)) - packed_bytes(N, proj_tiles(N));
+    return align256(n * sizeof(float)) + 256 * std::min<size_t>(17, room / (256 * kFields));
+}
+
 size_t droplet_bytes(int N)
 {
     const size_t n = (size_t)N * N * N;
-    return 20 * falign(n * sizeof(float)) + align256(n * sizeof(float2)) +
-           align256((size_t)proj_items_max(N) * kPartSums * sizeof(double)) + align256(2 * sizeof(double)) +
-           align256(sizeof(float)) + falign(n * sizeof(float));
+    return packed_bytes(N, proj_tiles(N)) + kFields * (field_bytes(N) - align256(n * sizeof(float)));
 }
 
 // K_rhs variant of a size without a tuning entry; 16x16 fits every supported N.
@@ -557,7 +574,7 @@ struct Engine {
         char* b = static_cast<char*>(mem);
         auto take = [&](size_t sz) {
             char* r = b;
-            b += sz == n * 4 ? falign(sz) : align256(sz);
+            b += sz == n * 4 ? field_bytes(N) : align256(sz);
             return r;
         };
         Drop& D = s.drop;

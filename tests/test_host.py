@@ -250,6 +250,19 @@ def test_droplet_bytes(ttsh):
     assert 23 * 4 * 128 ** 3 <= b < 24 * 4 * 128 ** 3
 
 
+@pytest.mark.parametrize("N", [32, 36, 40, 48, 50, 60, 64, 72, 80, 90, 96, 100, 120, 128, 144, 150, 160, 180, 192, 200,
+                               240, 256])
+def test_droplet_bytes_stay_within_what_budgets_were_sized_by(ttsh, N):
+    """A budget of k droplets admits k droplets: 21 FP32 fields, the complex
+    buffer, six FP64 sums per plane and 32 x 8 tile, two doubles and a float,
+    each on a 256-byte boundary, were the size of a droplet that callers'
+    budgets were made for, and a droplet takes no more."""
+    up = lambda b: -(-b // 256) * 256
+    n = N ** 3
+    sums = -(-N // 32) * -(-N // 8) * N * 6 * 8
+    assert 23 * 4 * n < ttsh.droplet_bytes(N) <= 21 * up(4 * n) + up(8 * n) + up(sums) + 512
+
+
 def test_cli_rejects_bad_sentinel(tmp_path):
     import subprocess
     exe = os.path.join(ROOT, "bacterial-droplet_amd", "bin", "ttsh3d")
