@@ -475,16 +475,6 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void k_rhs(const Drop* __restrict_
     }
 }
 
-// ---------------------------------------------------------------------------
-// Tile variants: the nominal tile a box has to hold, and the waves and records
-// per row of the kernel that runs it.
-struct RhsVar {
-    int tx, ty, nw, w;
-};
-static const RhsVar kRhsVars[RHS_NVARIANTS] = {
-    {32, 8, 8, 64}, {16, 16, 16, 64}, {64, 4, 8, 64}, {16, 8, 8, 64}, {32, 8, 8, 64}, {32, 16, 16, 36}, {64, 8, 8, 64},
-};
-
 hipError_t launch_rhs(int variant, const Drop* drops, const Work* work, const int* nwork_p, int parity, int kstep,
                       int grid, hipStream_t st)
 {
@@ -506,11 +496,6 @@ int rhs_rows(int variant)
 int rhs_cols(int variant, int N)
 {
     return variant >= 0 && variant < RHS_NVARIANTS ? rhs_tiles_x(N, kRhsVars[variant].w) : 0;
-}
-
-bool rhs_fits(int variant, int N)
-{
-    return variant >= 0 && variant < RHS_NVARIANTS && N >= kRhsVars[variant].tx + 2 && N >= kRhsVars[variant].ty + 2;
 }
 
 }  // namespace ttsh

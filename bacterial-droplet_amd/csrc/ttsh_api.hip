@@ -119,9 +119,6 @@ size_t droplet_bytes(int N)
     return packed_bytes(N, proj_tiles(N)) + kFields * (field_bytes(N) - align256(n * sizeof(float)));
 }
 
-// K_rhs variant of a size without a tuning entry; 16x16 fits every supported N.
-static int default_rhs_variant(int) { return RHS_16x16; }
-
 // K_corr work items of one z-range.
 static int corr_tiles(int N) { return ((N + kCorrTX - 1) / kCorrTX) * ((N + kCorrTY - 1) / kCorrTY); }
 
@@ -524,12 +521,8 @@ struct Engine {
         // tuned choices for N (autotuner table), unless the parameters fix them
         int tv = -1, ttz = 0, tpz = 0;
         if (!tune_lookup(N, &tv, &ttz, &tpz) || tv < 0 || tv >= RHS_NVARIANTS) { tv = -1; ttz = 0; tpz = 0; }
-        const int want = p.rhs_variant >= 0 ? p.rhs_variant : (tv >= 0 ? tv : default_rhs_variant(N));
-        int v = rhs_variant < 0 ? want : rhs_variant;
-        if (!rhs_fits(v, N)) {
-            if (p.rhs_variant >= 0) return fail(TTSH_EUNSUPPORTED, "grid smaller than the requested K_rhs tile");
-            v = RHS_16x16;  // engine-wide: every droplet fits it
-        }
+        const RhsChoice rhs = choose_rhs(N, p.rhs_variant, tv, rhs_variant);
+        if (rhs.engine < 0) return fail(TTSH_EUNSUPPORTED, "grid smaller than the requested K_rhs tile");
         HIPCHK(hipSetDevice(device));
         void* mem = nullptr;
         // a retired droplet's memory of the same size, once the work queued
@@ -560,8 +553,8 @@ struct Engine {
                 return fail(TTSH_ENOMEM, std::string("hipMalloc of droplet state failed: ") + hipGetErrorString(e));
             }
         }
-        if (v != rhs_variant) {
-            rhs_variant = v;
+        if (rhs.engine != rhs_variant) {
+            rhs_variant = rhs.engine;
             drop_graphs();
         }
         s.used = true;
@@ -615,7 +608,7 @@ struct Engine {
         s.steps = 0;
         s.limit = -1;
         s.T = p.T0;
-        s.rhs_want = want;
+        s.rhs_want = rhs.own;
         s.rhs_tz = std::min(p.rhs_tz > 0 ? p.rhs_tz : (ttz > 0 ? ttz : 16), N);
         s.rhs_tz_set = p.rhs_tz > 0;
         s.proj_tz = std::min(p.corr_tz > 0 ? p.corr_tz : (tpz > 0 ? tpz : 8), N);

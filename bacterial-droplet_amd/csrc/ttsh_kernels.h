@@ -8,8 +8,11 @@
 
 #include "ttsh_dev.h"
 #include "ttsh_internal.h"
+#include "ttsh_layout.h"
 
 namespace ttsh {
+
+static_assert(RHS_NVARIANTS == kRhsVariants, "tile variant count");
 
 // Events that the next step-kernel launch on this thread records from its
 // own dispatch (start) and completion (stop), as a profiler's kernel trace
@@ -31,12 +34,6 @@ inline hipError_t launch_kernel(K kernel, dim3 grid, dim3 block, hipStream_t st,
     return hipGetLastError();
 }
 
-// K_rhs tile variants; see kRhsVars in k_rhs.hip.  1 runs tiles of up to 60 x
-// 16 cells, 5 of up to 32 x 26, the others of up to 60 x 8.
-enum RhsVariant { RHS_32x8 = 0, RHS_16x16 = 1, RHS_64x4 = 2, RHS_16x8 = 3, RHS_32x8_O3 = 4, RHS_32x16 = 5,
-                  RHS_64x8 = 6, RHS_NVARIANTS = 7 };
-static_assert(RHS_NVARIANTS == kRhsVariants, "tile variant count");
-
 // Tile of the corrector.
 constexpr int kCorrTX = 32;
 constexpr int kCorrTY = 8;
@@ -49,11 +46,9 @@ enum { FFT_MODE_FWD = 0, FFT_MODE_INV = 1, FFT_MODE_POISSON = 2, FFT_MODE_FWD_FO
 
 hipError_t launch_rhs(int variant, const Drop* drops, const Work* work, const int* nwork_p, int parity, int kstep,
                       int grid, hipStream_t st);
-// Rows of a variant's tile, tiles across a box (0: no such variant), and
-// whether a box holds its nominal tile.
+// Rows of a variant's tile, and tiles across a box (0: no such variant).
 int rhs_rows(int variant);
 int rhs_cols(int variant, int N);
-bool rhs_fits(int variant, int N);
 
 // s = (D.v* + i D.P*)/dt0 with the stale-halo rule; FP64 partial sums of s.
 hipError_t launch_div(const Drop* drops, const Work* work, const int* nwork_p, int parity, int kstep, int grid,

@@ -1,12 +1,45 @@
-// ttsh_layout.h -- z-depths of the step kernels' work items over the active
-// droplets of a batch, by predicted time.  Host code without HIP; the tile
-// counts of the kernels are passed in.
+// ttsh_layout.h -- which K_rhs tile a droplet runs, and z-depths of the step
+// kernels' work items over the active droplets of a batch, by predicted time.
+// Host code without HIP; the tile counts of the kernels are passed in.
 #pragma once
 #include <algorithm>
 #include <cmath>
 #include <vector>
 
 namespace ttsh {
+
+// K_rhs tile variants, as callers and tuning tables number them: 1 runs tiles
+// of up to 60 x 16 cells, 5 of up to 32 x 26, the others of up to 60 x 8.
+enum RhsVariant { RHS_32x8 = 0, RHS_16x16 = 1, RHS_64x4 = 2, RHS_16x8 = 3, RHS_32x8_O3 = 4, RHS_32x16 = 5,
+                  RHS_64x8 = 6, RHS_NVARIANTS = 7 };
+
+// The smallest box that a variant is taken for, and the waves and records per
+// row of the kernel that runs it.
+struct RhsVar {
+    int least, nw, w;
+};
+constexpr RhsVar kRhsVars[RHS_NVARIANTS] = {
+    {34, 8, 64}, {18, 16, 64}, {66, 8, 64}, {18, 8, 64}, {34, 8, 64}, {34, 16, 36}, {66, 8, 64},
+};
+inline bool rhs_fits(int variant, int N)
+{
+    return variant >= 0 && variant < RHS_NVARIANTS && N >= kRhsVars[variant].least;
+}
+
+// K_rhs variant of a new droplet of size N: the one it asks for, or the tuning
+// table's where that fits, or 60 x 16, which fits every size (-1: none).
+// own: for the droplet by itself; engine: for droplets that share launches with
+// one that asks, `engine` before; -1: it asks for one that does not fit.
+struct RhsChoice {
+    int own, engine;
+};
+inline RhsChoice choose_rhs(int N, int asked, int tuned, int engine)
+{
+    const int own = asked >= 0 ? asked : rhs_fits(tuned, N) ? tuned : (int)RHS_16x16;
+    const int v = engine < 0 ? own : engine;
+    if (rhs_fits(v, N)) return {own, v};
+    return {own, asked >= 0 ? -1 : (int)RHS_16x16};
+}
 
 // Active droplets of one size and one depth of reduction blocks.  The
 // predictions below run over these and not over the slots: at many depths each,

@@ -2,7 +2,8 @@
 batches the depth of the least predicted time is the one that a search over
 every droplet and every depth finds, and the search takes no more tile counts
 than sizes times the depths that split one of them differently, however many
-droplets there are."""
+droplets there are.  And the K_rhs variant that a droplet runs: never one that
+its size does not fit."""
 import os
 import shutil
 import subprocess
@@ -93,11 +94,45 @@ int main()
 """
 
 
-def test_depths_equal_a_search_over_every_droplet(tmp_path):
+VARIANTS = r"""
+#include "ttsh_layout.h"
+#include <cstdio>
+using namespace ttsh;
+int main()
+{
+    // the tiles that boxes are measured against, by number: a box holds the
+    // tile and one cell around it
+    const int tx[7] = {32, 16, 64, 16, 32, 32, 64}, ty[7] = {8, 16, 4, 8, 8, 16, 8};
+    for (int N : {32, 33, 34, 36, 40, 64, 65, 66, 72, 128, 256}) {
+        for (int v = -2; v < 9; ++v)
+            if (rhs_fits(v, N) != (v >= 0 && v < 7 && N >= tx[v] + 2 && N >= ty[v] + 2)) return 1;
+        for (int asked = -1; asked < 7; ++asked)
+            for (int tuned = -1; tuned < 7; ++tuned)
+                for (int engine = -1; engine < 7; ++engine) {
+                    const RhsChoice c = choose_rhs(N, asked, tuned, engine);
+                    const bool first = engine < 0;
+                    if (asked >= 0 && !rhs_fits(first ? asked : engine, N)) {
+                        if (c.engine != -1) return 2;  // refused
+                        continue;
+                    }
+                    if (!rhs_fits(c.engine, N)) return 3;
+                    if (asked < 0 && !rhs_fits(c.own, N)) return 4;
+                    if (c.own != (asked >= 0 ? asked : rhs_fits(tuned, N) ? tuned : 1)) return 5;
+                    if (c.engine != (first ? c.own : rhs_fits(engine, N) ? engine : 1)) return 6;
+                }
+    }
+    std::printf("ok\n");
+    return 0;
+}
+"""
+
+
+@pytest.mark.parametrize("driver", [DRIVER, VARIANTS], ids=["depths", "variants"])
+def test_layout(tmp_path, driver):
     gxx = shutil.which("g++")
     if gxx is None:
         pytest.skip("g++ not available")
-    (tmp_path / "driver.cpp").write_text(DRIVER)
+    (tmp_path / "driver.cpp").write_text(driver)
     exe = tmp_path / "driver"
     r = subprocess.run([gxx, "-std=c++17", "-O1", "-fsanitize=address,undefined", "-fno-sanitize-recover=all", "-I", CSRC,
                         str(tmp_path / "driver.cpp"), "-o", str(exe)], capture_output=True, text=True, timeout=300)
