@@ -157,7 +157,7 @@ __global__ __launch_bounds__(64 * kProjWaves, 8) void k_div(const Drop* __restri
             zend = (ordb / ntile + 1) * N / D.nzp;
         };
         // D.v*/dt0 and D.P*/dt0 of a cell
-        const float scale = D.co.d1 * (1.f / 36.f) * D.co.inv_dt0;
+        const float scale = D.co.s_dt0;
         const unsigned oc = 2u * o;
         int buf = 0;
         const int own_i = wv * 64 + lane;

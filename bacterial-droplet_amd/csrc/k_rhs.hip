@@ -291,7 +291,7 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void k_rhs(const Drop* __restrict_
 #pragma unroll
         for (int j = 0; j < 7; ++j) nx[0][j] = 0.f;
         fvec4 *bx = lds, *by = lds + BUF;
-        const float s = co.d1 * (1.f / 36.f), lc = co.lc;
+        const float s = co.s, lc = co.lc;
 
         __syncthreads();  // the previous item has read both buffers
         auto body = [&](auto ph_, int zm) {

@@ -36,7 +36,8 @@ struct Coef {
     float sw0, sw1;   // transverse smoothing S=[sw1,sw0,sw1] = [1,4,1]/6
     float lc, lf, l0; // Laplacian: 8 corners 1/(12h^2), 6 faces 2/(3h^2), centre -14/(3h^2)
     float Dt;         // dt0 (Dt never changes in the reference, TTSH3D.cu:759)
-    float inv_dt0;    // 1/dt0, the getStream type-0 divisor (TTSH3D.cu:665)
+    float s;          // 1/(72 h): scale of the whole-number first-derivative stencils
+    float s_dt0;      // s/dt0, with the getStream type-0 divisor (TTSH3D.cu:665)
     float mu, cA, alpha, beta, eta, La2, lambda0, aPhi2, kPhi, gamma, A;
     float e0, e1;     // d1*sw0, d1*sw1: weights of a transverse-smoothed difference
     float f00, f01, f11;  // d1*sw0^2, d1*sw0*sw1, d1*sw1^2: weights of S (x) S (x) difference
