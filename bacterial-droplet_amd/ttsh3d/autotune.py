@@ -7,11 +7,12 @@ writes the fastest choices as the tuning table libttsh3d.so reads (tuned.txt
 beside the library, lines "N rhs_variant rhs_tz proj_tz").
 
 With --batch it tunes the layout of a batch that fills the device instead:
-on the 64-droplet sweep mix (L in {48, 64, 96, 128}) as one graph batch, it
-times whole batch steps for each K_rhs kernel that fits all sizes, minimum
-K_rhs z-depth and divergence/corrector z-depth, through the table's "batch"
-line (re-read between candidates; the batch is laid out again at its next
-step), and keeps the fastest.  The FFT passes' lines per work-group are
+on the 64-droplet sweep mix (L in {48, 64, 96, 128}) and on its first 20
+droplets, each as one graph batch, it times whole batch steps for each K_rhs
+kernel that fits all sizes, minimum K_rhs z-depth and divergence/corrector
+z-depth, through the table's "batch" line (re-read between candidates; the
+batches are laid out again at their next step), and keeps the layout with the
+least geometric mean of the two times.  The FFT passes' lines per work-group are
 compile-time constants and not part of the search.
 
     python -m ttsh3d.autotune [--sizes 48 64 96 128 192 256] [--steps 30] [--out PATH]
@@ -21,6 +22,7 @@ from __future__ import annotations
 
 import argparse
 import json
+import math
 import os
 import sys
 import time
@@ -112,44 +114,63 @@ def write_table(entries: dict, path: str, batch=None):
             f.write("batch {} {} {}\n".format(*batch))
 
 
+# Droplets of the sweep mix in the batches that the batch line is tuned on: a
+# layout that suits the full mix alone costs a share of it, as one of many GPUs
+# runs, more than it gains.
+BATCH_MIXES = (64, 20)
+
+
+def best_batch(results):
+    """The layout with the least geometric mean of its times over the mixes:
+    results holds dicts with variant, rhs_tz, corr_tz and ms, a time per mix.
+    Returns ((variant, rhs_tz, corr_tz), ms)."""
+    r = min(results, key=lambda r: sum(math.log(t) for t in r["ms"]))
+    return (r["variant"], r["rhs_tz"], r["corr_tz"]), r["ms"]
+
+
 def tune_batch(table: str, steps: int = 48, log=print):
-    """Fastest device-filling batch layout on the 64-droplet sweep mix.
-    Candidates are written one at a time into a scratch copy of the table
-    (its per-size lines kept) and re-read; returns ((variant, rhs_tz,
-    corr_tz), ms per batch step, all results)."""
+    """Fastest device-filling batch layout on the sweep mixes of BATCH_MIXES
+    droplets.  Candidates are written one at a time into a scratch copy of the
+    table (its per-size lines kept) and re-read; returns ((variant, rhs_tz,
+    corr_tz), ms per batch step of each mix, all results)."""
+    import ttsh3d
     from . import workloads
     entries, _ = read_table(table)
-    cases = workloads.sweep_mix(__import__("ttsh3d"))
+    cases = workloads.sweep_mix(ttsh3d, max(BATCH_MIXES))
     sizes = sorted({L for _, L, _ in cases})
     variants = [v for v in TUNED_VARIANTS if all(L >= max(RHS_VARIANTS[v]) + 2 for L in sizes)]
     scratch = table + ".tuning"
     results = []
-    best = None
-    b = Batch(max_slots=len(cases), use_graph=True)
+    batches = [Batch(max_slots=n, use_graph=True) for n in BATCH_MIXES]
     try:
-        for p, L, s in cases:
-            b.admit(p, *workloads.mix_state(__import__("ttsh3d"), L, s))
+        for i, (p, L, s) in enumerate(cases):
+            state = workloads.mix_state(ttsh3d, L, s)
+            for b, n in zip(batches, BATCH_MIXES):
+                if i < n:
+                    b.admit(p, *state)
         for var in variants:
             for rtz in (8, 12, 16, 24, 32, 48, 64):
                 for ctz in (8, 16, 32):
                     write_table(entries, scratch, (var, rtz, ctz))
                     tuning_reload(scratch)
-                    b.step(16)  # re-layout and graph capture
-                    b.synchronize()
-                    t0 = time.perf_counter()
-                    b.step(steps)
-                    b.synchronize()
-                    ms = (time.perf_counter() - t0) * 1e3 / steps
+                    ms = []
+                    for b in batches:
+                        b.step(16)  # re-layout and graph capture
+                        b.synchronize()
+                        t0 = time.perf_counter()
+                        b.step(steps)
+                        b.synchronize()
+                        ms.append((time.perf_counter() - t0) * 1e3 / steps)
                     results.append({"variant": var, "rhs_tz": rtz, "corr_tz": ctz, "ms": ms})
-                    log(f"batch variant {var} {RHS_VARIANTS[var]} rhs_tz {rtz} corr_tz {ctz}: {ms:.3f} ms/step")
-                    if best is None or ms < best[1]:
-                        best = ((var, rtz, ctz), ms)
+                    log(f"batch variant {var} rhs_tz {rtz} corr_tz {ctz}: " +
+                        ", ".join(f"{t:.3f} ms/step of {n}" for t, n in zip(ms, BATCH_MIXES)))
     finally:
-        b.close()
+        for b in batches:
+            b.close()
         if os.path.exists(scratch):
             os.remove(scratch)
         tuning_reload(table if os.path.exists(table) else None)
-    return best[0], best[1], results
+    return (*best_batch(results), results)
 
 
 def main(argv=None):
@@ -170,8 +191,8 @@ def main(argv=None):
         if a.json:
             with open(a.json, "w") as f:
                 json.dump({"batch": res, "best": best, "ms": ms}, f, indent=1)
-        print(f"batch layout: variant {best[0]} rhs_tz {best[1]} corr_tz {best[2]} ({ms:.3f} ms per batch step); "
-              f"wrote {a.out} in {time.time() - t0:.1f} s", flush=True)
+        print(f"batch layout: variant {best[0]} rhs_tz {best[1]} corr_tz {best[2]} ({', '.join(f'{t:.3f}' for t in ms)} ms "
+              f"per batch step); wrote {a.out} in {time.time() - t0:.1f} s", flush=True)
         tuning_reload(a.out)
         return 0
     entries, allres = {}, {}
