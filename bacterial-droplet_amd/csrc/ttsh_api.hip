@@ -677,7 +677,7 @@ struct Engine {
     // chunks of about batch_corr_tz planes in the same batches.  K_div's sums,
     // which set the k = 0 coefficient and sigma, stay per tuned chunk
     // (Drop::part), so they do not change either.
-    int batch_rhs_variant = RHS_16x16, batch_rhs_tz = 32, batch_corr_tz = 32;
+    int batch_rhs_variant = RHS_60x16, batch_rhs_tz = 32, batch_corr_tz = 32;
     int tune_gen_seen = -1;
 
     // Re-read the batch entry of the tuning table after a reload; a running
@@ -687,9 +687,9 @@ struct Engine {
         const int g = tune_generation();
         if (g == tune_gen_seen) return;
         tune_gen_seen = g;
-        int v = RHS_16x16, rtz = 32, ctz = 32;
+        int v = RHS_60x16, rtz = 32, ctz = 32;
         if (!tune_batch_lookup(&v, &rtz, &ctz) || v < 0 || v >= RHS_NVARIANTS) {
-            v = RHS_16x16;
+            v = RHS_60x16;
             rtz = 32;
             ctz = 32;
         }
@@ -756,12 +756,12 @@ struct Engine {
         }
         const std::vector<int> depths = chunk_depths(sizes, N);
         double best = 0.0;
-        for (int v : {(int)RHS_16x16, (int)RHS_32x16, (int)RHS_16x8}) {
+        for (int v : {(int)RHS_60x16, (int)RHS_32x26, (int)RHS_60x8}) {
             // the 32 x 26 tile only where a droplet asks for it: 192^3 + 128^3 +
             // 96^3 + 64^3 take 633 us a step with it, 621 without, and the
             // 64-droplet sweep 1175 and 1135
-            if (asked ? rhs_rows(v) != rhs_rows(l.variant) : v == RHS_32x16) continue;
-            const double unit = v == RHS_16x8 ? 2.2 : 3.6;
+            if (asked ? rhs_rows(v) != rhs_rows(l.variant) : v == RHS_32x26) continue;
+            const double unit = v == RHS_60x8 ? 2.2 : 3.6;
             const Depth d = least_depth(sizes, depths, 3.0, cus, [&](int n) { return rhs_tiles(v, n); });
             if (l.rhs_tz && unit * d.time >= best) continue;
             best = unit * d.time;

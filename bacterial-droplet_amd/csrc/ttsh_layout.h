@@ -8,13 +8,14 @@
 
 namespace ttsh {
 
-// K_rhs tile variants, as callers and tuning tables number them: 1 runs tiles
-// of up to 60 x 16 cells, 5 of up to 32 x 26, the others of up to 60 x 8.
-enum RhsVariant { RHS_32x8 = 0, RHS_16x16 = 1, RHS_64x4 = 2, RHS_16x8 = 3, RHS_32x8_O3 = 4, RHS_32x16 = 5,
-                  RHS_64x8 = 6, RHS_NVARIANTS = 7 };
+// K_rhs variants, as callers and tuning tables number them 0 .. 6.  There are
+// three kernels, named here by the largest tile they run; 0, 2, 4 and 6 are
+// further numbers of the second.
+enum RhsVariant { RHS_60x16 = 1, RHS_60x8 = 3, RHS_32x26 = 5, RHS_NVARIANTS = 7 };
 
-// The smallest box that a variant is taken for, and the waves and records per
-// row of the kernel that runs it.
+// By number: the smallest box that it is taken for (every kernel runs every
+// size; a number keeps the bound that callers know it by), and the waves and
+// records per tile row of its kernel.
 struct RhsVar {
     int least, nw, w;
 };
@@ -27,7 +28,7 @@ inline bool rhs_fits(int variant, int N)
 }
 
 // K_rhs variant of a new droplet of size N: the one it asks for, or the tuning
-// table's where that fits, or 60 x 16, which fits every size (-1: none).
+// table's where that fits, or 60 x 16, which is taken for every size (-1: none).
 // own: for the droplet by itself; engine: for droplets that share launches with
 // one that asks, `engine` before; -1: it asks for one that does not fit.
 struct RhsChoice {
@@ -35,10 +36,10 @@ struct RhsChoice {
 };
 inline RhsChoice choose_rhs(int N, int asked, int tuned, int engine)
 {
-    const int own = asked >= 0 ? asked : rhs_fits(tuned, N) ? tuned : (int)RHS_16x16;
+    const int own = asked >= 0 ? asked : rhs_fits(tuned, N) ? tuned : (int)RHS_60x16;
     const int v = engine < 0 ? own : engine;
     if (rhs_fits(v, N)) return {own, v};
-    return {own, asked >= 0 ? -1 : (int)RHS_16x16};
+    return {own, asked >= 0 ? -1 : (int)RHS_60x16};
 }
 
 // Active droplets of one size and one depth of reduction blocks.  The

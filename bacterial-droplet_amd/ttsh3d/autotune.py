@@ -29,7 +29,8 @@ import time
 
 from . import F64, TTSHError, Batch, Simulation, default_params, init_droplet, lib, LIB_PATH, tuning_reload
 
-# nominal tile of each variant: the box has to hold it
+# by variant, the tile that a box has to hold with a cell around it for the
+# variant to be taken; the kernels themselves run other tiles (TUNED_VARIANTS)
 RHS_VARIANTS = {0: (32, 8), 1: (16, 16), 2: (64, 4), 3: (16, 8), 4: (32, 8), 5: (32, 16), 6: (64, 8)}
 # one variant of each kernel, with the smallest nominal tile: tiles of up to
 # 60 x 16, 60 x 8 and 32 x 26 cells
