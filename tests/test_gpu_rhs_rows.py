@@ -1,9 +1,12 @@
-"""K_rhs's two kernels (16 and 8 rows per work-group, variants 1 and 3) on
-fields that are rough everywhere, at the sizes where a tile can go wrong: one
-tile narrower than a wave (32, 36), exactly 60 cells wide (60, 180), two equal
-tiles (64, 90), three with a last one narrower (128), rows that end inside a
-tile (36, 50, 60, 90, 180), and z-chunks of one plane, of unequal depths and of
-the whole box.
+"""K_rhs's three kernels (tiles of 60 x 16, 60 x 8 and 32 x 26 cells, variants 1,
+3 and 5) on fields that are rough everywhere, at the sizes where a tile can go
+wrong, with z-chunks of one plane, of unequal depths and of the whole box.  Tiles
+of a wave per row: one tile narrower than a wave (32, 36), exactly 60 cells wide
+(60, 180), two equal tiles (64, 90, 96), three with a last one narrower (128),
+rows that end inside a tile (36, 50, 60, 90, 180).  The flattened 32 x 26 tile:
+its smallest box (36), the full width of 32 (64, 96, 128), narrower tiles that
+divide the box (36: 18, 60: 30) or not (50: 25 is even, 80: 27, 27, 26), and last
+tiles of all but two rows less (128: 24 of 26) down to two rows (80).
 
 phi^{n+1}, v* and P* of one step against the FP64 oracle: a value is the end of
 fewer than 400 roundings of terms no larger than the field's largest value
@@ -21,7 +24,8 @@ KEYS = ("h", "dt0", "mu", "cA", "alpha", "beta", "eta", "La", "kappa", "lambda0"
 BAR = 400 * 2.0 ** -24
 
 
-@pytest.mark.parametrize("N,A", [(32, 0.0), (36, 0.4), (50, 0.0), (60, 0.4), (64, 0.0), (90, 0.4), (128, 0.0), (180, 0.0)])
+@pytest.mark.parametrize("N,A", [(32, 0.0), (36, 0.4), (50, 0.0), (60, 0.4), (64, 0.0), (80, 0.4), (90, 0.4), (96, 0.0), (128, 0.0),
+                                 (180, 0.0)])
 def test_rough_fields(ttsh, oracle_mod, N, A):
     print(f"[rough_fields N={N}]", flush=True)
     oracle_mod.set_threads(min(16, os.cpu_count() or 1))

@@ -63,22 +63,24 @@ def test_step_limits_and_divergence_isolation(ttsh):
         assert np.array_equal(a, c)
 
 
-def test_large_batch_fused_xy_equals_alone(ttsh):
-    """Eight 64^3 droplets give 512 z-planes, enough for the engine to switch
-    that size to the fused x+y FFT pass; alone, each droplet runs the
-    single-axis passes.  Both perform the same per-line arithmetic, so the
-    results are bitwise equal."""
-    log("[large_batch_fused_xy_equals_alone]")
-    N, steps = 64, 12
-    cases = [(-1.0 * (1 + 0.25 * i), 1.0 + 0.1 * i, 300 + i) for i in range(8)]
+def test_large_batch_separate_sums_equals_alone(ttsh):
+    """Twelve 64^3 droplets have 1,536 work-groups in an x pass, more than four
+    per CU, so the projection's sums are added by k_proj_stats and the x pass
+    only reads sigma; alone (128 groups), the x pass adds them itself.  Both add
+    in the same order, so the results are bitwise equal.  33 and 32 steps: two
+    replays of a graph that starts at each parity, a plain step between."""
+    log("[large_batch_separate_sums_equals_alone]")
+    N, steps = 64, 65
+    cases = [(-1.0 * (1 + 0.25 * i), 1.0 + 0.1 * i, 300 + i) for i in range(12)]
     f = lambda a: a.astype(np.float32)
-    with ttsh.Batch(max_slots=8, use_graph=True) as b:
+    with ttsh.Batch(max_slots=12, use_graph=True) as b:
         slots = []
         for cA, La, seed in cases:
             p = ttsh.default_params(N=N, dt0=0.01, cA=cA, La=La)
             phi, P, v = ttsh.init_droplet(N, 0.3 * N, 2.0, 0, seed)
             slots.append(b.admit(p, f(phi), f(P), f(v), dtype=ttsh.F32))
-        b.step(steps)
+        b.step(33)
+        b.step(steps - 33)
         got = [b.get_state(s) for s in slots]
     for (cA, La, seed), g in zip(cases, got):
         ref = alone(ttsh, N, cA, La, seed, steps)
@@ -109,12 +111,13 @@ def test_sweep_equals_runs_alone(ttsh, tmp_path):
 
 
 def test_device_filling_batch_layout_equals_alone(ttsh):
-    """Six 128^3 and two 96^3 droplets make 1,752 K_rhs items at the batch
-    layout (32x8 tiles, z-chunks of 32), more than two rounds of three groups
-    on 256 CUs, so the engine runs K_rhs that way and K_corr with chunks of 32.
-    Alone, each droplet runs its tuned 32x16 tile with chunks of 8 or 16
-    planes and K_corr with 8 or 16.  Neither kernel reduces anything, so the
-    results are bitwise equal."""
+    """Six 128^3 and two 96^3 droplets make 648 K_rhs items at the batch layout
+    (60x16 tiles, z-chunks of 32), more than two rounds of one group on 256 CUs,
+    so the engine runs K_rhs that way, K_corr with chunks of 16 and K_div with
+    items of several reduction blocks.  Alone, a 128^3 droplet runs 32x26 tiles
+    in chunks of 11 planes and a 96^3 droplet 60x16 tiles in chunks of 5, K_corr
+    8 and 6.  K_rhs and K_corr reduce nothing and K_div's sums are per block, so
+    the results are bitwise equal."""
     log("[device_filling_batch_layout_equals_alone]")
     steps = 6
     cases = [(128, -1.0 * (1 + 0.3 * i), 1.0 + 0.1 * i, 700 + i) for i in range(6)]
@@ -135,11 +138,11 @@ def test_device_filling_batch_layout_equals_alone(ttsh):
 
 
 def test_layout_switch_mid_run_equals_alone(ttsh):
-    """Six 128^3 and two 96^3 droplets start in the device-filling layout
-    (1,752 K_rhs items at depth 32).  Three 128^3 droplets stop after 8 steps,
-    leaving 984 items, so the engine returns to the tuned layout (and
-    re-captures its graphs) while the others run on to 40 steps.  Every
-    droplet still equals its run alone, bitwise."""
+    """Six 128^3 and two 96^3 droplets start in the device-filling layout (648
+    K_rhs items at depth 32).  Three 128^3 droplets stop after 8 steps, leaving
+    360 items, fewer than two rounds, so the engine goes over to a common depth
+    for the rest while the others run on to 40 steps.  Every droplet still
+    equals its run alone, bitwise."""
     log("[layout_switch_mid_run_equals_alone]")
     cases = [(128, -1.0 - 0.2 * i, 1.0 + 0.05 * i, 720 + i, 8 if i < 3 else 40) for i in range(6)]
     cases += [(96, -1.2, 1.1, 730, 40), (96, -0.8, 0.9, 731, 40)]

@@ -3,8 +3,8 @@ the FP64 oracle and against each droplet run alone.
 
   - The sweep mix (64 droplets, L in {48, 64, 96, 128}, seed 1004) runs 100
     steps as one graph batch; it fills the device, so K_rhs runs the batch
-    layout (32x8 tiles, z-chunks of 32) and the small sizes the fused x+y
-    FFT pass.  One droplet per size matches the oracle (relative RMS 1e-4,
+    layout (60x16 tiles, z-chunks of at least 32) and each FFT pass one launch
+    for several sizes.  One droplet per size matches the oracle (relative RMS 1e-4,
     the bar of every 100-step parity case) and its own plain-step run
     bitwise; every droplet stays finite.
   - A served stream over L in {64, 96, 128, 192} (12 requests, two or more
