@@ -100,12 +100,12 @@ class HostCopier {
 public:
     // Below this the threads cost more than they save.
     static constexpr size_t kMinBytes = (size_t)8 << 20;
-    // States below kLargeBytes use 4 chunks of 2 MiB, larger ones 8 of 4 MiB.
-    // The first copy through a ring takes the page faults of its host mapping,
-    // about 0.13 ms per MiB.  A first read of a 72^3 or 96^3 state takes 1.2 and
-    // 2.5 ms with the small ring, 1.9 and 4.7 with the large one, later ones
-    // 0.44 and 0.79 against 0.43 and 0.75.  Where a plain copy takes 5 ms and
-    // more (128^3) the large ring's first read costs no more than that.
+    // States below kLargeBytes use chunks of 2 MiB, larger ones of 4 MiB.  The
+    // first copy through a ring takes the page faults of its host mapping, about
+    // 0.13 ms per MiB: a first read of a 96^3 state (25 MB) takes 3.0 ms, with
+    // chunks of 4 MiB 4.7, with one plain copy 2.5.  Later reads take 0.79 ms
+    // against 0.75 (in FP64 0.89 and 1.0).  At 128^3 (59 MB) they would take 1.62
+    // against 1.47, and a plain copy takes as long as the larger ring's first.
     static constexpr size_t kLargeBytes = (size_t)32 << 20;
 
     HostCopier() { PinnedRings::get().join(); }
@@ -137,7 +137,6 @@ public:
         size_t bytes = 0;
         for (auto p = mine; p != pieces.end(); ++p) bytes += p->n * sizeof(float);
         if (bytes < kMinBytes || !events()) return hipSuccess;
-        slots = bytes < kLargeBytes ? kSlots / 2 : kSlots;
         chunk_n = bytes < kLargeBytes ? kChunk / 2 : kChunk;
         struct Loan {
             Ring r;
@@ -145,7 +144,7 @@ public:
             {
                 if (r.p) PinnedRings::get().give(r);
             }
-        } loan{PinnedRings::get().borrow(chunk_n * slots)};  // outlives the workers and every copy into it
+        } loan{PinnedRings::get().borrow(chunk_n * kSlots)};  // outlives the workers and every copy into it
         ring = loan.r.p;
         if (!ring) return hipSuccess;
         std::vector<HostPiece> chunk;
@@ -169,9 +168,9 @@ public:
         size_t issued = 0;
         for (size_t i = 0; i < chunk.size() && e == hipSuccess; ++i) {
             // keep every free slot's copy in flight; chunk i's slot frees up
-            // when the workers have stored chunk i - slots
-            while (issued < chunk.size() && issued < i + slots && e == hipSuccess) {
-                const int s = (int)(issued % slots);
+            // when the workers have stored chunk i - kSlots
+            while (issued < chunk.size() && issued < i + kSlots && e == hipSuccess) {
+                const int s = (int)(issued % kSlots);
                 {
                     std::unique_lock<std::mutex> lk(mu);
                     if (busy[s]) {
@@ -185,12 +184,12 @@ public:
                 ++issued;
             }
             if (e != hipSuccess) break;
-            const int s = (int)(i % slots);
+            const int s = (int)(i % kSlots);
             e = hipEventSynchronize(ev[s]);
             if (e != hipSuccess) break;
             {
                 std::lock_guard<std::mutex> lk(mu);
-                ready[tail++ % slots] = Job{s, chunk[i].dst, chunk[i].n};
+                ready[tail++ % kSlots] = Job{s, chunk[i].dst, chunk[i].n};
             }
             ready_cv.notify_one();
         }
@@ -242,7 +241,7 @@ private:
                 std::unique_lock<std::mutex> lk(mu);
                 ready_cv.wait(lk, [&] { return quit || head != tail; });
                 if (head == tail) return;
-                j = ready[head++ % slots];
+                j = ready[head++ % kSlots];
             }
             const float* s = slot(j.slot);
             if (f64) {
@@ -260,7 +259,7 @@ private:
     }
 
     float* ring = nullptr;
-    size_t slots = kSlots, chunk_n = kChunk;  // of the copy under way
+    size_t chunk_n = kChunk;  // of the copy under way
     hipEvent_t ev[kSlots] = {};
     std::mutex mu;
     std::condition_variable ready_cv, free_cv;
