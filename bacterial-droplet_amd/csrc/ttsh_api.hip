@@ -481,7 +481,7 @@ struct Engine {
         co.lc = (float)(1.0 / (12.0 * h * h));
         co.Dt = (float)p.dt0;
         co.s = (float)(1.0 / (72.0 * h));
-        co.s_dt0 = (float)(1.0 / (72.0 * h * p.dt0));
+        co.inv_dt0 = (float)(1.0 / p.dt0);
         co.mu = (float)p.mu;
         co.cA = (float)p.cA;
         co.alpha = (float)p.alpha;

@@ -37,7 +37,7 @@ struct Coef {
     float lc;         // 1/(12 h^2): scale of the whole-number Laplacian (1, 8, -56; TTSH3D.cu:3331-3343)
     float Dt;         // dt0 (Dt never changes in the reference, TTSH3D.cu:759)
     float s;          // 1/(72 h): scale of the whole-number first-derivative stencils
-    float s_dt0;      // s/dt0, with the getStream type-0 divisor (TTSH3D.cu:665)
+    float inv_dt0;    // 1/dt0, the getStream type-0 divisor (TTSH3D.cu:665)
     float mu, cA, alpha, beta, eta, La2, lambda0, aPhi2, kPhi, gamma, A;
     float pk0;        // -1/(k2s N^3), k2 = k2s*(mx^2+my^2+mz^2), k2s = (2 pi/(N h))^2 (TTSH3D.cu:1094-1114)
     float inv_n3;     // 1/N^3, the type-2 divisor (TTSH3D.cu:687)

@@ -1,5 +1,5 @@
-"""The stencils' scale s = 1/(72 h) and the divergence's s/dt0 are rounded once,
-from FP64.
+"""The stencils' scale s = 1/(72 h) is rounded once, from FP64, and the
+divergence's s/dt0 is its product with 1/dt0.
 
 K_rhs: phi is 0 on every second cell (a checkerboard) and a small whole number on
 the others, v = (1, 0, 0), gamma = 0, Dt = 2^-7.  At the zeros phi^{n+1} is then
@@ -10,9 +10,10 @@ K_div: p of one step against the FP64 oracle, as the ratio of the two fields, in
 which the roundings of 32^3 cells average out (2e-7/sqrt(32^3) = 1e-9).  What is
 left is the rounding of s/dt0 and of the Poisson factor's constant, both known,
 and that of the transform's constants, the same for every h.  At h = 1.377,
-dt0 = 0.006 the first two are -1e-8 together, where a product of rounded factors
-makes 1.3e-7; so the difference to h = 1, dt0 = 1/128, where such a product is
-exact, tells them apart, with a bar of 3e-8."""
+dt0 = 0.006 the first two are -1e-8 together, where a product of three rounded
+factors, 1/(2h), 1/36 and 1/dt0, makes 1.3e-7; so the difference to h = 1,
+dt0 = 1/128, where either product rounds as once, tells them apart, with a bar of
+3e-8."""
 import numpy as np
 import pytest
 
@@ -54,8 +55,9 @@ def test_rhs_scale(ttsh, h, variant):
 
 def scale_rounding(N, h, dt):
     """Relative roundings of s/dt0 and of -1/((2 pi/(N h))^2 N^3), added."""
-    once = lambda x: float(F(x)) / x - 1.0
-    return once(1.0 / (72.0 * h * dt)) + once(-1.0 / ((2.0 * np.pi / (N * h)) ** 2 * N ** 3))
+    off = lambda a, b: float(a) / b - 1.0
+    k = -1.0 / ((2.0 * np.pi / (N * h)) ** 2 * N ** 3)
+    return off(F(1.0 / (72.0 * h)) * F(1.0 / dt), 1.0 / (72.0 * h * dt)) + off(F(k), k)
 
 
 def test_div_scale(ttsh, oracle_mod):
