@@ -49,9 +49,10 @@ namespace ttsh {
 // neighbourhoods of six fields from LDS behind two barriers per plane and
 // fetched a 33% ring; here the apron is 64*16/(62*14), 18%.  Waves hold 64
 // VGPRs, so that two work-groups share a CU and one loads while the other
-// waits at its barrier.  Measured with the 4.7 us of k_proj_stats: 96^3 19.5
-// -> 15.8 us, 128^3 26.1 -> 23.1, 180^3 70 -> 53, 256^3 166 -> 149 (637 MB of
-// traffic in 144 us, 4.4 TB/s).
+// waits at its barrier.  Measured with the 4.7 us of k_proj_stats, which lone
+// droplets up to 128^3 do without: 96^3 19.5 -> 15.8 us, 128^3 26.1 -> 23.1,
+// 180^3 70 -> 55, 256^3 166 -> 142; k_div alone moves 604 MB in 137 us at 256^3,
+// 4.4 TB/s.
 __global__ __launch_bounds__(64 * kProjWaves, 8) void k_div(const Drop* __restrict__ drops,
                                                             const Work* __restrict__ work,
                                                             const int* __restrict__ nwork_p, int parity, int kstep)

@@ -43,10 +43,10 @@
 // at 230.  A record per row and field needs one 16-byte write and two 16-byte
 // reads per field where the 2D stencils took 22 values, and each one-axis sum
 // is made once instead of by every neighbour: 44 LDS and 430 VALU
-// instructions per plane and wave.  Measured, same boxes, 16-row tiles
-// against the best of the former tiles: 64^3 37 -> 19 us (in z-chunks of two
-// planes instead of eight), 128^3 75 -> 55 (47 with the flattened tile),
-// 180^3 216 -> 119, 240^3 463 -> 234, 256^3 498 -> 324.
+// instructions per plane and wave.  Measured, 16-row tiles against the best of
+// the former tiles, each at its best depth: 64^3 37 -> 17 us (in z-chunks of two
+// planes instead of eight), 128^3 75 -> 58 (46 with the flattened tile),
+// 180^3 216 -> 98, 240^3 463 -> 207, 256^3 498 -> 282.
 //
 // Tiles.  W = 64: one wave per row of TX <= 60 cells, whose 64 lanes include
 // the 2-cell x apron; 8 or 16 rows per work-group.  N is cut into ceil(N/60)
@@ -55,8 +55,8 @@
 // and two of its neighbours' on either side.  A wave of a 60-wide tile is
 // idle in part where 60 does not divide N well (64^3, 128^3: a third to a
 // half), a wave of the flattened tile only at its ends.  At 128^3 that makes
-// 20 tiles of 24 and 47 us of 52; where the counts are equal the flattened
-// tile is 3% (96^3) to 11% (256^3, its rows end inside cache lines more often)
+// 20 tiles of 24 and 46 us of 58; where the counts are equal the flattened
+// tile is 3% (96^3) to 12% (256^3, its rows end inside cache lines more often)
 // slower, so the tuning table chooses per size.  Two rows per wave (213
 // VGPRs, two waves per SIMD) measured 4% slower at 128^3 and equal at 240^3
 // and 256^3.  The rows above and below the tile are staged by all waves, one
@@ -65,7 +65,7 @@
 //
 // 16 waves (128 VGPRs, 160 KB of LDS: one group per CU, four waves per SIMD)
 // have the smaller share of apron rows and are faster wherever the device is
-// full: 240^3 234 against 317 us.  8 waves (98 KB) take 2.1 us per plane
+// full: 240^3 207 against 316 us.  8 waves (98 KB) take 2.1 us per plane
 // instead of 3.2 when a CU holds one group, which wins for small boxes.  All
 // do the same arithmetic in the same order (no contraction in this file), so a
 // droplet's result does not depend on the tile.

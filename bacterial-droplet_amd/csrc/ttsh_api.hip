@@ -2,19 +2,22 @@
 // graphs and batches of droplets.
 //
 // An Engine owns a set of droplet slots on one device and one stream.  One
-// step of the engine is eight kernel kinds, each launched once per step (the
-// FFT passes once per kind of size present), each covering every active
-// droplet through a work table (see ttsh_dev.h):
-//   K_rhs, K_div (for large droplets with k_proj_stats, the sums behind it), FFT x
-//   fwd, FFT y fwd, FFT z (fwd, -1/k^2, inv), FFT y inv, FFT x inv, K_corr
-// (sizes up to kMaxPlane do y, z and y in the z slot) standing in for the reference's EEuler (TTSH3D.cu:347-359: 107 kernel
-// launches and 4 cuFFT transforms per step).
+// step of the engine is a sequence of launches, each covering active droplets
+// through a work table (see ttsh_dev.h):
+//   K_rhs, K_div, k_proj_stats (its sums, unless the x pass adds them), FFT x,
+//   then for sizes up to kMaxPlane the y-z planes, for the others FFT y,
+//   z (fwd, -1/k^2, inv), y inv, then FFT x inv, K_corr
+// standing in for the reference's EEuler (TTSH3D.cu:347-359: 107 kernel
+// launches and 4 cuFFT transforms per step).  A lone droplet up to kMaxPlane is
+// stepped by six launches, a larger one by nine; a batch of several sizes has
+// one launch per FFT pass for all of them and one or more for the planes.
 //
 // ttsh_sim is an engine with one slot stepped with plain launches.  A
 // ttsh_batch may capture K steps in a HIP graph and replay it; the kernels
 // then run with fixed grids and read work counts from device memory, so
-// admitting or retiring droplets rewrites tables without re-capturing
-// (unless a table must grow or a grid size appears that the graph lacks).
+// admitting or retiring droplets rewrites tables.  It re-captures if a table
+// must grow, a grid size appears that the graph lacks, the K_rhs kernel changes,
+// or the FFT launches do (FftLayout).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -183,7 +186,10 @@ struct Engine {
     int ggrid[kNTables] = {};
     // What the FFT launches cover: the sizes present, and which launches serve
     // several sizes: x passes (T_MX), y and z passes (T_MY, T_MZ), planes of
-    // each group (T_MP).
+    // each group (T_MP).  A graph serves the same launches for fewer sizes; any
+    // other change captures again, 0.2 to 0.5 ms of the host's time.  A stream
+    // of requests of only 50 to 300 steps, 32^3 to 64^3, does so at every fourth
+    // step call, 3 to 6% of its time.
     struct FftLayout {
         unsigned sizes = 0;
         bool mx = false, mz = false, mp[2] = {false, false};
@@ -757,9 +763,12 @@ struct Engine {
         const std::vector<int> depths = chunk_depths(sizes, N);
         double best = 0.0;
         for (int v : {(int)RHS_60x16, (int)RHS_32x26, (int)RHS_60x8}) {
-            // the 32 x 26 tile only where a droplet asks for it: 192^3 + 128^3 +
-            // 96^3 + 64^3 take 633 us a step with it, 621 without, and the
-            // 64-droplet sweep 1175 and 1135
+            // the 32 x 26 tile only where a droplet asks for it.  Which tile is
+            // better hangs on the sizes, and these times do not tell: us a step
+            // with it and without, two 128^3 222 and 225, four 441 and 452,
+            // 64^3 + 96^3 + 128^3 206 and 217, 64^3 + 128^3 154 and 160, but
+            // 192^3 + 128^3 + 96^3 + 64^3 622 and 611, 128^3 + 120^3 220 and
+            // 214, two 96^3 110.8 and 109.5
             if (asked ? rhs_rows(v) != rhs_rows(l.variant) : v == RHS_32x26) continue;
             const double unit = v == RHS_60x8 ? 2.2 : 3.6;
             const Depth d = least_depth(sizes, depths, 3.0, cus, [&](int n) { return rhs_tiles(v, n); });
