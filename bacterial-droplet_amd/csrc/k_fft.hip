@@ -486,21 +486,17 @@ __global__ __launch_bounds__(PlanT<N>::NB) void k_fft(const Drop* __restrict__ d
     }
 }
 
-// The passes that a size has, and the largest work-group and exchange buffer
-// over the size list.
-template <int N, int AXIS, int MODE>
+// The largest work-group and exchange buffer over the size list.
+template <int N, int AXIS>
 constexpr bool fft_has_pass()
 {
-    if (MODE == FFT_FWD_FOLD) return N <= kMaxPlane;
     return AXIS == 0 || N > kMaxPlane;
 }
-template <int AXIS, int MODE, int I = 0>
+template <int AXIS, int I = 0>
 constexpr int fft_max_lds()
 {
     if constexpr (I == kNumGridSizes) return 0;
-    else
-        return std::max(fft_has_pass<kGridSizes[I], AXIS, MODE>() ? Xch<kGridSizes[I], AXIS>::SIZE : 0,
-                        fft_max_lds<AXIS, MODE, I + 1>());
+    else return std::max(fft_has_pass<kGridSizes[I], AXIS>() ? Xch<kGridSizes[I], AXIS>::SIZE : 0, fft_max_lds<AXIS, I + 1>());
 }
 template <int I = 0>
 constexpr int fft_max_threads()
@@ -514,7 +510,7 @@ template <int AXIS, int MODE, int I = 0>
 __device__ __forceinline__ void fft_any(int N, const Drop& D, const Work& wk, float2* sx, float2* stw)
 {
     if constexpr (I < kNumGridSizes) {
-        if constexpr (fft_has_pass<kGridSizes[I], AXIS, MODE>()) {
+        if constexpr (fft_has_pass<kGridSizes[I], AXIS>()) {
             if (N == kGridSizes[I]) {
                 fft_lines<kGridSizes[I], AXIS, MODE>(D, wk, sx, stw);
                 return;
@@ -537,7 +533,7 @@ __global__ __launch_bounds__(fft_max_threads(), 4) void k_fft_sizes(const Drop* 
                                                                 const Work* __restrict__ work,
                                                                 const int* __restrict__ nwork_p, int kstep)
 {
-    __shared__ float2 sx[fft_max_lds<AXIS, MODE>()];
+    __shared__ float2 sx[fft_max_lds<AXIS>()];
     __shared__ float2 stw[kMaxN + 1];
     const int nwork = *nwork_p;
     for (int v = blockIdx.x; v < xcd_span(nwork); v += gridDim.x) {
