@@ -132,10 +132,16 @@ public:
     // altogether, or all if threads or pinned memory were not to be had.
     hipError_t copy(std::vector<HostPiece>& pieces, bool f64, hipStream_t st)
     {
+        const auto bytes_from = [&](std::vector<HostPiece>::iterator p) {
+            size_t b = 0;
+            for (; p != pieces.end(); ++p) b += p->n * sizeof(float);
+            return b;
+        };
+        // before the look at each pointer, which small copies need not pay
+        if (bytes_from(pieces.begin()) < kMinBytes) return hipSuccess;
         const auto mine = std::stable_partition(pieces.begin(), pieces.end(),
                                                 [&](const HostPiece& p) { return !f64 && !pageable(p.dst); });
-        size_t bytes = 0;
-        for (auto p = mine; p != pieces.end(); ++p) bytes += p->n * sizeof(float);
+        const size_t bytes = bytes_from(mine);
         if (bytes < kMinBytes || !events()) return hipSuccess;
         chunk_n = bytes < kLargeBytes ? kChunk / 2 : kChunk;
         struct Loan {

@@ -29,7 +29,7 @@ struct hipPointerAttribute_t { hipMemoryType type; int device; };
 inline std::mutex g_mu;
 inline std::map<const char*, size_t> g_pinned;
 inline size_t g_pinned_bytes = 0, g_allocs = 0;
-inline std::atomic<size_t> g_async{0};
+inline std::atomic<size_t> g_async{0}, g_looked{0};
 inline bool g_no_memory = false;
 inline hipError_t hipHostMalloc(void** p, size_t n, unsigned)
 {
@@ -52,6 +52,7 @@ inline hipError_t hipHostFree(void* p)
 inline hipError_t hipPointerGetAttributes(hipPointerAttribute_t* a, const void* p)
 {
     std::lock_guard<std::mutex> lk(g_mu);
+    ++g_looked;
     auto it = g_pinned.upper_bound((const char*)p);
     const bool in = it != g_pinned.begin() && (--it, (const char*)p < it->first + it->second);
     a->type = in ? hipMemoryTypeHost : hipMemoryTypeUnregistered;
@@ -126,6 +127,11 @@ int main()
         for (int f = 0; f < 5; ++f) p[f].dst = pin + 4 * f * n;
         CHECK(hc.copy(p, false, nullptr) == hipSuccess && p.size() == 7);
         (void)hipHostFree(pin);
+
+        // a small state: not even a look at where it goes
+        const size_t looked = g_looked;
+        p = fields(src, 1000, (char*)a.data(), 4000);
+        CHECK(hc.copy(p, false, nullptr) == hipSuccess && p.size() == 7 && g_looked == looked);
     }
     CHECK(g_pinned_bytes == 0);  // given back with the last copier
     {
