@@ -106,14 +106,20 @@ static size_t packed_bytes(int N, int tiles)
 // put the same cell of every field on the same memory channels; a shift of 17
 // times 256 bytes per field took K_corr at 256^3 from 196 to 188 us, K_div from
 // 147 to 143 and the step of the 20-droplet sweep from 1201 to 1173 (256 bytes
-// do most of it, 129 times 256 no more).  The shift takes no more than what the
-// sums leave of the room of a 32 x 8 tile's, by which budgets were sized: 17
-// from 90^3 on, 2 to 12 below, none at 32^3, whose state stays in the caches.
+// do most of it, 129 times 256 no more).  The distance is an odd multiple of 256
+// where a shift is to be had (17 would make it a multiple of 4096 at 90^3 and
+// 150^3: with 16, steps of 76.9 -> 76.4 and 196.9 -> 196.3 us).  The shift takes
+// no more than what the sums leave of the room of a 32 x 8 tile's, by which
+// budgets were sized: 16 or 17 from 90^3 on, 1 to 11 below, none at 32^3, whose
+// state stays in the caches.
 static size_t field_bytes(int N)
 {
     const size_t n = (size_t)N * N * N;
     const size_t room = packed_bytes(N, ((N + 31) / 32) * ((N + 7) / 8)) - packed_bytes(N, proj_tiles(N));
-    return align256(n * sizeof(float)) + 256 * std::min<size_t>(17, room / (256 * kFields));
+    const size_t packed = align256(n * sizeof(float)) / 256;
+    size_t shift = std::min<size_t>(17, room / (256 * kFields));
+    if (shift > 0 && (packed + shift) % 2 == 0) --shift;
+    return 256 * (packed + shift);
 }
 
 size_t droplet_bytes(int N)
